@@ -1,0 +1,124 @@
+"""The FP32 tile kernel (attention.hip) at the sizes where it can go wrong: row
+blocks and staged key tiles with remainders, head sizes that end inside a build,
+rows that rule out vector loads, waves that share a row group's keys, and the
+diagnostics.  Bar: the reference's gate 1e-5 + 1e-4|e| (tests/cpu_attention.rs:6-14)
+on the stored values, for every storage type, since the kernel's arithmetic is
+FP32 throughout."""
+
+import numpy as np
+import pytest
+
+from gpu_util import dev, host, log, stored
+
+pytestmark = pytest.mark.gpu
+
+# (hq, hkv, D, queries, keys, window, softcap, dt, shift): `shift` elements in front
+# of every operand take it off its 16-byte boundary.
+CASES = [
+    (14, 2, 64, 9, 63, None, 0.0, "f32", 0),       # 63 packed rows, one short tile
+    (14, 2, 64, 10, 65, None, 0.0, "f32", 0),      # 70 rows: two blocks; a tile and one key
+    (8, 1, 64, 2, 700, None, 0.0, "f32", 0),       # 16 rows: four waves share the keys
+    (6, 2, 64, 7, 1000, 130, 50.0, "f32", 0),      # 21 rows: two waves each; window, softcap
+    (4, 4, 40, 70, 300, None, 0.0, "f32", 0),      # head size inside a build
+    (4, 2, 65, 33, 129, None, 0.0, "f32", 0),      # odd head size: element loads
+    (2, 1, 64, 40, 200, 17, 0.0, "f32", 1),        # unaligned operands
+    (2, 2, 128, 65, 97, None, 0.0, "f32", 0),
+    (8, 4, 256, 33, 161, 64, 30.0, "f32", 0),
+    (8, 1, 512, 5, 400, None, 0.0, "f32", 0),      # 40 rows
+    (8, 1, 512, 9, 1025, None, 0.0, "bf16", 0),
+    (8, 2, 512, 1, 2000, None, 0.0, "f16", 0),     # one decode token, 4 rows
+    (3, 1, 80, 1, 17, None, 0.0, "bf16", 0),
+    (4, 1, 7, 30, 64, None, 0.0, "f16", 3),
+]
+
+
+@pytest.fixture(scope="module")
+def torch_mod():
+    import torch
+
+    assert torch.cuda.is_available(), "GPU tests need a ROCm device"
+    return torch
+
+
+def _operand(torch, a, dt, shift):
+    t = dev(np.concatenate([np.zeros(shift, np.float32), a.reshape(-1)]), dt)
+    return t[shift:]
+
+
+def _close(got, ref, what):
+    got, ref = got.astype(np.float64), np.asarray(ref, np.float64)
+    worst = np.max(np.abs(got - ref) - 1e-4 * np.abs(ref))
+    log(f"  {what}: worst excess {worst:.2e}")
+    assert np.all(np.isfinite(got)) and worst <= 1e-5, what
+
+
+@pytest.mark.parametrize("diag", [False, True])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c))
+def test_tile_matches_oracle(torch_mod, orc, case, diag):
+    from toklet_amd import ops
+
+    torch = torch_mod
+    hq, hkv, D, Q, keys, W, softcap, dt, shift = case
+    rng = np.random.default_rng(hq * 1000 + D * 10 + keys)
+    q = stored(rng.standard_normal((Q, hq, D)), dt)
+    k = stored(rng.standard_normal((hkv, keys + 3, D)), dt)
+    v = stored(rng.standard_normal((hkv, keys + 3, D)), dt)
+    # Rows past the keys, and keys no query sees, hold NaN.
+    k[:, keys:] = v[:, keys:] = np.nan
+    if W and not diag and keys - Q - W > 0:
+        k[:, :keys - Q - W + 1] = v[:, :keys - Q - W + 1] = np.nan
+    scale = 1.0 / np.sqrt(D)
+    shape = ops.WindowAttentionShape(Q, keys, keys + 3, hq, hkv, D, keys - Q, 0, W, scale, softcap)
+    kr, vr = np.nan_to_num(k), np.nan_to_num(v)
+    ref, sref, pref = orc.window_attention(q, kr.reshape(-1), vr.reshape(-1), Q, keys, keys + 3, hq, hkv, D, keys - Q, 0,
+                                           W, scale, softcap=softcap)
+    args = [_operand(torch, x, dt, shift) for x in (q, k, v)]
+    log(f"{case} diag {diag}")
+    ctx = ops.Context(0)
+    for scores, probs in ((True, True), (False, True), (True, False)) if diag else ((False, False),):
+        out = torch.full((Q * hq * D,), np.nan, dtype=torch.float32, device="cuda")
+        sc = torch.full((hq * Q * keys,), np.nan, device="cuda") if scores else None
+        pr = torch.full((hq * Q * keys,), np.nan, device="cuda") if probs else None
+        # bf16/f16 calls without diagnostics at 64/128/256 belong to other kernels.
+        ops.window_attention(ctx, *args, out, sc, pr, shape)
+        _close(host(out), ref, "context")
+        if scores:
+            _close(host(sc), sref, "scores")
+        if probs:
+            _close(host(pr), pref, "probabilities")
+            seen = np.arange(keys) <= np.arange(keys - Q, keys)[:, None]
+            seen &= (np.arange(keys) > np.arange(keys - Q, keys)[:, None] - W) if W else True
+            got = host(pr).reshape(hq, Q, keys)
+            assert np.all(got[:, ~seen].view(np.uint32) == 0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dt,D,W", [("f32", 64, 33), ("f32", 256, 50), ("bf16", 512, 40)])
+def test_tile_over_ring_spans(torch_mod, orc, dt, D, W):
+    """Chunks over a wrapped ring: the keys come from three segments, whose
+    boundaries fall inside staged tiles."""
+    from toklet_amd import kv as kvmod, ops
+
+    torch = torch_mod
+    rng = np.random.default_rng(D + W)
+    hq, hkv, T = 4, 2, 4 * W
+    ctx = ops.Context(0)
+    ring = kvmod.WindowKvCache(ctx, hkv, D, W, T, W, {"f32": torch.float32, "bf16": torch.bfloat16}[dt])
+    k, v = (stored(rng.standard_normal((hkv, T, D)), dt) for _ in range(2))
+    q = stored(rng.standard_normal((T, hq, D)), dt)
+    pos, scale = 0, 1.0 / np.sqrt(D)
+    for n in (W - 3, 1, 20, 17, W + 2):
+        frame = ring.prepare(*(dev(np.ascontiguousarray(x[:, pos:pos + n]), dt) for x in (k, v)), n)
+        view = ring.view(frame)
+        out = torch.full((n * hq * D,), np.nan, dtype=torch.float32, device="cuda")
+        ops.span_attention(ctx, dev(q[pos:pos + n], dt), view.segments(), out, None, None, view.attention_shape(hq, scale))
+        keys = pos + n
+        ref, _, _ = orc.window_attention(q[pos:pos + n], np.ascontiguousarray(k[:, :keys]).reshape(-1),
+                                         np.ascontiguousarray(v[:, :keys]).reshape(-1), n, keys, keys, hq, hkv, D, pos, 0,
+                                         W, scale)
+        log(f"{dt} D={D} W={W} chunk {pos}+{n}")
+        if dt == "f32" or D == 512:
+            _close(host(out), ref, "context")
+        ring.commit(frame)
+        pos += n
+    ctx.close()

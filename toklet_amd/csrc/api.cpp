@@ -23,10 +23,13 @@
 #include "device.hpp"
 #include "host.hpp"
 
-extern "C" hipError_t tkh_launch_generic(const tkh::Params *p, int dtype, hipStream_t stream,
-                                         hipEvent_t start, hipEvent_t stop);
-extern "C" hipError_t tkh_launch_combine(const tkh::Params *p, int64_t total_rows,
-                                         hipStream_t stream, hipEvent_t start, hipEvent_t stop);
+extern "C" int tkh_tile_head(int head_dim);
+extern "C" int tkh_tile_keys(int head_dim);
+extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStream_t stream,
+                                      hipEvent_t start, hipEvent_t stop);
+extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
+                                            hipEvent_t start, hipEvent_t stop);
+extern "C" hipError_t tkh_launch_tile_probs(const tkh::TileArgs *a, hipStream_t stream);
 extern "C" hipError_t tkh_launch_kv_append(int src, int dst, const void *k, const void *v,
                                            void *kc, void *vc, int64_t tokens, int heads,
                                            int dims, int64_t capacity, int64_t offset,
@@ -642,6 +645,103 @@ uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
     return TKH_OK;
 }
 
+// FP32 storage, other head sizes and diagnostics: the FP32 tile kernel, then a
+// combine launch when the keys are split and a probability launch when asked.
+uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_error *err) {
+    const int64_t D = plan.head_dim, Hq = plan.query_heads, Hkv = plan.kv_heads, G = Hq / Hkv;
+    const int64_t DP = tkh_tile_head((int)D), KT = tkh_tile_keys((int)D);
+    // One partial per output row must fit the workspace, split or not.
+    {
+        size_t need = 0;
+        for (auto &p : group) need += (size_t)p.queries * Hq * (D + 2) * sizeof(float);
+        if (need > split_region_bytes(ctx))
+            return fail(err, TKH_UNSUPPORTED, "workspace", 0, need, split_region_bytes(ctx),
+                        "attention needs %zu workspace bytes, context has %zu for it", need,
+                        split_region_bytes(ctx));
+    }
+    tkh::TileArgs args{};
+    int64_t max_rows = 0, max_span = 0, rows = 0;
+    bool vec = D % 4 == 0;
+    const uintptr_t chunk = 4 * (uintptr_t)esize(plan.dtype);
+    for (auto &p : group) {
+        visible_union(plan, p);
+        max_rows = std::max<int64_t>(max_rows, p.queries * G);
+        max_span = std::max<int64_t>(max_span, plan.diag_mode == 1 ? p.keys : p.vis_hi - p.vis_lo);
+        rows += (int64_t)p.queries * Hq;
+        uintptr_t at = (uintptr_t)p.q;
+        int64_t strides = p.q_row_stride;
+        for (int i = 0; i < p.nseg; ++i) {
+            at |= (uintptr_t)p.seg[i].k | (uintptr_t)p.seg[i].v;
+            strides |= p.seg[i].head_stride | p.seg[i].row_stride;
+        }
+        vec = vec && at % chunk == 0 && strides % 4 == 0;
+    }
+    // Row groups per workgroup, then key splits for about tile_groups
+    // workgroups in all, each at least a staged tile long.
+    const int rw = max_rows <= 16 ? 1 : (max_rows <= 32 ? 2 : 4);
+    int64_t base = 0;
+    for (auto &p : group) base += Hkv * (((int64_t)p.queries * G + 16 * rw - 1) / (16 * rw));
+    int64_t splits = std::max<int64_t>(1, (ctx->tile_groups + base - 1) / base);
+    splits = std::min<int64_t>(splits, std::max<int64_t>(1, max_span / KT));
+    int kw = max_span > KT ? (int)std::min<int64_t>(4 / rw, KT / 16) : 1;
+    splits = std::min<int64_t>(splits, 64 / kw);
+    auto fits = [&](int64_t s) {
+        return s == 1 || (size_t)rows * s * (DP + 2) * sizeof(float) <= split_region_bytes(ctx);
+    };
+    while (!fits(splits * kw)) {
+        if (splits > 1) splits = (splits + 1) / 2;
+        else kw /= 2;
+    }
+    int64_t sk = (max_span + splits - 1) / splits;
+    sk = std::max<int64_t>(KT, (sk + 15) / 16 * 16);
+    if (sk > INT32_MAX) return fail(err, TKH_UNSUPPORTED, "keys", 0, 0, 0, "key range too large");
+    splits = std::max<int64_t>(1, (max_span + sk - 1) / sk);
+    int64_t tiles = 0, part_rows = 0;
+    for (auto &p : group) {
+        p.tile_base = tiles;
+        p.part_base = part_rows;
+        p.splits = (int32_t)splits;
+        p.split_keys = (int32_t)sk;
+        p.row_blocks = (int32_t)(((int64_t)p.queries * G + 16 * rw - 1) / (16 * rw));
+        p.slot_base = part_rows * splits * kw;
+        tiles += Hkv * p.row_blocks * splits;
+        part_rows += (int64_t)p.queries * Hq;
+    }
+    if (tiles > UINT32_MAX / 256) return fail(err, TKH_UNSUPPORTED, "grid", 0, 0, 0, "too many workgroups");
+
+    tkh::Problem *dev = nullptr;
+    if (group.size() > 1) TRY(upload(ctx, group.data(), (int)group.size(), &dev, err));
+    tkh::Params &prm = args.p;
+    prm = base_params(ctx, plan);
+    prm.problems = dev;
+    if (group.size() == 1) prm.single = group[0];
+    prm.nproblems = (int32_t)group.size();
+    prm.total_tiles = tiles;
+    prm.part_ml = reinterpret_cast<float *>(ctx->workspace);
+    prm.part_o = prm.part_ml + 2 * (size_t)rows * splits * kw;
+    prm.scores = plan.scores;
+    prm.probs = plan.probs;
+    prm.diag_mode = plan.diag_mode;
+    args.rw = rw;
+    args.kw = kw;
+    args.vec = vec ? 1 : 0;
+
+    const bool merge = splits * kw > 1;
+    hipEvent_t *ev = nullptr;
+    if (ctx->profiling) TRY(profile_slot(ctx, &ev, merge, err));
+    hipError_t e = tkh_launch_tile(&args, (int)plan.dtype, ctx->stream, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
+    if (e != hipSuccess) return device_error(e, "attention launch", err);
+    if (merge) {
+        e = tkh_launch_tile_merge(&args, rows, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);
+        if (e != hipSuccess) return device_error(e, "combine launch", err);
+    }
+    if (plan.probs) {
+        e = tkh_launch_tile_probs(&args, ctx->stream);
+        if (e != hipSuccess) return device_error(e, "probability launch", err);
+    }
+    return TKH_OK;
+}
+
 // Launch one group of problems (<= kSlotProblems) through the workspace.
 uint32_t launch_group(tkh_context *ctx, const Plan &plan, Problems group,
                       tkh_error *err) {
@@ -666,64 +766,7 @@ uint32_t launch_group(tkh_context *ctx, const Plan &plan, Problems group,
             (plan.dtype == TKH_BF16 || plan.dtype == TKH_F16) && (D == 64 || D == 128 || D == 256))
             return launch_prefill(ctx, plan, group, err);
     }
-    // FP32, odd head sizes and diagnostics: one wave per (query, head), then a
-    // combine launch that publishes the context.
-    const size_t ws_floats = split_region_bytes(ctx) / sizeof(float);
-    {
-        size_t need = 0;
-        for (auto &p : group) need += (size_t)p.queries * Hq * (D + 2);
-        if (need > ws_floats)
-            return fail(err, TKH_UNSUPPORTED, "workspace", 0, need * 4, split_region_bytes(ctx),
-                        "attention needs %zu workspace bytes, context has %zu for it", need * 4,
-                        split_region_bytes(ctx));
-    }
-    int64_t tiles = 0, rows = 0, part_rows = 0;
-    for (auto &p : group) {
-        p.tile_base = tiles;
-        p.part_base = rows;
-        p.splits = 1;
-        p.row_blocks = 1;
-        tiles += (int64_t)p.queries * Hq;
-        p.slot_base = part_rows;
-        rows += (int64_t)p.queries * Hq;
-        part_rows += (int64_t)p.queries * Hq;
-    }
-
-    tkh::Problem *dev = nullptr;
-    if (group.size() > 1) TRY(upload(ctx, group.data(), (int)group.size(), &dev, err));
-
-    tkh::Params prm{};
-    prm.problems = dev;
-    if (group.size() == 1) prm.single = group[0];
-    prm.nproblems = (int32_t)group.size();
-    prm.query_heads = (int32_t)Hq;
-    prm.kv_heads = (int32_t)Hkv;
-    prm.head_dim = (int32_t)D;
-    prm.group = (int32_t)G;
-    prm.has_window = plan.has_window ? 1 : 0;
-    prm.window = plan.window;
-    prm.scale = plan.scale;
-    prm.scale_log2 = plan.scale * 1.4426950408889634f;
-    prm.softcap = plan.softcap;
-    prm.softcap_inv = plan.softcap != 0.0f ? 1.0f / plan.softcap : 0.0f;
-    prm.softcap_y = prm.scale * prm.softcap_inv;
-    prm.softcap_log2 = plan.softcap * 1.4426950408889634f;
-    prm.total_tiles = tiles;
-    prm.part_ml = reinterpret_cast<float *>(ctx->workspace);
-    prm.part_o = reinterpret_cast<float *>(ctx->workspace) + 2 * part_rows;
-    prm.status = ctx->status_dev;
-    prm.scores = plan.scores;
-    prm.probs = plan.probs;
-    prm.diag_mode = plan.diag_mode;
-
-    hipEvent_t *ev = nullptr;
-    if (ctx->profiling) TRY(profile_slot(ctx, &ev, true, err));
-    hipError_t e = tkh_launch_generic(&prm, (int)plan.dtype, ctx->stream, ev ? ev[0] : nullptr,
-                                      ev ? ev[1] : nullptr);
-    if (e != hipSuccess) return device_error(e, "attention launch", err);
-    e = tkh_launch_combine(&prm, rows, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);
-    if (e != hipSuccess) return device_error(e, "combine launch", err);
-    return TKH_OK;
+    return launch_tile(ctx, plan, group, err);
 }
 
 // Launch `count` problems in groups of at most kSlotProblems (their planning
@@ -793,6 +836,7 @@ void init_tuning(tkh_context *ctx, int device) {
     ctx->prefill16 = env_int("TKH_PREFILL16", 1);
     ctx->prefill16_groups = std::max(1, env_int("TKH_PREFILL16_GROUPS", 64));
     ctx->prefill16_waves = env_int("TKH_PREFILL16_WAVES", 4) == 8 ? 8 : 4;
+    ctx->tile_groups = std::max(1, env_int("TKH_TILE_GROUPS", 512));
 }
 
 // First visible key (absolute) of a query at `position` (window_attention.rs:105-107).

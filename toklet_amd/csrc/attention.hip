@@ -1,123 +1,348 @@
-// attention.hip - generic attention kernels of the session path.
+// attention.hip - attention in FP32 arithmetic on the matrix cores: FP32
+// storage, head sizes outside 64/128/256, and the optional score/probability
+// diagnostics the reference operators can return.  bf16/f16 chunks and decode
+// at head_dim 64/128/256 take the MFMA prefill and streaming decode kernels
+// instead.
 //
-//  * attn_generic<DT>: one wave per (query, query head) with FP32 VALU math;
-//    any head_dim <= 512, FP32 storage, and the optional score/probability
-//    diagnostics the reference operators can return.  bf16/f16 chunks and
-//    decode at head_dim 64/128/256 take the MFMA prefill and streaming decode
-//    kernels instead.
-//  * attn_combine: merges split-K partials (max, mass, unnormalised context)
-//    and publishes FP32 context only when the status word is clean.
+//  * attn_tile<DT, DP>: any head_dim D <= DP.  A workgroup is four waves over
+//    16 packed rows each (query x head of the GQA group) of one (problem, KV
+//    head), optionally one key split of it.
+//  * attn_tile_merge: combines split-K partials (max, mass, unnormalised
+//    context) and writes the context.
+//  * attn_tile_probs: the diagnostics' probabilities from the stored scores
+//    and each row's merged (max, mass).
 //
-// Scores are kept in the exp2 domain (score * scale * log2 e) so the softmax
-// uses v_exp_f32 directly.  Masked keys contribute exactly zero.
+// Scores are kept in the exp2 domain (score * log2 e) so the softmax uses
+// v_exp_f32 directly.  Masked keys contribute exactly zero.
 #include "device.hpp"
 
 namespace tkh {
 
-// ---------------------------------------------------------------------------
-// Generic VALU kernel: one wave per (problem query, query head)
-// ---------------------------------------------------------------------------
+namespace {
 
+// Keys per staged tile: K and V tiles of FP32 rows in about 33 KiB of LDS at
+// head sizes to 128 (four workgroups per CU), 66 KiB above (two).
+__host__ __device__ constexpr int tile_keys(int DP) { return DP <= 64 ? 64 : (DP <= 256 ? 32 : 16); }
+
+// Four consecutive stored elements.
+template <int DT> struct Raw4 { using T = uint32_t __attribute__((ext_vector_type(2))); };
+template <> struct Raw4<F32> { using T = u32x4; };
+
+template <int DT> __device__ __forceinline__ f32x4 widen4(typename Raw4<DT>::T w) {
+    f32x4 x;
+    if constexpr (DT == F32) {
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t u = w[e];
+            x[e] = __builtin_bit_cast(float, u);
+        }
+    } else {
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t u = w[e];
+            if constexpr (DT == BF16) {
+                x[2 * e] = __builtin_bit_cast(float, u << 16);
+                x[2 * e + 1] = __builtin_bit_cast(float, u & 0xffff0000u);
+            } else {
+                const f16x2 h = __builtin_bit_cast(f16x2, u);
+                x[2 * e] = (float)h[0];
+                x[2 * e + 1] = (float)h[1];
+            }
+        }
+    }
+    return x;
+}
+
+// Elements [off, off + 4) of which the first n exist (the rest read as zero):
+// one vector load when every row of the launch allows it, else one by one.
 template <int DT>
-__global__ __launch_bounds__(64) void attn_generic(Params p) {
-    __shared__ float qs[512];
-    const int lane = threadIdx.x;
-    const int64_t tile = blockIdx.x;
-    if (tile >= p.total_tiles) return;
-    const Problem &pr = tile_problem(p, tile);
-    const int Hq = p.query_heads, D = p.head_dim;
-    const int64_t local = tile - pr.tile_base;
-    const int t = (int)(local / Hq), h = (int)(local % Hq);
-    const int kvh = h / p.group;
-    const int64_t pos = pr.q_pos0 + t;
-    int64_t lo, hi;
-    visible_range(p, pr, pos, &lo, &hi);
+__device__ __forceinline__ typename Raw4<DT>::T load4(const void *base, int64_t off, int n, bool vec) {
+    using T = typename Raw4<DT>::T;
+    T w{};
+    if (vec) {
+        if (n > 0) {
+            if constexpr (DT == F32) w = *gload_ptr<T>(reinterpret_cast<const float *>(base) + off);
+            else w = *gload_ptr<T>(reinterpret_cast<const uint16_t *>(base) + off);
+        }
+        return w;
+    }
+    for (int e = 0; e < 4; ++e)
+        if (e < n) {
+            if constexpr (DT == F32) w[e] = reinterpret_cast<const uint32_t *>(base)[off + e];
+            else w[e >> 1] |= (uint32_t)reinterpret_cast<const uint16_t *>(base)[off + e] << (16 * (e & 1));
+        }
+    return w;
+}
 
-    for (int d = lane; d < D; d += 64)
-        qs[d] = load_elem<DT>(pr.q, (int64_t)t * pr.q_row_stride + (int64_t)h * D + d);
-    __syncthreads();
+// Four floats at any 4-byte aligned address.
+using f32x4u = float __attribute__((ext_vector_type(4), aligned(4)));
 
-    auto score_of = [&](int64_t key, bool *finite_ok) -> float {
-        int which;
-        int64_t off = seg_offset(pr, key, kvh, &which);
-        const void *kbase = pr.seg[which].k;
-        float dot = 0.0f;
-        for (int d = 0; d < D; ++d) dot += qs[d] * load_elem<DT>(kbase, off + d);
-        float x = dot * p.scale;
-        if (p.softcap != 0.0f) x = softcap_f(x, p.softcap);
-        *finite_ok = is_finite_f(x);
-        return x;
+// Over the four lanes j, j + 16, j + 32, j + 48 of a query row.
+__device__ __forceinline__ float row4_sum(float x) { return xor_sum(xor_sum(x, 16), 32); }
+__device__ __forceinline__ float row4_max(float x) { return xor_max(xor_max(x, 16), 32); }
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+}  // namespace
+
+// What bounds it: v_mfma_f32_16x16x4 (32 cycles for 2,048 FLOP, 157 TFLOP/s
+// over the card) on long ranges, launches and memory round trips on short
+// ones.  Every product and sum stays FP32, as storage and reference have it.
+//
+// Lane (j, g) = (lane % 16, lane / 16) of a wave holds query row j:
+//  * S^T = K Q^T per 16-key block: A = K (key j, features 16 c + 4 g + e in
+//    step (c, e)), B = Q^T (row j, the same features), so both operands are
+//    read four features at a time; the result holds row j, keys 4 g + r.
+//  * O^T = V^T P^T: step r takes keys 4 g + r, where the scores already sit,
+//    so P needs no exchange; A = V at key 4 g + r, feature 64 fb + 4 j + e of
+//    MFMA (fb, e), again four features per LDS read.  The lane ends with
+//    features 64 fb + 16 g .. + 15 of its row.
+// K rows are padded by four floats in LDS, so the 16 rows of a read fall on
+// distinct banks.  A tile's global loads are in flight while the one before
+// it is multiplied.
+//
+// A workgroup takes a.rw row groups; with fewer than four the other waves
+// share the groups' keys (a.kw of them, 16-key blocks in turn), each writing
+// a partial of its own, so short row blocks keep every SIMD busy.
+//
+// It replaced one wave per (query, head) on the vector unit, whose lanes each
+// read a key row of their own.  Per call: a 128-token FP32 chunk at offset
+// 1920 (14/2/64) with its append 1017 -> 40 us, a 512-token FP32 prompt 313 ->
+// 42 us, 128 queries over 1025 keys at 8/1/512 (bf16) 2240 -> 281 us, and 300
+// tokens of 16/8/128 with both diagnostics 243 -> 57 us.
+template <int DT, int DP>
+__global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
+    warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
+    constexpr int KT = tile_keys(DP), NB = KT / 16, FC = DP / 16, FB = DP / 64;
+    constexpr int KS = DP + 4;               // staged K row stride
+    constexpr int NCH = KT * DP / 4 / 256;   // 4-element chunks per thread and tile
+    __shared__ __attribute__((aligned(16))) float kt[KT * KS];
+    __shared__ __attribute__((aligned(16))) float vt[KT * DP];
+    using Raw = typename Raw4<DT>::T;
+    const Params &p = a.p;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int j = lane & 15, g = lane >> 4;
+    const int G = p.group, Hq = p.query_heads, D = p.head_dim;
+    const bool vec = a.vec != 0, full_diag = p.diag_mode == 1;
+
+    // XCD-major tile order (dispatch slot b runs on XCD b % 8): the row blocks
+    // of one KV head, which read the same keys, share an XCD's L2.
+    int64_t tile;
+    {
+        const uint32_t nb = gridDim.x, per = (nb + 7) / 8;
+        const uint32_t x = blockIdx.x % 8, k = blockIdx.x / 8;
+        const uint32_t full = nb % 8 == 0 ? 8 : nb % 8;
+        tile = (int64_t)(x < full ? x * per + k : full * per + (x - full) * (per - 1) + k);
+    }
+    const_ptr<Problem> pr = problem_ptr(p, tile);
+    const uint32_t local = (uint32_t)(tile - pr->tile_base), nrb = (uint32_t)pr->row_blocks;
+    const uint32_t ns = (uint32_t)pr->splits;
+    const int rb = (int)(local % nrb), split = (int)(local / nrb % ns), kvh = (int)(local / (nrb * ns));
+    const int64_t k_pos0 = pr->k_pos0, keys = pr->keys, q_pos0 = pr->q_pos0;
+    const int m_kv = pr->queries * G, nseg = pr->nseg;
+
+    const int rw = a.rw, kw = a.kw;
+    const int rg = wave % rw, ks = wave / rw;
+    const int row0 = (rb * rw + rg) * 16;    // the wave's first packed row
+    const bool active = ks < kw && row0 < m_kv;
+    const int prow = row0 + j;
+    const bool rvalid = ks < kw && prow < m_kv;
+    const int rrow = prow < m_kv ? prow : m_kv - 1;
+    const int t_row = (int)((uint32_t)rrow / (uint32_t)G), h_row = kvh * G + (int)((uint32_t)rrow % (uint32_t)G);
+
+    // The split's keys; the workgroup's rows see [v_lo, v_hi) of them.  The
+    // full diagnostics score every key, so they walk the whole split.
+    const int64_t base_lo = full_diag ? 0 : pr->vis_lo, base_hi = full_diag ? keys : pr->vis_hi;
+    const int64_t s_lo = base_lo + (int64_t)split * pr->split_keys;
+    const int64_t s_hi = s_lo + pr->split_keys < base_hi ? s_lo + pr->split_keys : base_hi;
+    int64_t r_lo, r_hi, v_lo, v_hi, w_lo, w_hi, tmp;
+    visible_range(p, k_pos0, keys, q_pos0 + t_row, &r_lo, &r_hi);
+    const int wg_first = rb * rw * 16, wg_last = min(wg_first + rw * 16, m_kv) - 1;
+    visible_range(p, k_pos0, keys, q_pos0 + wg_first / G, &v_lo, &tmp);
+    visible_range(p, k_pos0, keys, q_pos0 + wg_last / G, &tmp, &v_hi);
+    v_lo = v_lo > s_lo ? v_lo : s_lo;
+    v_hi = v_hi < s_hi ? v_hi : s_hi;
+    const int wv_first = min(row0, m_kv - 1), wv_last = min(row0 + 15, m_kv - 1);
+    visible_range(p, k_pos0, keys, q_pos0 + wv_first / G, &w_lo, &tmp);
+    visible_range(p, k_pos0, keys, q_pos0 + wv_last / G, &tmp, &w_hi);
+    const int64_t lo = full_diag ? s_lo : v_lo, hi = full_diag ? s_hi : v_hi;
+    const int n = hi > lo ? (int)(hi - lo) : 0;
+    // Relative to `lo` from here on.
+    auto rel = [&](int64_t x) { return (int)(x < lo ? 0 : (x > lo + n ? n : x - lo)); };
+    const int rlo = rvalid ? rel(r_lo) : 0, rhi = rvalid ? rel(r_hi) : 0;
+    const int wlo = rel(w_lo), whi = active ? rel(w_hi) : 0;
+    const int vlo = rel(v_lo), vhi = rel(v_hi);
+
+    f32x4 q[FC];
+    for (int c = 0; c < FC; ++c) {
+        const int d = 16 * c + 4 * g;
+        q[c] = widen4<DT>(load4<DT>(pr->q, (int64_t)t_row * pr->q_row_stride + (int64_t)h_row * D + d, D - d, vec));
+    }
+
+    // A thread's chunk m of a tile: row i / (DP / 4), features 4 (i % (DP / 4)).
+    // Rows past the range read its last row (K: masked; V: zeroed on staging,
+    // so a stored non-finite value outside the visible keys never meets a zero
+    // probability), features past the head are zeros.
+    constexpr int CPR = DP / 4;
+    Raw kreg[NCH], vreg[NCH];
+    auto fetch = [&](int t0) {
+        for (int m = 0; m < NCH; ++m) {
+            const int i = tid + 256 * m, c = i % CPR;
+            const int64_t key = lo + min(t0 + i / CPR, n - 1);
+            const void *kb, *vb;
+            int64_t off;
+            if (nseg == 1) {
+                kb = pr->seg[0].k;
+                vb = pr->seg[0].v;
+                off = (int64_t)kvh * pr->seg[0].head_stride + key * pr->seg[0].row_stride;
+            } else {
+                off = seg_select(pr, key, kvh, &kb, &vb);
+            }
+            kreg[m] = load4<DT>(kb, off + 4 * c, D - 4 * c, vec);
+            vreg[m] = load4<DT>(vb, off + 4 * c, D - 4 * c, vec);
+        }
+    };
+    auto stage = [&](int t0) {
+        for (int m = 0; m < NCH; ++m) {
+            const int i = tid + 256 * m, r = i / CPR, c = i % CPR;
+            *reinterpret_cast<f32x4 *>(kt + r * KS + 4 * c) = widen4<DT>(kreg[m]);
+            const bool in = t0 + r >= vlo && t0 + r < vhi;
+            *reinterpret_cast<f32x4 *>(vt + r * DP + 4 * c) = in ? widen4<DT>(vreg[m]) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     };
 
-    float acc[8];
-    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    float m = NEG_INF, l = 0.0f;
+    const float scale = p.scale, cap = p.softcap;
+    const bool last_row = h_row == Hq - 1 && t_row == pr->queries - 1;
+    float *const xs = p.scores ? p.scores : p.probs;  // raw scores (attn_tile_probs turns them into probabilities)
+    f32x4 acc[FB][4];
+    for (int fb = 0; fb < FB; ++fb)
+        for (int e = 0; e < 4; ++e) acc[fb][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = NEG_INF, l_run = 0.0f;
     bool bad = false;
-    for (int64_t j0 = lo; j0 < hi; j0 += 64) {
-        int64_t key = j0 + lane;
-        float s2 = NEG_INF;
-        if (key < hi) {
-            bool ok;
-            float x = score_of(key, &ok);
-            bad |= !ok;
-            s2 = x * LOG2E;
+
+    if (n > 0) fetch(0);
+    for (int t0 = 0; t0 < n; t0 += KT) {
+        __syncthreads();
+        stage(t0);
+        __syncthreads();
+        if (t0 + KT < n) fetch(t0 + KT);
+        f32x4 st[NB];
+        bool seen[NB];  // some row of the wave sees a key of the block
+        float tmax = NEG_INF;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int k0 = t0 + 16 * b;
+            const bool mine = active && b % kw == ks;
+            seen[b] = mine && k0 < whi && k0 + 16 > wlo;
+            st[b] = f32x4{NEG_INF, NEG_INF, NEG_INF, NEG_INF};
+            if (!(seen[b] || (full_diag && mine && k0 < n))) continue;
+            f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;  // two chains
+            const float *kr = kt + (16 * b + j) * KS + 4 * g;
+#pragma unroll
+            for (int c = 0; c < FC; c += 2) {
+                const f32x4 k0v = *reinterpret_cast<const f32x4 *>(kr + 16 * c);
+                const f32x4 k1v = *reinterpret_cast<const f32x4 *>(kr + 16 * c + 16);
+                for (int e = 0; e < 4; ++e) {
+                    s0 = mfma4(k0v[e], q[c][e], s0);
+                    s1 = mfma4(k1v[e], q[c + 1][e], s1);
+                }
+            }
+            f32x4 x;
+            for (int r = 0; r < 4; ++r) {
+                x[r] = (s0[r] + s1[r]) * scale;
+                if (cap != 0.0f) x[r] = softcap_f(x[r], cap);
+            }
+            const int key = k0 + 4 * g;
+            for (int r = 0; r < 4; ++r) {
+                const bool vis = key + r >= rlo && key + r < rhi;
+                bad |= vis && !is_finite_f(x[r]);
+                st[b][r] = vis ? x[r] * LOG2E : NEG_INF;
+                tmax = fmaxf(tmax, st[b][r]);
+            }
+            if (p.diag_mode != 0 && rvalid && (full_diag || last_row)) {
+                const int first = full_diag ? 0 : rlo, end = full_diag ? n : rhi;
+                float *xr = xs + (full_diag ? ((int64_t)h_row * pr->queries + t_row) * keys : 0) + lo + key;
+                if (key >= first && key + 4 <= end) *reinterpret_cast<f32x4u *>(xr) = x;
+                else
+                    for (int r = 0; r < 4; ++r)
+                        if (key + r >= first && key + r < end) xr[r] = x[r];
+            }
         }
-        float m_new = fmaxf(m, wave_max(s2));
-        float m_use = m_new == NEG_INF ? 0.0f : m_new;
-        float corr = __builtin_amdgcn_exp2f(m - m_use);
-        float e = __builtin_amdgcn_exp2f(s2 - m_use);
-        l = l * corr + wave_sum(e);
-        m = m_new;
-        for (int i = 0; i < 8; ++i) acc[i] *= corr;
-        int n = (int)min<int64_t>(64, hi - j0);
-        for (int jj = 0; jj < n; ++jj) {
-            float pj = __shfl(e, jj, 64);
-            int which;
-            int64_t off = seg_offset(pr, j0 + jj, kvh, &which);
-            const void *vbase = pr.seg[which].v;
-            for (int i = 0; i < 8; ++i) {
-                int d = lane + 64 * i;
-                if (d < D) acc[i] += pj * load_elem<DT>(vbase, off + d);
+        // The tile's maximum over the row's four lanes; O and l move with it.
+        tmax = row4_max(tmax);
+        const float m_new = fmaxf(m_run, tmax);
+        const float base = m_new == NEG_INF ? 0.0f : m_new;
+        if (__ballot(m_new > m_run) != 0) {
+            const float corr = __builtin_amdgcn_exp2f(m_run - base);
+            l_run *= corr;
+            for (int fb = 0; fb < FB; ++fb)
+                for (int e = 0; e < 4; ++e)
+                    for (int r = 0; r < 4; ++r) acc[fb][e][r] *= corr;
+            m_run = m_new;
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (!seen[b]) continue;
+            for (int r = 0; r < 4; ++r) {
+                const float e = __builtin_amdgcn_exp2f(st[b][r] - base);
+                st[b][r] = e;
+                l_run += e;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float *vr = vt + (16 * b + 4 * g + r) * DP + 4 * j;
+                for (int fb = 0; fb < FB; ++fb) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(vr + 64 * fb);
+                    for (int e = 0; e < 4; ++e) acc[fb][e] = mfma4(v[e], st[b][r], acc[fb][e]);
+                }
             }
         }
     }
 
-    // Diagnostics: raw scores and normalised probabilities in the reference layouts.
-    const bool last_row = (h == Hq - 1) && (t == pr.queries - 1);
-    if (p.diag_mode == 1 || (p.diag_mode == 2 && last_row)) {
-        int64_t d_lo = p.diag_mode == 1 ? 0 : lo;
-        int64_t d_hi = p.diag_mode == 1 ? pr.keys : hi;
-        int64_t row = p.diag_mode == 1 ? ((int64_t)h * pr.queries + t) * pr.keys : 0;
-        float inv = 1.0f / l;
-        for (int64_t j0 = d_lo; j0 < d_hi; j0 += 64) {
-            int64_t key = j0 + lane;
-            if (key >= d_hi) continue;
-            bool ok;
-            float x = score_of(key, &ok);
-            float pr_v = (key >= lo && key < hi) ? __builtin_amdgcn_exp2f(x * LOG2E - m) * inv : 0.0f;
-            if (p.scores) p.scores[row + key] = x;
-            if (p.probs) p.probs[row + key] = pr_v;
+    l_run = row4_sum(l_run);
+    const bool direct = ns == 1 && kw == 1;
+    bool bad_mass = false, bad_out = false;
+    if (rvalid) {
+        const int64_t part = pr->slot_base + ((int64_t)kvh * m_kv + prow) * (ns * kw) + split * kw + ks;
+        if (g == 0 && (!direct || p.diag_mode != 0)) {
+            const f32x2 ml = {m_run, l_run};
+            *gstore_ptr<f32x2>(p.part_ml + 2 * part) = ml;
         }
-    }
-
-    const int64_t prow = pr.slot_base + ((int64_t)t * Hq + h) * pr.splits;
-    for (int i = 0; i < 8; ++i) {
-        int d = lane + 64 * i;
-        if (d < D) {
-            bad |= !is_finite_f(acc[i]);
-            p.part_o[prow * D + d] = acc[i];
-        }
-    }
-    if (lane == 0) {
-        p.part_ml[prow * 2 + 0] = m;
-        p.part_ml[prow * 2 + 1] = l;
+        const float inv = direct ? 1.0f / l_run : 1.0f;
+        bad_mass = direct && (!(l_run > 0.0f) || !is_finite_f(l_run));
+        float *orow = direct ? pr->out + ((int64_t)t_row * Hq + h_row) * D : p.part_o + part * DP;
+        for (int fb = 0; fb < FB; ++fb)
+            for (int r = 0; r < 4; ++r) {
+                const int d = 64 * fb + 16 * g + 4 * r;
+                f32x4 o;
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = acc[fb][e][r];
+                    bad |= d + e < D && !is_finite_f(o[e]);
+                    o[e] *= inv;
+                    bad_out |= d + e < D && !is_finite_f(o[e]);
+                }
+                // A partial whose split shows the row no key is never read.
+                if (d + 4 <= D) {
+                    if (direct || m_run != NEG_INF) *reinterpret_cast<f32x4u *>(orow + d) = o;
+                } else {
+                    for (int e = 0; e < 4; ++e)
+                        if (d + e < D) orow[d + e] = o[e];
+                }
+            }
     }
     raise_status(p, bad, ST_NONFINITE_INPUT);
+    raise_status(p, bad_mass, ST_BAD_MASS);
+    raise_status(p, direct && bad_out, ST_NONFINITE_OUTPUT);
 }
 
-// ---------------------------------------------------------------------------
-// Split-K combine + gated publish: one wave per output row
-// ---------------------------------------------------------------------------
+// Merged (max, mass) of a row's S partials.
+__device__ __forceinline__ void merged_stats(const float *ml, int S, float &M, float &L) {
+    M = NEG_INF;
+    for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * s]);
+    L = 0.0f;
+    for (int s = 0; s < S; ++s)
+        if (ml[2 * s] != NEG_INF) L += __builtin_amdgcn_exp2f(ml[2 * s] - M) * ml[2 * s + 1];
+}
 
 __device__ __forceinline__ int find_row_problem(const Params &p, int64_t row) {
     int lo = 0, hi = p.nproblems - 1;
@@ -128,97 +353,134 @@ __device__ __forceinline__ int find_row_problem(const Params &p, int64_t row) {
     return lo;
 }
 
-__global__ __launch_bounds__(256) void attn_combine(Params p, int64_t total_rows) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+// Split-K combine: one thread per four features of a row, so a launch has
+// rows x D / 4 threads and a thread's partials (16 splits at a time) are all
+// in flight together; the time is one memory round trip.
+__global__ __launch_bounds__(256) void attn_tile_merge(TileArgs a, int64_t total_rows, int dp) {
+    const Params &p = a.p;
+    const int D = p.head_dim, Hq = p.query_heads, G = p.group;
+    const uint32_t per = (uint32_t)(D + 3) / 4;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t row = i / per;
     if (row >= total_rows) return;
-    if (__atomic_load_n(p.status, __ATOMIC_RELAXED) != 0) return;  // never publish after bad input
+    const int d = 4 * (int)(i - row * per);
     const Problem &pr = p.nproblems == 1 ? p.single : p.problems[find_row_problem(p, row)];
-    const int D = p.head_dim, Hq = p.query_heads;
+    const int m_kv = pr.queries * G, S = pr.splits * a.kw;
     const int64_t local = row - pr.part_base;
-    const int t = (int)(local / Hq), h = (int)(local % Hq);
-    const int S = pr.splits;
-    const int64_t base = pr.slot_base + local * S;
-    // Lanes over splits: global max, then weights 2^(m_s - M) and the total mass.
-    float M = NEG_INF;
-    for (int s0 = 0; s0 < S; s0 += 64) {
-        int s = s0 + lane;
-        M = fmaxf(M, s < S ? p.part_ml[(base + s) * 2] : NEG_INF);
-    }
-    M = wave_max(M);
-    float L = 0.0f;
-    for (int s0 = 0; s0 < S; s0 += 64) {
-        int s = s0 + lane;
-        if (s < S) {
-            float ms = p.part_ml[(base + s) * 2];
-            float ws = ms == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-            L += ws * p.part_ml[(base + s) * 2 + 1];
-        }
-    }
-    L = wave_sum(L);
-    bool bad_mass = !(L > 0.0f) || !is_finite_f(L);
-    float inv = 1.0f / L;
-    float o[8];
-    for (int i = 0; i < 8; ++i) o[i] = 0.0f;
-    for (int s0 = 0; s0 < S; s0 += 64) {
-        int s = s0 + lane;
-        float ws = 0.0f;
-        if (s < S) {
-            float ms = p.part_ml[(base + s) * 2];
-            ws = ms == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-        }
-        int n = S - s0 < 64 ? S - s0 : 64;
-        for (int j = 0; j < n; ++j) {
-            float wj = __shfl(ws, j, 64);
-            if (wj == 0.0f) continue;
-            const float *src = p.part_o + (base + s0 + j) * D;
-            for (int i = 0; i < 8; ++i) {
-                int d = lane + 64 * i;
-                if (d < D) o[i] += wj * src[d];
+    const int kvh = (int)(local / m_kv), prow = (int)(local % m_kv);
+    const int64_t part = pr.slot_base + local * S;
+    const float *ml = p.part_ml + 2 * part, *po = p.part_o + part * dp + d;
+    constexpr int W = 16;
+    float M = NEG_INF, L = 0.0f;
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < S; s0 += W) {
+        f32x2 mv[W];
+        f32x4 ov[W];
+        float M1 = M;
+#pragma unroll
+        for (int s = 0; s < W; ++s)
+            if (s0 + s < S) {
+                mv[s] = *gload_ptr<f32x2>(ml + 2 * (s0 + s));
+                ov[s] = *gload_ptr<f32x4>(po + (int64_t)(s0 + s) * dp);
             }
-        }
+#pragma unroll
+        for (int s = 0; s < W; ++s)
+            if (s0 + s < S) M1 = fmaxf(M1, mv[s][0]);
+        const float base = M1 == NEG_INF ? 0.0f : M1, corr = __builtin_amdgcn_exp2f(M - base);
+        L *= corr;
+        for (int e = 0; e < 4; ++e) o[e] *= corr;
+#pragma unroll
+        for (int s = 0; s < W; ++s)
+            if (s0 + s < S && mv[s][0] != NEG_INF) {
+                const float w = __builtin_amdgcn_exp2f(mv[s][0] - base);
+                L = __builtin_fmaf(w, mv[s][1], L);
+                for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(w, ov[s][e], o[e]);
+            }
+        M = M1;
     }
+    const bool bad_mass = !(L > 0.0f) || !is_finite_f(L);
+    const float inv = 1.0f / L;
     bool bad_out = false;
-    float *out = pr.out + (int64_t)t * Hq * D + (int64_t)h * D;
-    for (int i = 0; i < 8; ++i) {
-        int d = lane + 64 * i;
-        if (d < D) {
-            float v = o[i] * inv;
-            bad_out |= !is_finite_f(v);
-            out[d] = v;
-        }
+    float *out = pr.out + ((int64_t)(prow / G) * Hq + kvh * G + prow % G) * D + d;
+    for (int e = 0; e < 4; ++e) {
+        o[e] *= inv;
+        bad_out |= d + e < D && !is_finite_f(o[e]);
     }
+    if (d + 4 <= D) *reinterpret_cast<f32x4u *>(out) = o;
+    else
+        for (int e = 0; e < 4; ++e)
+            if (d + e < D) out[e] = o[e];
     raise_status(p, bad_mass, ST_BAD_MASS);
     raise_status(p, bad_out, ST_NONFINITE_OUTPUT);
 }
 
-// ---------------------------------------------------------------------------
-// Launch helpers (host side, same translation unit)
-// ---------------------------------------------------------------------------
+// The probabilities of one diagnostics row per workgroup, from the scores
+// attn_tile stored (in the probability buffer itself when the caller asked for
+// no scores): masked keys are exactly +0.
+__global__ __launch_bounds__(256) void attn_tile_probs(TileArgs a) {
+    const Params &p = a.p;
+    const Problem &pr = p.single;  // diagnostics are single-problem calls
+    const int G = p.group, Hq = p.query_heads;
+    const bool full = p.diag_mode == 1;
+    const int64_t hr = full ? (int64_t)blockIdx.x : (int64_t)Hq * pr.queries - 1;
+    const int h = (int)(hr / pr.queries), t = (int)(hr % pr.queries);
+    const int m_kv = pr.queries * G, S = pr.splits * a.kw;
+    const int64_t local = (int64_t)(h / G) * m_kv + (int64_t)t * G + h % G;
+    float M, L;
+    merged_stats(p.part_ml + 2 * (pr.slot_base + local * S), S, M, L);
+    const float inv = 1.0f / L;
+    int64_t lo, hi;
+    visible_range(p, pr, pr.q_pos0 + t, &lo, &hi);
+    const int64_t row = full ? hr * pr.keys : 0, end = full ? pr.keys : hi;
+    const float *xs = (p.scores ? p.scores : p.probs) + row;
+    for (int64_t key = (full ? 0 : lo) + threadIdx.x; key < end; key += 256) {
+        const float x = xs[key];
+        p.probs[row + key] = key >= lo && key < hi ? __builtin_amdgcn_exp2f(x * LOG2E - M) * inv : 0.0f;
+    }
+}
 
 }  // namespace tkh
+
+// Head sizes the kernel is built for (the smallest that holds `head_dim`), the
+// keys of its staged tile, and the 16-row groups of a workgroup.
+extern "C" int tkh_tile_head(int head_dim) {
+    return head_dim <= 64 ? 64 : (head_dim <= 128 ? 128 : (head_dim <= 256 ? 256 : 512));
+}
+extern "C" int tkh_tile_keys(int head_dim) { return tkh::tile_keys(tkh_tile_head(head_dim)); }
 
 // start/stop, when not null, are recorded around the kernel by the dispatch
 // itself (hipExtLaunchKernelGGL), so profiled durations exclude the host gap
 // that separate hipEventRecord calls would add.
-extern "C" hipError_t tkh_launch_generic(const tkh::Params *p, int dtype, hipStream_t stream,
-                                         hipEvent_t start, hipEvent_t stop) {
+extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStream_t stream,
+                                      hipEvent_t start, hipEvent_t stop) {
     using namespace tkh;
-    dim3 grid((unsigned)p->total_tiles), block(64);
-    if (dtype == F32)
-        hipExtLaunchKernelGGL((attn_generic<F32>), grid, block, 0, stream, start, stop, 0, *p);
-    else if (dtype == F16)
-        hipExtLaunchKernelGGL((attn_generic<F16>), grid, block, 0, stream, start, stop, 0, *p);
-    else if (dtype == BF16)
-        hipExtLaunchKernelGGL((attn_generic<BF16>), grid, block, 0, stream, start, stop, 0, *p);
-    else return hipErrorInvalidValue;
+    const int dp = tkh_tile_head(a->p.head_dim);
+    dim3 grid((unsigned)a->p.total_tiles), block(256);
+#define TKH_TILE(DT, DP)                                                                            \
+    if (dtype == DT && dp == DP) {                                                                  \
+        hipExtLaunchKernelGGL((attn_tile<DT, DP>), grid, block, 0, stream, start, stop, 0, *a);     \
+        return hipGetLastError();                                                                   \
+    }
+    TKH_TILE(F32, 64) TKH_TILE(F32, 128) TKH_TILE(F32, 256) TKH_TILE(F32, 512)
+    TKH_TILE(F16, 64) TKH_TILE(F16, 128) TKH_TILE(F16, 256) TKH_TILE(F16, 512)
+    TKH_TILE(BF16, 64) TKH_TILE(BF16, 128) TKH_TILE(BF16, 256) TKH_TILE(BF16, 512)
+#undef TKH_TILE
+    return hipErrorInvalidValue;
+}
+
+extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
+                                            hipEvent_t start, hipEvent_t stop) {
+    using namespace tkh;
+    const int64_t threads = total_rows * ((a->p.head_dim + 3) / 4);
+    dim3 grid((unsigned)((threads + 255) / 256)), block(256);
+    hipExtLaunchKernelGGL(attn_tile_merge, grid, block, 0, stream, start, stop, 0, *a, total_rows,
+                          tkh_tile_head(a->p.head_dim));
     return hipGetLastError();
 }
 
-extern "C" hipError_t tkh_launch_combine(const tkh::Params *p, int64_t total_rows,
-                                         hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+extern "C" hipError_t tkh_launch_tile_probs(const tkh::TileArgs *a, hipStream_t stream) {
     using namespace tkh;
-    dim3 grid((unsigned)((total_rows + 3) / 4)), block(256);
-    hipExtLaunchKernelGGL(attn_combine, grid, block, 0, stream, start, stop, 0, *p, total_rows);
+    const int64_t rows = a->p.diag_mode == 1 ? (int64_t)a->p.query_heads * a->p.single.queries : 1;
+    hipLaunchKernelGGL(attn_tile_probs, dim3((unsigned)rows), dim3(256), 0, stream, *a);
     return hipGetLastError();
 }

@@ -141,10 +141,10 @@ struct Params {
     float softcap_log2;     // softcap * log2(e): tanh units -> log2 units
     int64_t total_tiles;
     // split-K partials
-    float *part_o;          // per slot: [rows, D] (generic kernel), [D, rows] (chunk kernel)
+    float *part_o;          // per slot: [head size] (tile kernel), [D, rows] (chunk kernel)
     float *part_ml;         // [rows, splits, 2] (max in log2 units, mass)
     uint32_t *status;
-    // optional diagnostics (generic kernel only)
+    // optional diagnostics (tile kernel only)
     float *scores;
     float *probs;
     int32_t diag_mode;      // 0 none, 1 full [Hq, queries, keys], 2 last row [keys]
@@ -235,6 +235,13 @@ struct PrefillBatch {
 struct PrefillArgs {
     Params p;             // first: the single-problem path reads it at the kernel-argument base
     PrefillBatch b;
+};
+// The FP32 tile kernels' argument (attention.hip).
+struct TileArgs {
+    Params p;             // first: the single-problem path reads it at the kernel-argument base
+    int32_t rw;           // 16-row groups per workgroup (1, 2 or 4)
+    int32_t kw;           // waves sharing a row group's keys, each with a partial of its own
+    int32_t vec;          // every row starts on a whole 4-element chunk: vector loads
 };
 static_assert(sizeof(PrefillArgs) <= 4096, "kernel arguments");
 static_assert(sizeof(DecodeArgs) <= 4096, "kernel arguments");

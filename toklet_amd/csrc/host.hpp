@@ -138,6 +138,7 @@ struct tkh_context {
     int prefill16 = 1;           // four-wave launches at head_dim 128/256 on the 16-row kernel (0: never)
     int prefill16_groups = 64;   // split target of the 16-row kernel's launches (in 128-row workgroups)
     int prefill16_waves = 4;     // 16-row waves per workgroup: 4 (64-row blocks) or 8 (128-row blocks)
+    int tile_groups = 512;       // FP32 tile kernel: below this many row-block workgroups, split the keys
     // profiling: per launch, start/stop of the attention kernel and of the combine kernel
     bool profiling = false;
     std::vector<hipEvent_t> prof_events;
