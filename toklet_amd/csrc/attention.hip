@@ -24,6 +24,10 @@ namespace {
 // head sizes to 128 (four workgroups per CU), 66 KiB above (two).
 __host__ __device__ constexpr int tile_keys(int DP) { return DP <= 64 ? 64 : (DP <= 256 ? 32 : 16); }
 
+// Waves that share a row group's features: a wave holds the Q and context of at
+// most 128, so head sizes above that fit two waves per SIMD without spills.
+__host__ __device__ constexpr int tile_feature_waves(int DP) { return DP <= 128 ? 1 : DP / 128; }
+
 // Four consecutive stored elements.
 template <int DT> struct Raw4 { using T = uint32_t __attribute__((ext_vector_type(2))); };
 template <> struct Raw4<F32> { using T = u32x4; };
@@ -51,23 +55,21 @@ template <int DT> __device__ __forceinline__ f32x4 widen4(typename Raw4<DT>::T w
     return x;
 }
 
-// Elements [off, off + 4) of which the first n exist (the rest read as zero):
-// one vector load when every row of the launch allows it, else one by one.
-template <int DT>
-__device__ __forceinline__ typename Raw4<DT>::T load4(const void *base, int64_t off, int n, bool vec) {
+// Elements [off, off + 4) of a row of which the first n exist.  VEC (every row
+// starts on a whole chunk and ends with one): one vector load, the caller
+// keeps `off` inside the row.  Otherwise one by one, the rest zeros.
+template <int DT, bool VEC>
+__device__ __forceinline__ typename Raw4<DT>::T load4(const void *base, int64_t off, int n) {
     using T = typename Raw4<DT>::T;
-    T w{};
-    if (vec) {
-        if (n > 0) {
-            if constexpr (DT == F32) w = *gload_ptr<T>(reinterpret_cast<const float *>(base) + off);
-            else w = *gload_ptr<T>(reinterpret_cast<const uint16_t *>(base) + off);
-        }
-        return w;
+    if constexpr (VEC) {
+        if constexpr (DT == F32) return *gload_ptr<T>(reinterpret_cast<const float *>(base) + off);
+        else return *gload_ptr<T>(reinterpret_cast<const uint16_t *>(base) + off);
     }
+    T w{};
     for (int e = 0; e < 4; ++e)
         if (e < n) {
-            if constexpr (DT == F32) w[e] = reinterpret_cast<const uint32_t *>(base)[off + e];
-            else w[e >> 1] |= (uint32_t)reinterpret_cast<const uint16_t *>(base)[off + e] << (16 * (e & 1));
+            if constexpr (DT == F32) w[e] = *gload_ptr<uint32_t>(reinterpret_cast<const uint32_t *>(base) + off + e);
+            else w[e >> 1] |= (uint32_t)*gload_ptr<uint16_t>(reinterpret_cast<const uint16_t *>(base) + off + e) << (16 * (e & 1));
         }
     return w;
 }
@@ -107,23 +109,27 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 //
 // It replaced one wave per (query, head) on the vector unit, whose lanes each
 // read a key row of their own.  Per call: a 128-token FP32 chunk at offset
-// 1920 (14/2/64) with its append 1017 -> 40 us, a 512-token FP32 prompt 313 ->
-// 42 us, 128 queries over 1025 keys at 8/1/512 (bf16) 2240 -> 281 us, and 300
-// tokens of 16/8/128 with both diagnostics 243 -> 57 us.
-template <int DT, int DP>
-__global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
+// 1920 (14/2/64) with its append 1017 -> 25 us, a 512-token FP32 prompt 313 ->
+// 39 us, 128 queries over 1025 keys at 8/1/512 (bf16) 2240 -> 71 us, and 300
+// tokens of 16/8/128 with both diagnostics 243 -> 52 us.  (With each chunk's
+// load under a branch of its own the compiler waited for one before the next:
+// 40, 42, 281 and 57 us; whole 512-wide rows per wave spilled 390 registers.)
+template <int DT, int DP, bool VEC>
+__global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
-    constexpr int KT = tile_keys(DP), NB = KT / 16, FC = DP / 16, FB = DP / 64;
+    constexpr int KT = tile_keys(DP), NB = KT / 16, FS = tile_feature_waves(DP);
+    constexpr int DW = DP / FS, FC = DW / 16, FB = DW / 64;  // a wave's features
     constexpr int KS = DP + 4;               // staged K row stride
     constexpr int NCH = KT * DP / 4 / 256;   // 4-element chunks per thread and tile
     __shared__ __attribute__((aligned(16))) float kt[KT * KS];
     __shared__ __attribute__((aligned(16))) float vt[KT * DP];
+    __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? 4 * NB * 64 : 1];  // partial scores
     using Raw = typename Raw4<DT>::T;
     const Params &p = a.p;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int j = lane & 15, g = lane >> 4;
     const int G = p.group, Hq = p.query_heads, D = p.head_dim;
-    const bool vec = a.vec != 0, full_diag = p.diag_mode == 1;
+    const bool full_diag = p.diag_mode == 1;
 
     // XCD-major tile order (dispatch slot b runs on XCD b % 8): the row blocks
     // of one KV head, which read the same keys, share an XCD's L2.
@@ -142,7 +148,8 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
     const int m_kv = pr->queries * G, nseg = pr->nseg;
 
     const int rw = a.rw, kw = a.kw;
-    const int rg = wave % rw, ks = wave / rw;
+    const int fs = wave % FS, f0 = fs * DW;  // the wave's features start at f0
+    const int rg = wave / FS % rw, ks = wave / FS / rw;
     const int row0 = (rb * rw + rg) * 16;    // the wave's first packed row
     const bool active = ks < kw && row0 < m_kv;
     const int prow = row0 + j;
@@ -173,41 +180,57 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
     const int wlo = rel(w_lo), whi = active ? rel(w_hi) : 0;
     const int vlo = rel(v_lo), vhi = rel(v_hi);
 
+    // Features past the head are zeros in Q, K and V.  A vector load of one
+    // reads the row's last chunk instead, so that no load is under a branch: the
+    // loads of a tile stay in flight together.
+    const int last = D - 4;  // first feature of a row's last whole chunk
+    auto feature = [&](int d) { return VEC ? min(d, last) : d; };
     f32x4 q[FC];
     for (int c = 0; c < FC; ++c) {
-        const int d = 16 * c + 4 * g;
-        q[c] = widen4<DT>(load4<DT>(pr->q, (int64_t)t_row * pr->q_row_stride + (int64_t)h_row * D + d, D - d, vec));
+        const int d = f0 + 16 * c + 4 * g;
+        const int64_t at = (int64_t)t_row * pr->q_row_stride + (int64_t)h_row * D;
+        q[c] = widen4<DT>(load4<DT, VEC>(pr->q, at + feature(d), D - d));
     }
+    if constexpr (VEC)
+        for (int c = 0; c < FC; ++c)
+            if (f0 + 16 * c + 4 * g > last) q[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     // A thread's chunk m of a tile: row i / (DP / 4), features 4 (i % (DP / 4)).
     // Rows past the range read its last row (K: masked; V: zeroed on staging,
     // so a stored non-finite value outside the visible keys never meets a zero
-    // probability), features past the head are zeros.
+    // probability).
     constexpr int CPR = DP / 4;
     Raw kreg[NCH], vreg[NCH];
     auto fetch = [&](int t0) {
-        for (int m = 0; m < NCH; ++m) {
-            const int i = tid + 256 * m, c = i % CPR;
-            const int64_t key = lo + min(t0 + i / CPR, n - 1);
-            const void *kb, *vb;
-            int64_t off;
-            if (nseg == 1) {
-                kb = pr->seg[0].k;
-                vb = pr->seg[0].v;
-                off = (int64_t)kvh * pr->seg[0].head_stride + key * pr->seg[0].row_stride;
-            } else {
-                off = seg_select(pr, key, kvh, &kb, &vb);
+        if (nseg == 1) {
+            const void *kb = pr->seg[0].k, *vb = pr->seg[0].v;
+            const int64_t rs = pr->seg[0].row_stride, at = (int64_t)kvh * pr->seg[0].head_stride + lo * rs;
+#pragma unroll
+            for (int m = 0; m < NCH; ++m) {
+                const int i = tid + 256 * m, d = 4 * (i % CPR);
+                const int64_t off = at + min(t0 + i / CPR, n - 1) * rs + feature(d);
+                kreg[m] = load4<DT, VEC>(kb, off, D - d);
+                vreg[m] = load4<DT, VEC>(vb, off, D - d);
             }
-            kreg[m] = load4<DT>(kb, off + 4 * c, D - 4 * c, vec);
-            vreg[m] = load4<DT>(vb, off + 4 * c, D - 4 * c, vec);
+        } else {
+#pragma unroll
+            for (int m = 0; m < NCH; ++m) {
+                const int i = tid + 256 * m, d = 4 * (i % CPR);
+                const void *kb, *vb;
+                const int64_t off = seg_select(pr, lo + min(t0 + i / CPR, n - 1), kvh, &kb, &vb) + feature(d);
+                kreg[m] = load4<DT, VEC>(kb, off, D - d);
+                vreg[m] = load4<DT, VEC>(vb, off, D - d);
+            }
         }
     };
     auto stage = [&](int t0) {
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
         for (int m = 0; m < NCH; ++m) {
-            const int i = tid + 256 * m, r = i / CPR, c = i % CPR;
-            *reinterpret_cast<f32x4 *>(kt + r * KS + 4 * c) = widen4<DT>(kreg[m]);
-            const bool in = t0 + r >= vlo && t0 + r < vhi;
-            *reinterpret_cast<f32x4 *>(vt + r * DP + 4 * c) = in ? widen4<DT>(vreg[m]) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            const int i = tid + 256 * m, r = i / CPR, d = 4 * (i % CPR);
+            const bool head = !VEC || d <= last, in = t0 + r >= vlo && t0 + r < vhi;
+            *reinterpret_cast<f32x4 *>(kt + r * KS + d) = head ? widen4<DT>(kreg[m]) : zero;
+            *reinterpret_cast<f32x4 *>(vt + r * DP + d) = head && in ? widen4<DT>(vreg[m]) : zero;
         }
     };
 
@@ -226,40 +249,58 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
         stage(t0);
         __syncthreads();
         if (t0 + KT < n) fetch(t0 + KT);
+        // Scores of the wave's blocks: dots over its features, then, when waves
+        // share the features, the sum of their dots (the same order in each).
         f32x4 st[NB];
-        bool seen[NB];  // some row of the wave sees a key of the block
-        float tmax = NEG_INF;
+        bool seen[NB], scored[NB];  // some row of the wave sees a key of the block; its scores are wanted
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int k0 = t0 + 16 * b;
             const bool mine = active && b % kw == ks;
             seen[b] = mine && k0 < whi && k0 + 16 > wlo;
-            st[b] = f32x4{NEG_INF, NEG_INF, NEG_INF, NEG_INF};
-            if (!(seen[b] || (full_diag && mine && k0 < n))) continue;
+            scored[b] = seen[b] || (full_diag && mine && k0 < n);
             f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;  // two chains
-            const float *kr = kt + (16 * b + j) * KS + 4 * g;
+            if (scored[b]) {
+                const float *kr = kt + (16 * b + j) * KS + f0 + 4 * g;
 #pragma unroll
-            for (int c = 0; c < FC; c += 2) {
-                const f32x4 k0v = *reinterpret_cast<const f32x4 *>(kr + 16 * c);
-                const f32x4 k1v = *reinterpret_cast<const f32x4 *>(kr + 16 * c + 16);
-                for (int e = 0; e < 4; ++e) {
-                    s0 = mfma4(k0v[e], q[c][e], s0);
-                    s1 = mfma4(k1v[e], q[c + 1][e], s1);
+                for (int c = 0; c < FC; c += 2) {
+                    const f32x4 k0v = *reinterpret_cast<const f32x4 *>(kr + 16 * c);
+                    const f32x4 k1v = *reinterpret_cast<const f32x4 *>(kr + 16 * c + 16);
+                    for (int e = 0; e < 4; ++e) {
+                        s0 = mfma4(k0v[e], q[c][e], s0);
+                        s1 = mfma4(k1v[e], q[c + 1][e], s1);
+                    }
                 }
             }
-            f32x4 x;
-            for (int r = 0; r < 4; ++r) {
-                x[r] = (s0[r] + s1[r]) * scale;
-                if (cap != 0.0f) x[r] = softcap_f(x[r], cap);
+            for (int r = 0; r < 4; ++r) st[b][r] = s0[r] + s1[r];
+            if constexpr (FS > 1) dots[(wave * NB + b) * 64 + lane] = st[b];
+        }
+        if constexpr (FS > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const f32x4 *d = dots + (wave - fs) * NB * 64 + b * 64 + lane;
+                st[b] = d[0];
+                for (int w = 1; w < FS; ++w)
+                    for (int r = 0; r < 4; ++r) st[b][r] += d[w * NB * 64][r];
             }
-            const int key = k0 + 4 * g;
+        }
+        float tmax = NEG_INF;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (!scored[b]) continue;
+            f32x4 x;
+            for (int r = 0; r < 4; ++r) x[r] = st[b][r] * scale;
+            if (cap != 0.0f)
+                for (int r = 0; r < 4; ++r) x[r] = softcap_f(x[r], cap);
+            const int key = t0 + 16 * b + 4 * g;
             for (int r = 0; r < 4; ++r) {
                 const bool vis = key + r >= rlo && key + r < rhi;
                 bad |= vis && !is_finite_f(x[r]);
                 st[b][r] = vis ? x[r] * LOG2E : NEG_INF;
                 tmax = fmaxf(tmax, st[b][r]);
             }
-            if (p.diag_mode != 0 && rvalid && (full_diag || last_row)) {
+            if (fs == 0 && p.diag_mode != 0 && rvalid && (full_diag || last_row)) {
                 const int first = full_diag ? 0 : rlo, end = full_diag ? n : rhi;
                 float *xr = xs + (full_diag ? ((int64_t)h_row * pr->queries + t_row) * keys : 0) + lo + key;
                 if (key >= first && key + 4 <= end) *reinterpret_cast<f32x4u *>(xr) = x;
@@ -290,7 +331,7 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float *vr = vt + (16 * b + 4 * g + r) * DP + 4 * j;
+                const float *vr = vt + (16 * b + 4 * g + r) * DP + f0 + 4 * j;
                 for (int fb = 0; fb < FB; ++fb) {
                     const f32x4 v = *reinterpret_cast<const f32x4 *>(vr + 64 * fb);
                     for (int e = 0; e < 4; ++e) acc[fb][e] = mfma4(v[e], st[b][r], acc[fb][e]);
@@ -304,7 +345,7 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
     bool bad_mass = false, bad_out = false;
     if (rvalid) {
         const int64_t part = pr->slot_base + ((int64_t)kvh * m_kv + prow) * (ns * kw) + split * kw + ks;
-        if (g == 0 && (!direct || p.diag_mode != 0)) {
+        if (g == 0 && fs == 0 && (!direct || p.diag_mode != 0)) {
             const f32x2 ml = {m_run, l_run};
             *gstore_ptr<f32x2>(p.part_ml + 2 * part) = ml;
         }
@@ -313,7 +354,7 @@ __global__ __launch_bounds__(256) void attn_tile(TileArgs a) {
         float *orow = direct ? pr->out + ((int64_t)t_row * Hq + h_row) * D : p.part_o + part * DP;
         for (int fb = 0; fb < FB; ++fb)
             for (int r = 0; r < 4; ++r) {
-                const int d = 64 * fb + 16 * g + 4 * r;
+                const int d = f0 + 64 * fb + 16 * g + 4 * r;
                 f32x4 o;
                 for (int e = 0; e < 4; ++e) {
                     o[e] = acc[fb][e][r];
@@ -442,11 +483,12 @@ __global__ __launch_bounds__(256) void attn_tile_probs(TileArgs a) {
 }  // namespace tkh
 
 // Head sizes the kernel is built for (the smallest that holds `head_dim`), the
-// keys of its staged tile, and the 16-row groups of a workgroup.
+// keys of its staged tile, and the row groups a workgroup has waves for.
 extern "C" int tkh_tile_head(int head_dim) {
     return head_dim <= 64 ? 64 : (head_dim <= 128 ? 128 : (head_dim <= 256 ? 256 : 512));
 }
 extern "C" int tkh_tile_keys(int head_dim) { return tkh::tile_keys(tkh_tile_head(head_dim)); }
+extern "C" int tkh_tile_row_waves(int head_dim) { return 4 / tkh::tile_feature_waves(tkh_tile_head(head_dim)); }
 
 // start/stop, when not null, are recorded around the kernel by the dispatch
 // itself (hipExtLaunchKernelGGL), so profiled durations exclude the host gap
@@ -456,10 +498,11 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
     using namespace tkh;
     const int dp = tkh_tile_head(a->p.head_dim);
     dim3 grid((unsigned)a->p.total_tiles), block(256);
-#define TKH_TILE(DT, DP)                                                                            \
-    if (dtype == DT && dp == DP) {                                                                  \
-        hipExtLaunchKernelGGL((attn_tile<DT, DP>), grid, block, 0, stream, start, stop, 0, *a);     \
-        return hipGetLastError();                                                                   \
+#define TKH_TILE(DT, DP)                                                                               \
+    if (dtype == DT && dp == DP) {                                                                     \
+        if (a->vec) hipExtLaunchKernelGGL((attn_tile<DT, DP, true>), grid, block, 0, stream, start, stop, 0, *a); \
+        else hipExtLaunchKernelGGL((attn_tile<DT, DP, false>), grid, block, 0, stream, start, stop, 0, *a);       \
+        return hipGetLastError();                                                                      \
     }
     TKH_TILE(F32, 64) TKH_TILE(F32, 128) TKH_TILE(F32, 256) TKH_TILE(F32, 512)
     TKH_TILE(F16, 64) TKH_TILE(F16, 128) TKH_TILE(F16, 256) TKH_TILE(F16, 512)
