@@ -37,7 +37,8 @@ extern "C" hipError_t tkh_launch_kv_append(int src, int dst, const void *k, cons
                                            uint32_t *status, hipStream_t stream);
 extern "C" hipError_t tkh_launch_check_finite(int dtype, const void *a, const void *b, int64_t n,
                                               uint32_t *status, hipStream_t stream);
-extern "C" hipError_t tkh_launch_softcap(float *x, int64_t n, float cap, uint32_t *status,
+extern "C" int tkh_softcap_verdicts(void);
+extern "C" hipError_t tkh_launch_softcap(float *x, int64_t n, float cap, uint32_t *verdict, uint32_t *status,
                                          hipStream_t stream);
 extern "C" hipError_t tkh_launch_fill_u32(uint32_t *p, uint32_t v, hipStream_t stream);
 extern "C" hipError_t tkh_launch_zero_u64(uint64_t *p, int64_t words, hipStream_t stream);
@@ -878,8 +879,10 @@ uint32_t tkh_context_create(int device, void *stream, size_t workspace_bytes, in
     // The caller's stream, or the device's null stream: work is ordered with
     // whatever the caller queued there (no private stream, no priorities).
     ctx->stream = reinterpret_cast<hipStream_t>(stream);
-    if ((e = hipMalloc(&ctx->status_dev, 256)) != hipSuccess) return cleanup(e, "status");
-    if ((e = hipMemset(ctx->status_dev, 0, 256)) != hipSuccess) return cleanup(e, "status");
+    const size_t status_bytes = 256 + sizeof(uint32_t) * tkh_softcap_verdicts();
+    if ((e = hipMalloc(&ctx->status_dev, status_bytes)) != hipSuccess) return cleanup(e, "status");
+    if ((e = hipMemset(ctx->status_dev, 0, status_bytes)) != hipSuccess) return cleanup(e, "status");
+    ctx->verdict_dev = ctx->status_dev + 256 / sizeof(uint32_t);
     if ((e = hipHostMalloc(&ctx->status_host, sizeof(uint32_t), hipHostMallocDefault)) != hipSuccess)
         return cleanup(e, "status");
     if ((e = hipMalloc(&ctx->workspace, ctx->workspace_bytes)) != hipSuccess)
@@ -1443,7 +1446,7 @@ uint32_t tkh_logit_softcap(tkh_context *ctx, float *logits, uint64_t len, float 
     if (!std::isfinite(cap) || cap <= 0.0f) return invalid("logit softcap", err);
     if (!ctx) return invalid("context", err);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
-    HIP_TRY(tkh_launch_softcap(logits, (int64_t)len, cap, ctx->status_dev, ctx->stream), "softcap");
+    HIP_TRY(tkh_launch_softcap(logits, (int64_t)len, cap, ctx->verdict_dev, ctx->status_dev, ctx->stream), "softcap");
     return after_launch(ctx, err);
 }
 

@@ -100,6 +100,7 @@ struct tkh_context {
     hipStream_t stream = nullptr;
     bool synchronous = true;
     uint32_t *status_dev = nullptr;
+    uint32_t *verdict_dev = nullptr;  // the softcap check's words, in status_dev's allocation
     uint32_t *status_host = nullptr;
     uint8_t *workspace = nullptr;
     size_t workspace_bytes = 0;

@@ -139,20 +139,60 @@ __global__ __launch_bounds__(256) void check_finite(const void *a, const void *b
     flag(status, bad, ST_NONFINITE_INPUT);
 }
 
-// Single block: the whole input is checked (block-wide OR) before any write,
-// as the reference checks finiteness before writing (src/cpu/softcap.rs:20-23).
-__global__ __launch_bounds__(256) void logit_softcap(float *x, int64_t n, float cap,
-                                                     uint32_t *status) {
-    const double c = (double)cap;
-    int bad = 0;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) bad |= !is_finite_f(x[i]);
-    bad = __syncthreads_or(bad);
-    if (bad) {
+// cap * tanh(x / cap), where the whole input is checked before any write, as
+// the reference checks finiteness before writing (src/cpu/softcap.rs:20-23).
+// The FP64 tanh bounds it (about 100 FP64 instructions per value).  Up to
+// SOFTCAP_ONE values one workgroup holds the input in registers, so the check
+// and the result are one launch; above, a check launch stores one verdict per
+// workgroup and the next launch's workgroups each read all of them, so no
+// word has to be cleared between calls and a captured call replays.  One
+// workgroup for every size took 725 us for 262,144 logits, the two launches
+// 3.3 + 4.1 us.  The line between the forms: back to back, one workgroup takes
+// 4.5 us for 2,048 values and 7.3 for 4,096, two launches 6.7 for either.
+constexpr int SOFTCAP_ONE = 2048, SOFTCAP_CHECKS = 256;
+
+__device__ __forceinline__ float softcap_f64(float x, double c) { return (float)(tanh((double)x / c) * c); }
+
+__global__ __launch_bounds__(1024) void softcap_one(float *x, int n, float cap, uint32_t *status) {
+    constexpr int PER = SOFTCAP_ONE / 1024;
+    float v[PER];
+    bool bad = false;
+    for (int k = 0; k < PER; ++k) {
+        const int i = threadIdx.x + 1024 * k;
+        v[k] = i < n ? x[i] : 0.0f;
+        bad |= !is_finite_f(v[k]);
+    }
+    if (__syncthreads_or(bad)) {
         if (threadIdx.x == 0) atomicOr(status, (uint32_t)ST_NONFINITE_INPUT);
         return;
     }
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x)
-        x[i] = (float)(tanh((double)x[i] / c) * c);
+    for (int k = 0; k < PER; ++k) {
+        const int i = threadIdx.x + 1024 * k;
+        if (i < n) x[i] = softcap_f64(v[k], (double)cap);
+    }
+}
+
+__global__ __launch_bounds__(256) void softcap_check(const float *x, int64_t n, uint32_t *verdict,
+                                                     uint32_t *status) {
+    int bad = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += SOFTCAP_CHECKS * 256)
+        bad |= !is_finite_f(x[i]);
+    bad = __syncthreads_or(bad);
+    if (threadIdx.x != 0) return;
+    verdict[blockIdx.x] = bad ? 1u : 0u;
+    if (bad) atomicOr(status, (uint32_t)ST_NONFINITE_INPUT);
+}
+
+__global__ __launch_bounds__(256) void softcap_apply(float *x, int64_t n, float cap, const uint32_t *verdict) {
+    static_assert(SOFTCAP_CHECKS == 256, "one verdict per thread");
+    const double c = (double)cap;
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    float v = i0 < n ? x[i0] : 0.0f;  // with the verdicts: one memory round trip
+    if (__syncthreads_or(verdict[threadIdx.x] != 0)) return;
+    for (int64_t i = i0; i < n; i += step) {
+        if (i != i0) v = x[i];
+        x[i] = softcap_f64(v, c);
+    }
 }
 
 template <int DT>
@@ -231,9 +271,19 @@ extern "C" hipError_t tkh_launch_check_finite(int dtype, const void *a, const vo
     return hipGetLastError();
 }
 
-extern "C" hipError_t tkh_launch_softcap(float *x, int64_t n, float cap, uint32_t *status,
+extern "C" int tkh_softcap_verdicts(void) { return tkh::SOFTCAP_CHECKS; }
+
+// `verdict`: tkh_softcap_verdicts() words of device scratch.
+extern "C" hipError_t tkh_launch_softcap(float *x, int64_t n, float cap, uint32_t *verdict, uint32_t *status,
                                          hipStream_t stream) {
-    hipLaunchKernelGGL(logit_softcap, dim3(1), dim3(256), 0, stream, x, n, cap, status);
+    if (n <= SOFTCAP_ONE) {
+        hipLaunchKernelGGL(softcap_one, dim3(1), dim3(1024), 0, stream, x, (int)n, cap, status);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(softcap_check, dim3(SOFTCAP_CHECKS), dim3(256), 0, stream, x, n, verdict, status);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(softcap_apply, dim3(grid_for(n)), dim3(256), 0, stream, x, n, cap, verdict);
     return hipGetLastError();
 }
 
