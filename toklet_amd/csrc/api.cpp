@@ -70,6 +70,12 @@ extern "C" hipError_t tkh_launch_decode(const tkh::DecodeArgs *p, int dtype, int
                                         int keys_per_lane, int waves, int64_t groups, int fused,
                                         hipStream_t stream, hipEvent_t start, hipEvent_t stop);
 
+extern "C" hipError_t tkh_launch_decode_layers(const tkh::DecodeLayersArgs *a, int dtype, int head_dim, int rows,
+                                               int keys_per_lane, int waves, int64_t groups, hipStream_t stream,
+                                               hipEvent_t start, hipEvent_t stop);
+extern "C" hipError_t tkh_launch_decode_merge_layers(const tkh::DecodeLayersArgs *a, int head_dim, int rows,
+                                                     hipStream_t stream, hipEvent_t start, hipEvent_t stop);
+
 using namespace tkh_host;
 
 namespace {
@@ -255,9 +261,18 @@ tkh::Params base_params(tkh_context *ctx, const Plan &plan) {
     return prm;
 }
 
-// Few query rows per KV head: the streaming decode kernel, one launch.
-uint32_t launch_decode(tkh_context *ctx, const Plan &plan, Problems group,
-                       int rows, tkh_error *err) {
+// How a decode launch covers its problems (plan_decode): the kernel build, the
+// waves per workgroup and the split layout.
+struct DecodePlan {
+    int R, u, nw;
+    int64_t wgs, slots, split_keys;
+    bool bulk, split;
+    size_t flag_bytes;
+};
+
+// Splits and waves of a decode launch of `group`, whose planning fields are
+// filled in place.
+uint32_t plan_decode(tkh_context *ctx, const Plan &plan, Problems group, int rows, DecodePlan *out, tkh_error *err) {
     const int64_t D = plan.head_dim, Hkv = plan.kv_heads;
     const int R = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
     double work = 0;
@@ -368,6 +383,20 @@ uint32_t launch_decode(tkh_context *ctx, const Plan &plan, Problems group,
     if (part_bytes > (size_t)INT32_MAX)
         return fail(err, TKH_UNSUPPORTED, "workspace", 0, (size_t)INT32_MAX, part_bytes,
                     "decode partials of %zu bytes exceed the merge's 2 GiB range", part_bytes);
+    *out = DecodePlan{R, u, nw, wgs, slots, sk, bulk, any_split, flag_bytes};
+    return TKH_OK;
+}
+
+// Few query rows per KV head: the streaming decode kernel, one launch.
+uint32_t launch_decode(tkh_context *ctx, const Plan &plan, Problems group,
+                       int rows, tkh_error *err) {
+    const int64_t D = plan.head_dim, Hkv = plan.kv_heads;
+    DecodePlan dp;
+    TRY(plan_decode(ctx, plan, group, rows, &dp, err));
+    const int R = dp.R, u = dp.u, nw = dp.nw;
+    const int64_t wgs = dp.wgs, slots = dp.slots, sk = dp.split_keys;
+    const bool bulk = dp.bulk, split = dp.split;
+    const size_t flag_bytes = dp.flag_bytes;
 
     // Up to DECODE_BATCH_MAX single-token sessions laid out as tkh_decode_batch
     // lays them out (Q/context rows consecutive, K and V at one offset from
@@ -416,8 +445,6 @@ uint32_t launch_decode(tkh_context *ctx, const Plan &plan, Problems group,
     if (group.size() == 1) prm.single = group[0];
     prm.nproblems = (int32_t)group.size();
     prm.total_tiles = wgs;
-    bool split = false;
-    for (auto &p : group) split |= p.splits > 1;
     if (split && ++ctx->epoch == 0) {
         // The epoch wrapped: clear every flag so no stale one can match again.
         HIP_TRY(tkh_launch_zero_u64(reinterpret_cast<uint64_t *>(decode_region(ctx)),
@@ -793,6 +820,77 @@ uint32_t run(tkh_context *ctx, Plan &plan, tkh_error *err) {
 }
 
 
+// Whether two ranges of device memory share a byte.
+bool overlap(const void *a, uint64_t na, const void *b, uint64_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && b && x < y + nb && y < x + na;
+}
+
+// Whether layer `a` writes something that layer `b` reads or writes (contexts
+// against inputs and contexts), so that their order matters.
+bool layer_feeds(const tkh::DecodeLayer &a, const tkh::DecodeLayer &b, uint64_t hq, uint64_t hkv, uint64_t d) {
+    const uint64_t q = hq * d * sizeof(float), k = hkv * d * sizeof(float), w = d * sizeof(float);
+    const tkh::FusedDecode &f = b.fused;
+    return overlap(a.pr.out, q, b.pr.out, q) || overlap(a.pr.out, q, f.q_proj, q) || overlap(a.pr.out, q, f.k_proj, k) ||
+           overlap(a.pr.out, q, f.v_proj, k) || overlap(a.pr.out, q, f.q_norm, w) || overlap(a.pr.out, q, f.k_norm, w);
+}
+
+// The launch of a fused decode step: at once, or into `batch` (the step of a
+// session whose layers' inputs were all given together).  A layer joins the
+// batch when it is combined by the merge launch or not split, and neither it nor a
+// layer in the batch reads or overwrites what the other writes.
+uint32_t run_fused(tkh_context *ctx, Plan &plan, DecodeBatchOfLayers *batch, tkh_error *err) {
+    if (!batch) return run(ctx, plan, err);
+    const int64_t D = plan.head_dim, Hkv = plan.kv_heads, G = plan.query_heads / Hkv;
+    const int limit = tkh_decode_max_rows((int)plan.dtype, (int)D);
+    DecodePlan dp{};
+    bool joins = G <= limit && (plan.softcap == 0.0f || D == 256) && !ctx->test_flag_skew;
+    if (joins) {
+        TRY(plan_decode(ctx, plan, Problems{plan.store, 1}, (int)G, &dp, err));
+        joins = !dp.split || (!dp.bulk && ctx->decode_merge_launch);
+    }
+    if (!joins) {
+        TRY(flush_decode_layers(ctx, batch, err));
+        return run(ctx, plan, err);
+    }
+    tkh::DecodeLayersArgs &a = batch->args;
+    tkh::DecodeLayer e{};
+    e.pr = plan.store[0];
+    e.fused = *plan.fused;
+    e.has_window = plan.has_window ? 1 : 0;
+    e.window = plan.window;
+    e.nw = dp.nw;
+    auto part_bytes = [&](int64_t slots) { return (size_t)slots * dp.R * (D + 2) * sizeof(float); };
+    bool fits = a.count < tkh::DECODE_LAYERS_MAX && (a.count == 0 || (dp.R == batch->R && dp.u == batch->u));
+    const size_t all = part_bytes(batch->slots + dp.slots);
+    fits = fits && all <= (size_t)INT32_MAX && all <= decode_region_bytes(ctx);
+    for (int i = 0; i < a.count && fits; ++i)
+        fits = !layer_feeds(a.e[i], e, plan.query_heads, Hkv, D) && !layer_feeds(e, a.e[i], plan.query_heads, Hkv, D);
+    if (!fits) TRY(flush_decode_layers(ctx, batch, err));
+    if (a.count == 0) {
+        a.p = base_params(ctx, plan);
+        a.p.nproblems = 1;
+        a.p.merge_launch = 1;
+        a.p.stream_nt = ctx->decode_stream_nt < 0 ? 0 : ctx->decode_stream_nt;
+        batch->dtype = (int)plan.dtype;
+        batch->R = dp.R;
+        batch->u = dp.u;
+        batch->nw = 0;
+        batch->wgs = batch->slots = 0;
+        batch->split = false;
+    }
+    if (dp.bulk && ctx->decode_stream_nt < 0) a.p.stream_nt = 1;
+    e.pr.tile_base = batch->wgs;
+    e.pr.slot_base = batch->slots;
+    a.first[a.count] = (int32_t)batch->wgs;
+    a.e[a.count++] = e;
+    batch->nw = std::max(batch->nw, dp.nw);
+    batch->wgs += dp.wgs;
+    batch->slots += dp.slots;
+    batch->split |= dp.split;
+    return ok(err);
+}
+
 // The planner's settings of a context on `device`: the defaults, each
 // overridable by a TKH_* environment variable, and the device's CU count.
 void init_tuning(tkh_context *ctx, int device) {
@@ -852,6 +950,42 @@ uint64_t first_visible(uint64_t key_start, uint64_t position, bool has_window, u
 }
 
 }  // namespace
+
+// The batched layers' launch, and the merge of those that are split.  The flags
+// of the decode region's layout are not used: the merge launch orders the
+// partials, which take the region from its start.
+uint32_t tkh_host::flush_decode_layers(tkh_context *ctx, DecodeBatchOfLayers *batch, tkh_error *err) {
+    tkh::DecodeLayersArgs &a = batch->args;
+    if (a.count == 0) return TKH_OK;
+    const int count = a.count, D = a.p.head_dim;
+    if (hipSetDevice(ctx->device) != hipSuccess)
+        return fail(err, TKH_DEVICE, "device", 0, 0, 0, "hipSetDevice failed");
+    a.p.total_tiles = batch->wgs;
+    a.p.part_ml = reinterpret_cast<float *>(decode_region(ctx));
+    a.p.part_o = a.p.part_ml + (size_t)batch->slots * batch->R * 2;
+    hipEvent_t *ev = nullptr;
+    if (ctx->profiling) TRY(profile_slot(ctx, &ev, batch->split, err));
+    hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr, e2 = ev ? ev[2] : nullptr, e3 = ev ? ev[3] : nullptr;
+    hipError_t e;
+    if (count > 1) {
+        e = tkh_launch_decode_layers(&a, batch->dtype, D, batch->R, batch->u, batch->nw, batch->wgs, ctx->stream, e0, e1);
+        if (e == hipSuccess && batch->split) e = tkh_launch_decode_merge_layers(&a, D, batch->R, ctx->stream, e2, e3);
+    } else {
+        // One layer: its own launch, whose problem needs no lookup.
+        tkh::DecodeArgs one{};
+        one.p = a.p;
+        one.p.single = a.e[0].pr;
+        one.p.fused = a.e[0].fused;
+        one.p.has_window = a.e[0].has_window;
+        one.p.window = a.e[0].window;
+        e = tkh_launch_decode(&one, batch->dtype, D, batch->R, batch->u, batch->nw, batch->wgs, 1, ctx->stream, e0, e1);
+        if (e == hipSuccess && batch->split)
+            e = tkh_launch_decode_merge(&one.p, D, batch->R, a.p.kv_heads, ctx->stream, e2, e3);
+    }
+    a.count = 0;
+    if (e != hipSuccess) return device_error(e, count > 1 ? "decode layers launch" : "decode launch", err);
+    return after_launch(ctx, err);
+}
 
 extern "C" {
 
@@ -1121,7 +1255,7 @@ uint32_t tkh_attention_cached_static(int device, void *stream, const tkh_cached_
 uint32_t tkh_host::attention_cached_fused(tkh_context *ctx, const tkh_cached_shape *shape,
                                           tkh_dtype dtype, const void *k, const void *v,
                                           float *context, const tkh::FusedDecode &fused,
-                                          tkh_error *err) {
+                                          DecodeBatchOfLayers *batch, tkh_error *err) {
     if (!valid_dtype(dtype)) return invalid("dtype", err);
     if (!shape || !ctx) return invalid("shape", err);
     const tkh_cached_shape s = *shape;
@@ -1145,13 +1279,13 @@ uint32_t tkh_host::attention_cached_fused(tkh_context *ctx, const tkh_cached_sha
     tkh::Problem p = make_problem(nullptr, context, s.query_heads * s.head_dim, s.offset, 0, end, 1);
     add_segment(p, k, v, s.capacity * s.head_dim, s.head_dim, end, 0);
     plan.add(p);
-    return run(ctx, plan, err);
+    return run_fused(ctx, plan, batch, err);
 }
 
 uint32_t tkh_host::span_attention_fused(tkh_context *ctx, const tkh_span_shape *shape,
                                         tkh_dtype dtype, const tkh_segment segments[3],
                                         float *context, const tkh::FusedDecode &fused,
-                                        tkh_error *err) {
+                                        DecodeBatchOfLayers *batch, tkh_error *err) {
     if (!valid_dtype(dtype)) return invalid("dtype", err);
     if (!ctx || !shape || !segments) return invalid("shape", err);
     const tkh_span_shape s = *shape;
@@ -1192,7 +1326,7 @@ uint32_t tkh_host::span_attention_fused(tkh_context *ctx, const tkh_span_shape *
     }
     if (logical != s.keys) return invalid("attention segment keys", err);
     plan.add(p);
-    return run(ctx, plan, err);
+    return run_fused(ctx, plan, batch, err);
 }
 
 extern "C" {

@@ -187,7 +187,41 @@ __global__ __launch_bounds__(64) void attn_decode_merge_batch(Params p, DecodeBa
     const MergeFields mf{p.group, p.query_heads, p.part_ml, p.part_o, p.status};
     merge_chunk<D>(mf, rows, S, (int64_t)e.tile_base, bt.out + (int64_t)i * p.query_heads * D, kvh, r, c);
 }
+// The same for a step of several layers (attn_decode_layers): the layers share
+// Hkv, the GQA group and D, so wave b serves layer b / (Hkv G D/64).
+template <int D>
+__global__ __launch_bounds__(64) void attn_decode_merge_layers(DecodeLayersArgs a, int rows) {
+    constexpr int CH = D / 64;
+    const_ptr<DecodeLayersArgs> args = (const_ptr<DecodeLayersArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+    const Params &p = a.p;
+    const uint32_t G = (uint32_t)p.group, per = (uint32_t)p.kv_heads * G * CH;
+    const uint32_t i = blockIdx.x / per, b = blockIdx.x % per;
+    const_ptr<Problem> pr = &args->e[i].pr;
+    const int S = pr->splits;
+    if (S <= 1) return;
+    const int c = (int)(b % CH), r = (int)(b / CH % G), kvh = (int)(b / (CH * G));
+    const MergeFields mf{p.group, p.query_heads, p.part_ml, p.part_o, p.status};
+    merge_chunk<D>(mf, rows, S, pr->slot_base, pr->out, kvh, r, c);
+}
 }  // namespace tkh
+
+// A step of several layers: fields as tkh_launch_decode's.
+extern "C" hipError_t tkh_launch_decode_layers(const tkh::DecodeLayersArgs *a, int dtype, int head_dim, int rows,
+                                               int keys_per_lane, int waves, int64_t groups, hipStream_t stream,
+                                               hipEvent_t start, hipEvent_t stop) {
+    return tkh_launch_decode(reinterpret_cast<const tkh::DecodeArgs *>(a), dtype, head_dim, rows, keys_per_lane, waves,
+                             groups, 2, stream, start, stop);
+}
+extern "C" hipError_t tkh_launch_decode_merge_layers(const tkh::DecodeLayersArgs *a, int head_dim, int rows,
+                                                     hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+    using namespace tkh;
+    const dim3 grid((unsigned)(a->count * a->p.kv_heads * a->p.group * (head_dim / 64))), block(64);
+    if (head_dim == 64) hipExtLaunchKernelGGL(attn_decode_merge_layers<64>, grid, block, 0, stream, start, stop, 0, *a, rows);
+    else if (head_dim == 128) hipExtLaunchKernelGGL(attn_decode_merge_layers<128>, grid, block, 0, stream, start, stop, 0, *a, rows);
+    else if (head_dim == 256) hipExtLaunchKernelGGL(attn_decode_merge_layers<256>, grid, block, 0, stream, start, stop, 0, *a, rows);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
 
 extern "C" hipError_t tkh_launch_decode_merge_batch(const tkh::DecodeArgs *a, int head_dim, int rows,
                                                      hipStream_t stream, hipEvent_t start, hipEvent_t stop) {

@@ -345,9 +345,13 @@ __device__ __forceinline__ int find_batch_entry(const_ptr<DecodeBatch> b, int co
     return __builtin_amdgcn_readfirstlane(63 - __builtin_clzll(m));
 }
 
-template <int DT, int D, int R, int U, bool CAP, bool FUSED>
-__global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void attn_decode(DecodeArgs kargs) {
-    const Params &p = kargs.p;
+// LAYERS: a session step of several layers (attn_decode_layers), each
+// workgroup's problem, window and producer descriptor taken from its layer's
+// entry; splits are combined by the merge launch.  Each layer keeps the splits
+// and streaming waves of its own launch, so its context has the same bits.
+template <int DT, int D, int R, int U, bool CAP, bool FUSED, bool LAYERS>
+__device__ __forceinline__ void decode_body(const Params &p) {
+    static_assert(FUSED || !LAYERS, "layers are session steps");
     constexpr int ES = Elem<DT>::size;
     constexpr int NWMAX = decode_waves_for(D * ES, R);
     constexpr int ROWB = D * ES;            // bytes per K/V row
@@ -368,7 +372,8 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
     __shared__ u32x4 lds_q[FUSED ? R * CPL * 8 : 1];
     __shared__ float lds_prow[FUSED ? NWMAX * D : 1];
 
-    const int nw = blockDim.x >> 6;
+    const int block_waves = blockDim.x >> 6;
+    int nw = block_waves;  // waves that stream keys
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int sub = lane & 7;   // which chunks of the row
@@ -382,7 +387,17 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
     const_ptr<DecodeArgs> dargs = (const_ptr<DecodeArgs>)__builtin_amdgcn_kernarg_segment_ptr();
     const_ptr<Params> args = &dargs->p;
     const_ptr<DecodeBatch> batch = &dargs->b;
-    const_ptr<Problem> pr = &args->single;
+    const_ptr<DecodeLayersArgs> largs = (const_ptr<DecodeLayersArgs>)dargs;
+    int layer = 0;
+    if constexpr (LAYERS) {
+        // The layers' first workgroups share a line: one trip, then the
+        // entry's fields in the batch below.
+        const int count = largs->count;
+        for (int i = 1; i < DECODE_LAYERS_MAX; ++i)
+            layer = i < count && (int)blockIdx.x >= largs->first[i] ? i : layer;
+    }
+    const_ptr<DecodeLayer> entry = &largs->e[layer];
+    const_ptr<Problem> pr = LAYERS ? &entry->pr : &args->single;
     // Every kernel-argument field the prologue and the stream need, read
     // before the first use of any (the pins below then cost one wait): the
     // problem view, the launch fields and the fused producer's descriptor.  A
@@ -390,17 +405,20 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
     DecodeView pv = decode_view(pr);
     int64_t slot_base = pr->slot_base;
     float *out = pr->out;
-    int nproblems = args->nproblems;
-    int bcount = batch->count;
-    int G = args->group, Hq = args->query_heads, has_window = args->has_window;
-    int64_t window = args->window;
+    int nproblems = LAYERS ? 1 : args->nproblems;
+    int bcount = LAYERS ? 0 : batch->count;
+    int G = args->group, Hq = args->query_heads;
+    int has_window = LAYERS ? entry->has_window : args->has_window;
+    int64_t window = LAYERS ? entry->window : args->window;
+    if constexpr (LAYERS) nw = entry->nw;
     float scale_log2 = args->scale_log2;
     // Capped score in log2 units: tanh(raw * scale / cap) * cap * log2(e).
     float ycap = args->softcap_y, caplog2 = args->softcap_log2;
     int stream_nt = args->stream_nt;
     FusedDecode fz{};
     if constexpr (FUSED) {
-        const auto &fa = args->fused;
+        const_ptr<FusedDecode> fp = LAYERS ? &entry->fused : &args->fused;
+        const auto &fa = *fp;
         fz.q_proj = fa.q_proj;
         fz.k_proj = fa.k_proj;
         fz.v_proj = fa.v_proj;
@@ -415,8 +433,12 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
         fz.new_key = fa.new_key;
         fz.new_row = fa.new_row;
     }
-    pin_scalar(nproblems);
-    pin_scalar(bcount);
+    if constexpr (LAYERS) {
+        pin_scalar(nw);
+    } else {
+        pin_scalar(nproblems);
+        pin_scalar(bcount);
+    }
     pin_scalar(slot_base);
     pin_scalar(out);
     pin_view(pv);
@@ -443,7 +465,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
         pin_scalar(fz.new_key);
         pin_scalar(fz.new_row);
     }
-    if (bcount > 0) {
+    if (!LAYERS && bcount > 0) {
         // A compact batch: one segment, one query token at the last key.
         const int i = find_batch_entry(batch, bcount, blockIdx.x);
         const auto &e = batch->e[i];
@@ -469,7 +491,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
                                 (int64_t)head_stride, D, (int64_t)keys, 0};
         slot_base = tile_base;
         out = batch->out + (int64_t)i * row;
-    } else if (nproblems != 1) {
+    } else if (!LAYERS && nproblems != 1) {
         pr = (const_ptr<Problem>)p.problems + find_problem_wave(p.problems, p.nproblems, blockIdx.x);
         pv = decode_view(pr);
         slot_base = pr->slot_base;
@@ -554,7 +576,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
             const FusedDecode &f = fz;
             const int jobs = nrows + (rel_new >= 0 ? 2 : 0);
             float *row = lds_prow + wave * D;
-            for (int job = wave; job < jobs; job += nw) {
+            for (int job = wave; job < jobs; job += block_waves) {
                 const bool is_q = job < nrows, is_k = job == nrows;
                 const float *src = is_q ? f.q_proj + (int64_t)(kvh * G + job % G) * D
                                         : (is_k ? f.k_proj : f.v_proj) + (int64_t)kvh * D;
@@ -674,7 +696,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
     // launch, so the whole stream is built once per form rather than
     // branching per block.
     auto stream = [&](auto nt_tag) {
-        int blk = wave;
+        int blk = LAYERS && wave >= nw ? nblk : wave;
         u32x4 kc[U][CPL], vc[U][CPL];
         if (blk < nblk) load_block_as(nt_tag, blk, kc, vc);
         produce();
@@ -809,7 +831,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
             const float v = O / L;
             bad_out |= !is_finite_f(v);
             gstore_ptr<float>(out)[((int64_t)t * Hq + h) * D + d] = v;
-        } else if (p.merge_launch) {
+        } else if (LAYERS || p.merge_launch) {
             // Combined by attn_decode_merge after this kernel: the kernel
             // boundary orders the stores, so they are plain.
             p.part_o[(slot * R + r) * D + d] = O;
@@ -837,7 +859,7 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
         raise_status(p, bad_out, ST_NONFINITE_OUTPUT);
         return;
     }
-    if (p.merge_launch) return;
+    if (LAYERS || p.merge_launch) return;
 
     // Split-K completion without atomics: every split but the last stores its
     // partial, waits until the stores are acknowledged, and then stores this
@@ -978,6 +1000,16 @@ __global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void 
     raise_status(p, bad_out, ST_NONFINITE_OUTPUT);
 }
 
+template <int DT, int D, int R, int U, bool CAP, bool FUSED>
+__global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void attn_decode(DecodeArgs kargs) {
+    decode_body<DT, D, R, U, CAP, FUSED, false>(kargs.p);
+}
+
+template <int DT, int D, int R, int U, bool CAP>
+__global__ __launch_bounds__(64 * decode_waves_for(D * Elem<DT>::size, R)) void attn_decode_layers(DecodeLayersArgs kargs) {
+    decode_body<DT, D, R, U, CAP, true, true>(kargs.p);
+}
+
 }  // namespace tkh
 
 namespace tkh {
@@ -985,11 +1017,26 @@ namespace tkh {
 // Launch of one attn_decode geometry: the softcap and fused-producer variants.
 // The producer is folded in for bf16/f16 rows (head_dim 64 to 256) and, with
 // the score softcap, for head_dim 256 (Gemma's sliding and global layers).
+// fused 2: `a` is the head of a DecodeLayersArgs.
 template <int DT, int DD, int RR, int UU>
 hipError_t decode_launch_variant(const DecodeArgs *a, int fused, dim3 grid, dim3 block,
                                  hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
     if (fused) {
         if constexpr (DT != F32 && DD * Elem<DT>::size <= 512) {
+            if (fused == 2) {
+                const DecodeLayersArgs *la = reinterpret_cast<const DecodeLayersArgs *>(a);
+                if (la->p.softcap != 0.0f) {
+                    if constexpr (DD == 256) {
+                        hipExtLaunchKernelGGL((attn_decode_layers<DT, DD, RR, UU, true>), grid, block, 0,
+                                              stream, start, stop, 0, *la);
+                        return hipGetLastError();
+                    }
+                    return hipErrorInvalidValue;
+                }
+                hipExtLaunchKernelGGL((attn_decode_layers<DT, DD, RR, UU, false>), grid, block, 0, stream,
+                                      start, stop, 0, *la);
+                return hipGetLastError();
+            }
             if (a->p.softcap != 0.0f) {
                 if constexpr (DD == 256) {
                     hipExtLaunchKernelGGL((attn_decode<DT, DD, RR, UU, true, true>), grid, block, 0,

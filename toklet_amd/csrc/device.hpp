@@ -207,6 +207,25 @@ struct DecodeArgs {
     DecodeBatch b;
 };
 
+// One session step of several layers in one launch: the layers' problems and
+// producer descriptors in the kernel's arguments (the launch fields that the
+// layers share are Params).  Layer i's workgroups start at first[i].
+constexpr int DECODE_LAYERS_MAX = 8;
+struct DecodeLayer {
+    Problem pr;
+    FusedDecode fused;
+    int64_t window;
+    int32_t has_window;
+    int32_t nw;            // waves that stream the layer's keys (the launch may have more)
+};
+struct DecodeLayersArgs {
+    Params p;
+    int32_t first[DECODE_LAYERS_MAX];
+    int32_t count;
+    DecodeLayer e[DECODE_LAYERS_MAX];
+};
+static_assert(sizeof(DecodeLayersArgs) <= 4096, "kernel arguments");
+
 // Chunks of one shape (tkh_prefill_batch: equal query counts, one K/V segment
 // from key 0 each, no window, no key splits; at most PREFILL_BATCH_MAX) carried
 // in the prefill kernel's own arguments, so the launch needs no descriptor

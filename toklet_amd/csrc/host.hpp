@@ -176,18 +176,28 @@ struct tkh_kv {
 };
 
 namespace tkh_host {
+// The fused decode steps of layers that are launched together
+// (flush_decode_layers), with the launch they have in common.
+struct DecodeBatchOfLayers {
+    tkh::DecodeLayersArgs args{};
+    int dtype = 0, R = 0, u = 0, nw = 0;
+    int64_t wgs = 0, slots = 0;
+    bool split = false;
+};
+uint32_t flush_decode_layers(tkh_context *ctx, DecodeBatchOfLayers *batch, tkh_error *err);
 // attention_cached of one token with the producer folded into the decode
-// kernel (api.cpp); used by the session for decode steps.
+// kernel (api.cpp); used by the session for decode steps.  With `batch` the
+// step is added to it, to be launched by flush_decode_layers at the latest.
 uint32_t attention_cached_fused(tkh_context *ctx, const tkh_cached_shape *shape, tkh_dtype dtype,
                                 const void *k, const void *v, float *context,
-                                const tkh::FusedDecode &fused, tkh_error *err);
+                                const tkh::FusedDecode &fused, DecodeBatchOfLayers *batch, tkh_error *err);
 // span_attention of one token (the last key of the view) with the producer
 // folded into the decode kernel: the session's decode steps of layers with a
 // score scale, softcap or window, and of ring caches (the new K/V row goes to
 // the layer's staging row, fused.new_row 0).
 uint32_t span_attention_fused(tkh_context *ctx, const tkh_span_shape *shape, tkh_dtype dtype,
                               const tkh_segment segments[3], float *context,
-                              const tkh::FusedDecode &fused, tkh_error *err);
+                              const tkh::FusedDecode &fused, DecodeBatchOfLayers *batch, tkh_error *err);
 // tkh_kv_commit_batch with an optional device gate (api.cpp).
 uint32_t commit_frames(tkh_kv *const *kvs, const tkh_kv_frame *frames, uint64_t count,
                        const uint32_t *gate, uint64_t *committed, uint64_t committed_value,
