@@ -60,6 +60,13 @@ extern "C" hipError_t tkh_launch_prefill16(const tkh::PrefillArgs *p, int dtype,
 extern "C" hipError_t tkh_launch_prefill(const tkh::PrefillArgs *p, int dtype, int head_dim, int waves,
                                          int64_t groups, hipStream_t stream, hipEvent_t start,
                                          hipEvent_t stop);
+extern "C" int tkh_prefill_layer_rows(int head_dim);
+extern "C" hipError_t tkh_launch_prefill_layers(const tkh::PrefillLayersArgs *a, int dtype, int head_dim, int64_t groups,
+                                                hipStream_t stream, hipEvent_t start, hipEvent_t stop);
+extern "C" hipError_t tkh_launch_prefill_merge_layers(const tkh::PrefillLayersArgs *a, int head_dim, int64_t blocks,
+                                                      hipStream_t stream, hipEvent_t start, hipEvent_t stop);
+extern "C" hipError_t tkh_launch_produce(const tkh::ProduceParams *p, int dtype, hipStream_t stream);
+extern "C" hipError_t tkh_launch_produce_layers(const tkh::ProduceLayersArgs *a, int dtype, hipStream_t stream);
 extern "C" int tkh_decode_keys_per_lane(int dtype, int head_dim, int rows, int want);
 extern "C" int tkh_decode_max_waves(int dtype, int head_dim, int rows);
 extern "C" int tkh_decode_max_splits(void);
@@ -534,9 +541,18 @@ bool compact_prefill(const Plan &plan, const Problems &group, tkh::PrefillBatch 
     return true;
 }
 
-// Many query rows per KV head (bf16/f16): the MFMA flash kernel, one launch.
-uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
-                        tkh_error *err) {
+// How a prefill launch covers its problems (plan_prefill).
+struct PrefillPlan {
+    int waves;         // 32-row waves per workgroup
+    bool rows16;       // the 16-row kernel, with waves16 waves
+    int waves16;
+    int64_t rows_per;  // packed rows per workgroup
+    int64_t wgs, slots, merge_blocks;
+};
+
+// Kernel, splits and workspace slots of a prefill launch of `group`, whose
+// planning fields are filled in place.
+uint32_t plan_prefill(tkh_context *ctx, const Plan &plan, Problems group, PrefillPlan *out, tkh_error *err) {
     const int64_t D = plan.head_dim, Hkv = plan.kv_heads, G = plan.query_heads / plan.kv_heads;
     // Eight-wave (256-row) workgroups where the head_dim has them and their row
     // blocks alone fill the device (the target is set in 128-row workgroups);
@@ -645,6 +661,19 @@ uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
         return fail(err, TKH_UNSUPPORTED, "workspace", 0, need, split_region_bytes(ctx),
                     "attention needs %zu workspace bytes, context has %zu for it", need,
                     split_region_bytes(ctx));
+    *out = PrefillPlan{waves, rows16, waves16, rows_per, wgs, slots, merge_blocks};
+    return TKH_OK;
+}
+
+// Many query rows per KV head (bf16/f16): the MFMA flash kernel, one launch.
+uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
+                        tkh_error *err) {
+    const int64_t D = plan.head_dim;
+    PrefillPlan pp;
+    TRY(plan_prefill(ctx, plan, group, &pp, err));
+    const bool rows16 = pp.rows16;
+    const int waves = pp.waves, waves16 = pp.waves16;
+    const int64_t rows_per = pp.rows_per, wgs = pp.wgs, slots = pp.slots, merge_blocks = pp.merge_blocks;
     tkh::PrefillArgs args{};
     tkh::Problem *dev = nullptr;
     if (group.size() > 1 && !(ctx->prefill_compact && compact_prefill(plan, group, &args.b)))
@@ -814,17 +843,64 @@ uint32_t launch_all(tkh_context *ctx, const Plan &plan, tkh::Problem *probs, siz
     return TKH_OK;
 }
 
-uint32_t run(tkh_context *ctx, Plan &plan, tkh_error *err) {
-    TRY(launch_all(ctx, plan, plan.store, plan.count, err));
-    return after_launch(ctx, err);
-}
-
-
 // Whether two ranges of device memory share a byte.
 bool overlap(const void *a, uint64_t na, const void *b, uint64_t nb) {
     const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
     return a && b && x < y + nb && y < x + na;
 }
+
+// A session chunk's attention call into the batch of its layers: its producer
+// is there already.  False (and nothing added): the call is for another kernel
+// than the layers' build, or does not fit behind the others.
+uint32_t join_chunk_layers(tkh_context *ctx, Plan &plan, ChunkBatchOfLayers *batch, bool *joined, tkh_error *err) {
+    *joined = false;
+    const int64_t D = plan.head_dim, Hkv = plan.kv_heads, G = plan.query_heads / Hkv;
+    tkh::Problem &p = plan.store[0];
+    if (ctx->force_generic || plan.diag_mode != 0 || plan.dtype == TKH_F32 || tkh_prefill_layer_rows((int)D) == 0 ||
+        p.queries * G <= tkh_decode_max_rows((int)plan.dtype, (int)D))
+        return TKH_OK;
+    PrefillPlan pp;
+    TRY(plan_prefill(ctx, plan, Problems{&p, 1}, &pp, err));
+    if (pp.waves != 4 || pp.rows_per != tkh_prefill_layer_rows((int)D) || pp.rows16 != (D != 64)) return TKH_OK;
+    tkh::PrefillLayersArgs &a = batch->args;
+    const size_t all = (size_t)(batch->slots + pp.slots) * pp.rows_per * (D + 2) * sizeof(float);
+    if (all > split_region_bytes(ctx) || batch->wgs + pp.wgs > INT32_MAX / 64) return TKH_OK;
+    if (a.count == 0) {
+        a.p = base_params(ctx, plan);
+        a.p.nproblems = 1;
+        batch->dtype = (int)plan.dtype;
+        batch->rows_per = pp.rows_per;
+    }
+    p.tile_base = batch->wgs;
+    p.slot_base = batch->slots;
+    p.part_base = batch->merge_blocks;
+    tkh::PrefillLayer &e = a.e[a.count];
+    e.pr = p;
+    e.has_window = plan.has_window ? 1 : 0;
+    e.window = plan.window;
+    a.first[a.count] = (int32_t)batch->wgs;
+    a.merge_first[a.count] = (int32_t)batch->merge_blocks;
+    ++a.count;
+    batch->wgs += pp.wgs;
+    batch->slots += pp.slots;
+    batch->merge_blocks += pp.merge_blocks;
+    *joined = true;
+    return TKH_OK;
+}
+
+uint32_t run(tkh_context *ctx, Plan &plan, tkh_error *err) {
+    if (ChunkBatchOfLayers *batch = ctx->collect) {
+        bool joined;
+        TRY(join_chunk_layers(ctx, plan, batch, &joined, err));
+        if (joined) return ok(err);
+        // Everything before this call first, its own producer included.
+        ctx->collect = nullptr;
+        TRY(flush_chunk_layers(ctx, batch, err));
+    }
+    TRY(launch_all(ctx, plan, plan.store, plan.count, err));
+    return after_launch(ctx, err);
+}
+
 
 // Whether layer `a` writes something that layer `b` reads or writes (contexts
 // against inputs and contexts), so that their order matters.
@@ -984,6 +1060,77 @@ uint32_t tkh_host::flush_decode_layers(tkh_context *ctx, DecodeBatchOfLayers *ba
     }
     a.count = 0;
     if (e != hipSuccess) return device_error(e, count > 1 ? "decode layers launch" : "decode launch", err);
+    return after_launch(ctx, err);
+}
+
+// A layer's producer into the batch of a chunk's layers, whose Q goes to a slot
+// of the Q scratch: at most as many layers as there are slots, and none that reads
+// or overwrites what another writes (contexts are written after every producer
+// of the batch has run).
+uint32_t tkh_host::add_chunk_producer(tkh_context *ctx, ChunkBatchOfLayers *batch, const tkh::ProduceParams &p,
+                                      tkh_dtype dtype, const float *context, int slots, void **q_scratch,
+                                      uint64_t slot_bytes, tkh_error *err) {
+    tkh::ProduceLayersArgs &a = batch->produce;
+    const uint64_t rows = (uint64_t)p.tokens * p.d * sizeof(float);
+    const uint64_t q = rows * p.hq, k = rows * batch->kv_heads, w = (uint64_t)p.d * sizeof(float);
+    auto feeds = [&](const float *out, const tkh::ProduceLayer &x) {
+        return overlap(out, q, x.q, q) || overlap(out, q, x.k, k) || overlap(out, q, x.v, k) || overlap(out, q, x.q_norm, w) ||
+               overlap(out, q, x.k_norm, w);
+    };
+    tkh::ProduceLayer e{p.q, p.k, p.v, p.q_norm, p.k_norm, nullptr, p.k_out, p.v_out, p.out_head_stride};
+    bool fits = a.count < std::min(slots, tkh::DECODE_LAYERS_MAX);
+    for (int i = 0; i < a.count && fits; ++i)
+        fits = !overlap(batch->context[i], q, context, q) && !feeds(batch->context[i], e) && !feeds(context, a.e[i]);
+    if (!fits) TRY(flush_chunk_layers(ctx, batch, err));
+    if (a.count == 0) {
+        a.p = p;
+        batch->produce_dtype = (int)dtype;
+    }
+    *q_scratch = static_cast<uint8_t *>(*q_scratch) + (uint64_t)a.count * slot_bytes;
+    e.q_out = *q_scratch;
+    batch->context[a.count] = context;
+    a.e[a.count++] = e;
+    return TKH_OK;
+}
+
+// The batched layers' producers, then the attention calls that joined, then the
+// merge of those that are split: three launches.
+uint32_t tkh_host::flush_chunk_layers(tkh_context *ctx, ChunkBatchOfLayers *batch, tkh_error *err) {
+    tkh::ProduceLayersArgs &pa = batch->produce;
+    tkh::PrefillLayersArgs &a = batch->args;
+    const int producers = pa.count, layers = a.count;
+    const int64_t wgs = batch->wgs, slots = batch->slots, merge_blocks = batch->merge_blocks;
+    batch->clear();
+    if (producers == 0) return TKH_OK;
+    HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
+    pa.count = producers;
+    pa.p.hkv = (int32_t)batch->kv_heads;
+    if (producers == 1) {
+        // One layer: its own launch, whose fields need no lookup.
+        const tkh::ProduceLayer &e = pa.e[0];
+        tkh::ProduceParams p = pa.p;
+        p.q_out = e.q_out;
+        if (!e.k_out) p.hkv = 0;
+        pa.count = 0;
+        HIP_TRY(tkh_launch_produce(&p, batch->produce_dtype, ctx->stream), "producer launch");
+    } else {
+        const hipError_t e = tkh_launch_produce_layers(&pa, batch->produce_dtype, ctx->stream);
+        pa.count = 0;
+        HIP_TRY(e, "producer launch");
+    }
+    if (layers == 0) return TKH_OK;
+    const int D = a.p.head_dim;
+    a.p.total_tiles = wgs;
+    a.p.part_ml = reinterpret_cast<float *>(ctx->workspace);
+    a.p.part_o = a.p.part_ml + (size_t)slots * batch->rows_per * 2;
+    hipEvent_t *ev = nullptr;
+    if (ctx->profiling) TRY(profile_slot(ctx, &ev, merge_blocks > 0, err));
+    a.count = layers;
+    hipError_t e = tkh_launch_prefill_layers(&a, batch->dtype, D, wgs, ctx->stream, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
+    if (e == hipSuccess && merge_blocks > 0)
+        e = tkh_launch_prefill_merge_layers(&a, D, merge_blocks, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);
+    a.count = 0;
+    if (e != hipSuccess) return device_error(e, "prefill layers launch", err);
     return after_launch(ctx, err);
 }
 

@@ -255,6 +255,36 @@ struct PrefillArgs {
     Params p;             // first: the single-problem path reads it at the kernel-argument base
     PrefillBatch b;
 };
+// One chunk of several layers in one launch (as DecodeLayersArgs for a step):
+// layer i's workgroups start at first[i].  Also the argument of the merge, whose
+// blocks start at merge_first[i].
+struct PrefillLayer {
+    Problem pr;
+    int64_t window;
+    int32_t has_window;
+    int32_t pad;
+};
+struct PrefillLayersArgs {
+    Params p;
+    int32_t first[DECODE_LAYERS_MAX];
+    int32_t merge_first[DECODE_LAYERS_MAX];
+    int32_t count;
+    PrefillLayer e[DECODE_LAYERS_MAX];
+};
+static_assert(sizeof(PrefillLayersArgs) <= 4096, "kernel arguments");
+
+// The producers of those layers: what differs between them.
+struct ProduceLayer {
+    const float *q, *k, *v, *q_norm, *k_norm;
+    void *q_out, *k_out, *v_out;  // k_out null: a layer without K/V of its own
+    int64_t out_head_stride;
+};
+struct ProduceLayersArgs {
+    ProduceParams p;
+    int32_t count;
+    ProduceLayer e[DECODE_LAYERS_MAX];
+};
+
 // The FP32 tile kernels' argument (attention.hip).
 struct TileArgs {
     Params p;             // first: the single-problem path reads it at the kernel-argument base

@@ -95,6 +95,24 @@ using namespace tkh_host;
 
 // ---------------------------------------------------------------- context
 
+namespace tkh_host {
+// The producers and attention calls of a session chunk's layers that are
+// launched together (flush_chunk_layers).
+struct ChunkBatchOfLayers {
+    tkh::ProduceLayersArgs produce{};
+    tkh::PrefillLayersArgs args{};
+    const float *context[tkh::DECODE_LAYERS_MAX] = {};  // what the layers of `produce` write in the end
+    uint64_t kv_heads = 0;
+    int dtype = 0, produce_dtype = 0;
+    int64_t rows_per = 0, wgs = 0, slots = 0, merge_blocks = 0;
+    void clear() {
+        produce.count = 0;
+        args.count = 0;
+        wgs = slots = merge_blocks = 0;
+    }
+};
+}  // namespace tkh_host
+
 struct tkh_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -140,6 +158,8 @@ struct tkh_context {
     int prefill16_groups = 64;   // split target of the 16-row kernel's launches (in 128-row workgroups)
     int prefill16_waves = 4;     // 16-row waves per workgroup: 4 (64-row blocks) or 8 (128-row blocks)
     int tile_groups = 512;       // FP32 tile kernel: below this many row-block workgroups, split the keys
+    // Set only while a session adds a chunk's layer: where its attention call goes.
+    tkh_host::ChunkBatchOfLayers *collect = nullptr;
     // profiling: per launch, start/stop of the attention kernel and of the combine kernel
     bool profiling = false;
     std::vector<hipEvent_t> prof_events;
@@ -185,6 +205,9 @@ struct DecodeBatchOfLayers {
     bool split = false;
 };
 uint32_t flush_decode_layers(tkh_context *ctx, DecodeBatchOfLayers *batch, tkh_error *err);
+uint32_t add_chunk_producer(tkh_context *ctx, ChunkBatchOfLayers *batch, const tkh::ProduceParams &p, tkh_dtype dtype,
+                            const float *context, int slots, void **q_scratch, uint64_t slot_bytes, tkh_error *err);
+uint32_t flush_chunk_layers(tkh_context *ctx, ChunkBatchOfLayers *batch, tkh_error *err);
 // attention_cached of one token with the producer folded into the decode
 // kernel (api.cpp); used by the session for decode steps.  With `batch` the
 // step is added to it, to be launched by flush_decode_layers at the latest.

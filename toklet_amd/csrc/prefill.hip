@@ -317,6 +317,8 @@ struct PfView {
     float *out;
     int64_t q_row_stride, q_pos0, k_pos0, keys, vis_lo, vis_hi, tile_base, slot_base;
     int32_t queries, row_blocks, splits, split_keys;
+    int64_t window;
+    int32_t has_window;
     Segment sg;
 };
 
@@ -333,7 +335,9 @@ __device__ __forceinline__ int find_prefill_entry(const_ptr<PrefillBatch> b, int
 // The workgroup's logical tile and what it covers: its problem (from the
 // descriptors, or built from a compact batch entry), row block, key split,
 // KV head and the split's index inside its segment.
-template <int D>
+// LAYERS: the arguments are a PrefillLayersArgs, the problem its layer's.
+template <bool LAYERS> using prefill_args = std::conditional_t<LAYERS, PrefillLayersArgs, PrefillArgs>;
+template <int D, bool LAYERS>
 __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, int &split, int &kvh, int &sidx) {
     // XCD-major tile order: dispatch slot b runs on XCD b % 8; give each XCD
     // a contiguous range of logical tiles.
@@ -349,8 +353,10 @@ __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, 
     {
         const_ptr<PrefillArgs> args = (const_ptr<PrefillArgs>)__builtin_amdgcn_kernarg_segment_ptr();
         const_ptr<PrefillBatch> batch = &args->b;
-        const int bcount = batch->count;
-        if (bcount > 0) {
+        const int bcount = LAYERS ? 0 : batch->count;
+        pv.has_window = p.has_window;
+        pv.window = p.window;
+        if (!LAYERS && bcount > 0) {
             // A compact batch: one segment from key 0, no key splits.
             const int i = find_prefill_entry(batch, bcount, tile);
             const auto &e = batch->e[i];
@@ -380,7 +386,19 @@ __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, 
             split = 0;
             sidx = 0;
         } else {
-            const_ptr<Problem> pr = problem_ptr(p, tile);
+            const_ptr<Problem> pr;
+            if constexpr (LAYERS) {
+                const_ptr<PrefillLayersArgs> la = (const_ptr<PrefillLayersArgs>)args;
+                int layer = 0;
+                for (int i = 1; i < DECODE_LAYERS_MAX; ++i)
+                    layer = i < la->count && (int)tile >= la->first[i] ? i : layer;
+                const_ptr<PrefillLayer> e = &la->e[uniform32(layer)];
+                pr = &e->pr;
+                pv.has_window = e->has_window;
+                pv.window = e->window;
+            } else {
+                pr = problem_ptr(p, tile);
+            }
             pv.q = pr->q;
             pv.out = pr->out;
             pv.q_row_stride = pr->q_row_stride;
@@ -457,15 +475,15 @@ __device__ __forceinline__ PfRows pf_rows(const Params &p, const PfView &pv, int
     r.t_row = (int)((uint32_t)rrow / ug);
     r.h_row = kvh * G + (int)((uint32_t)rrow % ug);
     int64_t r_lo, r_hi;
-    visible_range(p, pv.k_pos0, pv.keys, pv.q_pos0 + r.t_row, &r_lo, &r_hi);
+    visible_range(pv.has_window != 0, pv.window, pv.k_pos0, pv.keys, pv.q_pos0 + r.t_row, &r_lo, &r_hi);
     if (!r.rvalid) r_hi = r_lo;  // no visible keys: never contributes, never stored
 
     // Key range of the workgroup: the union over its rows, clipped to the split.
     const int wg_row_first = rb * ROWS;
     const int wg_row_last = min(wg_row_first + ROWS, m_kv) - 1;
     int64_t k_lo, k_hi, tmp;
-    visible_range(p, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)wg_row_first / ug, &k_lo, &tmp);
-    visible_range(p, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)wg_row_last / ug, &tmp, &k_hi);
+    visible_range(pv.has_window != 0, pv.window, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)wg_row_first / ug, &k_lo, &tmp);
+    visible_range(pv.has_window != 0, pv.window, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)wg_row_last / ug, &tmp, &k_hi);
     if (k_lo < s_lo) k_lo = s_lo;
     if (k_hi > s_hi) k_hi = s_hi;
     if (k_hi < k_lo) k_hi = k_lo;
@@ -480,8 +498,8 @@ __device__ __forceinline__ PfRows pf_rows(const Params &p, const PfView &pv, int
         const int w_first = min(wg_row_first + wave * RW, m_kv - 1);
         const int w_last = min(wg_row_first + wave * RW + RW - 1, m_kv - 1);
         int64_t a, b, full_lo, full_hi;
-        visible_range(p, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)w_first / ug, &a, &full_hi);
-        visible_range(p, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)w_last / ug, &full_lo, &b);
+        visible_range(pv.has_window != 0, pv.window, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)w_first / ug, &a, &full_hi);
+        visible_range(pv.has_window != 0, pv.window, pv.k_pos0, pv.keys, pv.q_pos0 + (uint32_t)w_last / ug, &full_lo, &b);
         int64_t lo_t = full_lo - k_lo;
         lo_t = lo_t <= 0 ? 0 : (lo_t + PF_KT - 1) / PF_KT;
         int64_t hi_t = full_hi - k_lo;
@@ -575,13 +593,14 @@ __device__ __forceinline__ void pf_scan_v(const uint8_t *vrows, int nkeys, int p
     }
 }
 
-template <int DT, int D, bool CAP, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill(PrefillArgs a) {
+template <int DT, int D, bool CAP, int W, bool LAYERS>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill(prefill_args<LAYERS> a) {
     // The problem's fields are read by dependent scalar loads (the batch
     // count, then the problem, then its segment); with their lines already in
     // the scalar cache the chain costs one memory round trip, not one per
     // line (chunk launches: about 0.7 us less before the first tile).
-    warm_kernarg<(offsetof(PrefillArgs, b) + offsetof(PrefillBatch, e) + 63) / 64, sizeof(PrefillArgs)>();
+    constexpr int ARGS = LAYERS ? offsetof(PrefillLayersArgs, e) : offsetof(PrefillArgs, b) + offsetof(PrefillBatch, e);
+    warm_kernarg<(ARGS + 63) / 64, sizeof(prefill_args<LAYERS>)>();
     const Params &p = a.p;
     constexpr int ROWS = 32 * W;  // packed rows per workgroup
     constexpr int KS = D / 16;        // QK k-steps (16 features each)
@@ -606,7 +625,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int Hq = p.query_heads;
     PfView pv;
     int rb, split, kvh, sidx;
-    pf_locate<D>(p, pv, rb, split, kvh, sidx);
+    pf_locate<D, LAYERS>(p, pv, rb, split, kvh, sidx);
     const PfRows rows = pf_rows<ROWS, 32>(p, pv, rb, kvh, sidx, wave, j);
     const int t_row = rows.t_row, h_row = rows.h_row;
     const bool rvalid = rows.rvalid;
@@ -1259,9 +1278,10 @@ __device__ __forceinline__ float row4_max(float x) {
 
 // W 16-row waves per workgroup: eight make the four-wave 32-row kernel's
 // 128-row block; four make 64-row blocks.
-template <int DT, int D, bool CAP, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill16(PrefillArgs a) {
-    warm_kernarg<(offsetof(PrefillArgs, b) + offsetof(PrefillBatch, e) + 63) / 64, sizeof(PrefillArgs)>();
+template <int DT, int D, bool CAP, int W, bool LAYERS>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill16(prefill_args<LAYERS> a) {
+    constexpr int ARGS = LAYERS ? offsetof(PrefillLayersArgs, e) : offsetof(PrefillArgs, b) + offsetof(PrefillBatch, e);
+    warm_kernarg<(ARGS + 63) / 64, sizeof(prefill_args<LAYERS>)>();
     const Params &p = a.p;
     constexpr int RW = 16;            // packed rows per wave
     constexpr int ROWS = RW * W;      // packed rows per workgroup
@@ -1293,7 +1313,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int Hq = p.query_heads;
     PfView pv;
     int rb, split, kvh, sidx;
-    pf_locate<D>(p, pv, rb, split, kvh, sidx);
+    pf_locate<D, LAYERS>(p, pv, rb, split, kvh, sidx);
     const PfRows rows = pf_rows<ROWS, RW>(p, pv, rb, kvh, sidx, wave, j);
     const int t_row = rows.t_row, h_row = rows.h_row;
     const bool rvalid = rows.rvalid;
@@ -1641,29 +1661,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
 // thread owns four features of one row and reads the S partials of its row at
 // once (one round trip): m and l of every split, then the weighted sum of the
 // unnormalised contexts.  Problem::part_base is the problem's first merge block.
+// `b` counts the problem's own merge blocks from its part_base.
 template <int D, int ROWS>
-__global__ __launch_bounds__(256) void attn_prefill_merge(Params p, int64_t blocks) {
-    // The fields below arrive through dependent scalar loads (the block
-    // count, the problem count, the problem): their lines are brought in
-    // together first (Params, `blocks` and the hidden arguments after them).
-    warm_kernarg<(sizeof(Params) + sizeof(int64_t) + 63) / 64, 0>();
+__device__ __forceinline__ void prefill_merge_block(const Params &p, const_ptr<Problem> pr, int64_t b) {
     constexpr int FB = D / 16;                  // 16-feature blocks per row
     constexpr int RC = ROWS / 64;               // 64-row chunks per row block
     constexpr int MAXS = 16;
-    const int64_t b = blockIdx.x;
-    if (b >= blocks) return;
-    const_ptr<Problem> pr;
-    if (p.nproblems == 1) {
-        pr = &((const_ptr<Params>)__builtin_amdgcn_kernarg_segment_ptr())->single;
-    } else {
-        const_ptr<Problem> probs = (const_ptr<Problem>)p.problems;
-        int lo = 0, hi = p.nproblems - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (probs[mid].part_base <= b) lo = mid; else hi = mid - 1;
-        }
-        pr = probs + lo;
-    }
     const int G = p.group, Hq = p.query_heads;
     const int m_kv = pr->queries * G;
     const int64_t local = b - pr->part_base;
@@ -1720,6 +1723,41 @@ __global__ __launch_bounds__(256) void attn_prefill_merge(Params p, int64_t bloc
     raise_status(p, bad_out, ST_NONFINITE_OUTPUT);
 }
 
+template <int D, int ROWS>
+__global__ __launch_bounds__(256) void attn_prefill_merge(Params p, int64_t blocks) {
+    // The fields below arrive through dependent scalar loads (the block
+    // count, the problem count, the problem): their lines are brought in
+    // together first (Params, `blocks` and the hidden arguments after them).
+    warm_kernarg<(sizeof(Params) + sizeof(int64_t) + 63) / 64, 0>();
+    const int64_t b = blockIdx.x;
+    if (b >= blocks) return;
+    const_ptr<Problem> pr;
+    if (p.nproblems == 1) {
+        pr = &((const_ptr<Params>)__builtin_amdgcn_kernarg_segment_ptr())->single;
+    } else {
+        const_ptr<Problem> probs = (const_ptr<Problem>)p.problems;
+        int lo = 0, hi = p.nproblems - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (probs[mid].part_base <= b) lo = mid; else hi = mid - 1;
+        }
+        pr = probs + lo;
+    }
+    prefill_merge_block<D, ROWS>(p, pr, b);
+}
+
+// The merge of a chunk of several layers: layer i's blocks start at
+// merge_first[i] (a layer without splits has none).
+template <int D, int ROWS>
+__global__ __launch_bounds__(256) void attn_prefill_merge_layers(PrefillLayersArgs a) {
+    warm_kernarg<(offsetof(PrefillLayersArgs, e) + 63) / 64, 0>();
+    const_ptr<PrefillLayersArgs> la = (const_ptr<PrefillLayersArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+    const int b = (int)blockIdx.x;
+    int layer = 0;
+    for (int i = 1; i < DECODE_LAYERS_MAX; ++i) layer = i < la->count && b >= la->merge_first[i] ? i : layer;
+    prefill_merge_block<D, ROWS>(a.p, &la->e[layer].pr, b);
+}
+
 }  // namespace tkh
 
 extern "C" int tkh_prefill_waves(int head_dim, int wide) {
@@ -1754,9 +1792,9 @@ extern "C" hipError_t tkh_launch_prefill(const tkh::PrefillArgs *p, int dtype, i
 #define TKH_PF(DT, DD, WW)                                                              \
     if (dtype == DT && head_dim == DD && waves == WW) {                                 \
         if (p->p.softcap != 0.0f)                                                       \
-            hipExtLaunchKernelGGL((attn_prefill<DT, DD, true, WW>), grid, block, 0, stream, start, stop, 0, *p);  \
+            hipExtLaunchKernelGGL((attn_prefill<DT, DD, true, WW, false>), grid, block, 0, stream, start, stop, 0, *p);  \
         else                                                                            \
-            hipExtLaunchKernelGGL((attn_prefill<DT, DD, false, WW>), grid, block, 0, stream, start, stop, 0, *p); \
+            hipExtLaunchKernelGGL((attn_prefill<DT, DD, false, WW, false>), grid, block, 0, stream, start, stop, 0, *p); \
         return hipGetLastError();                                                       \
     }
     TKH_PF(BF16, 64, 4) TKH_PF(BF16, 128, 4) TKH_PF(BF16, 128, 8) TKH_PF(BF16, 256, 4)
@@ -1775,13 +1813,45 @@ extern "C" hipError_t tkh_launch_prefill16(const tkh::PrefillArgs *p, int dtype,
 #define TKH_PF16(DT, DD, WW)                                                            \
     if (dtype == DT && head_dim == DD && waves == WW) {                                 \
         if (p->p.softcap != 0.0f)                                                       \
-            hipExtLaunchKernelGGL((attn_prefill16<DT, DD, true, WW>), grid, block, 0, stream, start, stop, 0, *p);  \
+            hipExtLaunchKernelGGL((attn_prefill16<DT, DD, true, WW, false>), grid, block, 0, stream, start, stop, 0, *p);  \
         else                                                                            \
-            hipExtLaunchKernelGGL((attn_prefill16<DT, DD, false, WW>), grid, block, 0, stream, start, stop, 0, *p); \
+            hipExtLaunchKernelGGL((attn_prefill16<DT, DD, false, WW, false>), grid, block, 0, stream, start, stop, 0, *p); \
         return hipGetLastError();                                                       \
     }
     TKH_PF16(BF16, 128, 8) TKH_PF16(BF16, 256, 8) TKH_PF16(F16, 128, 8) TKH_PF16(F16, 256, 8)
     TKH_PF16(BF16, 128, 4) TKH_PF16(BF16, 256, 4) TKH_PF16(F16, 128, 4) TKH_PF16(F16, 256, 4)
 #undef TKH_PF16
     return hipErrorInvalidValue;
+}
+
+// A chunk of several layers: the builds a session's chunk takes by default
+// (head_dim 64: 32-row waves, 128 and 256: the 16-row kernel in 64-row blocks).
+extern "C" int tkh_prefill_layer_rows(int head_dim) { return head_dim == 64 ? 128 : (head_dim == 128 || head_dim == 256 ? 64 : 0); }
+extern "C" hipError_t tkh_launch_prefill_layers(const tkh::PrefillLayersArgs *a, int dtype, int head_dim, int64_t groups,
+                                                hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+    using namespace tkh;
+    dim3 grid((unsigned)groups), block(256);
+#define TKH_PFL(KERNEL, DT, DD)                                                                       \
+    if (dtype == DT && head_dim == DD) {                                                              \
+        if (a->p.softcap != 0.0f)                                                                     \
+            hipExtLaunchKernelGGL((KERNEL<DT, DD, true, 4, true>), grid, block, 0, stream, start, stop, 0, *a);  \
+        else                                                                                          \
+            hipExtLaunchKernelGGL((KERNEL<DT, DD, false, 4, true>), grid, block, 0, stream, start, stop, 0, *a); \
+        return hipGetLastError();                                                                     \
+    }
+    TKH_PFL(attn_prefill, BF16, 64) TKH_PFL(attn_prefill, F16, 64)
+    TKH_PFL(attn_prefill16, BF16, 128) TKH_PFL(attn_prefill16, F16, 128)
+    TKH_PFL(attn_prefill16, BF16, 256) TKH_PFL(attn_prefill16, F16, 256)
+#undef TKH_PFL
+    return hipErrorInvalidValue;
+}
+extern "C" hipError_t tkh_launch_prefill_merge_layers(const tkh::PrefillLayersArgs *a, int head_dim, int64_t blocks,
+                                                      hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+    using namespace tkh;
+    dim3 grid((unsigned)blocks), block(256);
+    if (head_dim == 64) hipExtLaunchKernelGGL((attn_prefill_merge_layers<64, 128>), grid, block, 0, stream, start, stop, 0, *a);
+    else if (head_dim == 128) hipExtLaunchKernelGGL((attn_prefill_merge_layers<128, 64>), grid, block, 0, stream, start, stop, 0, *a);
+    else if (head_dim == 256) hipExtLaunchKernelGGL((attn_prefill_merge_layers<256, 64>), grid, block, 0, stream, start, stop, 0, *a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
 }

@@ -23,9 +23,11 @@
 // the denominator can differ in its last FP64 bit, which reaches an FP32
 // result only at a rounding tie.
 //
-// One wave per (token, head slot): slots [0, Hq) are query heads, [Hq,
-// Hq + Hkv) key heads, the rest value heads.  Non-finite inputs or results set
-// the device status word (the reference returns Error::NonFinite).
+// Non-finite inputs or results set the device status word (the reference
+// returns Error::NonFinite).
+#include <cstddef>
+#include <type_traits>
+
 #include "device.hpp"
 
 namespace tkh {
@@ -57,12 +59,10 @@ __device__ __forceinline__ double inverse_frequency(const RotarySpec &r, int D, 
 // Rotation of pair j at absolute position pos: angle and sine/cosine in FP64,
 // rounded once to FP32 (src/cpu/attention.rs:41-46,
 // src/cpu/proportional_rotary.rs:68-74, src/cpu/llama3_rotary.rs:126-128).
-__device__ __forceinline__ void rotary_cos_sin(const RotarySpec &r, int D, int64_t pos, int j,
-                                               float *c, float *s) {
+__device__ __forceinline__ float rotary_part(const RotarySpec &r, int D, int64_t pos, int j, bool sine) {
 #pragma clang fp contract(off)
     const double angle = (double)pos * inverse_frequency(r, D, j);
-    *s = (float)sin(angle);
-    *c = (float)cos(angle);
+    return sine ? (float)sin(angle) : (float)cos(angle);
 }
 
 template <int DT> __device__ __forceinline__ void store_out(void *base, int64_t i, float x);
@@ -79,104 +79,161 @@ template <> __device__ __forceinline__ void store_out<BF16>(void *base, int64_t 
 
 }  // namespace
 
-// TABLE: (cos, sin) come from p.rope.  Without it the kernel carries the FP64
-// pow/sin/cos of rotary_cos_sin, which takes its register count to 129: three
-// waves per SIMD instead of four, so a session chunk's 4096 waves
-// needed a second round (launch span 6.7 us, the last waves starting 3.9 us
-// late).  Sessions always pass the table.
-template <int DT, bool TABLE>
-__global__ __launch_bounds__(64) void produce_qkv(ProduceParams p) {
+// One workgroup covers `rows` head slots of one token: slots [0, Hq) are query
+// heads, [Hq, Hq + Hkv) key heads, the rest value heads; a wave takes slots wave,
+// wave + waves, ..., RG of them at a time, so their loads and their FP64 chains
+// overlap.  Lane l holds elements l, l + 64, ... of a row (K of them, D <= 64 K).
+//
+// The token's (cos, sin) are the same for every head.  TABLE: each wave reads
+// them from p->rope once.  Without it a wave per 64 pairs and function evaluates
+// the FP64 pow and sine or cosine and the others read the result from LDS, so the host gives a workgroup every slot of its token:
+// evaluating them in each of 32 slots' waves made 128 tokens of 16/8/128 take
+// 9.3 us, this 7.6 (4,096 tokens 169 and 49 us).
+template <int DT, int K, bool TABLE>
+__device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const ProduceLayer io, int hkv, int64_t t,
+                                             int first, int rows) {
 #pragma clang fp contract(off)
-    // Its fields arrive through dependent scalar loads: their lines (and the
-    // hidden arguments' start) first, in one round trip.
-    warm_kernarg<(sizeof(ProduceParams) + 63) / 64, 0>();
-    __shared__ float row[512];
-    const int lane = threadIdx.x;
-    const int D = p.d;
-    const int slots = p.hq + 2 * p.hkv;
-    const int64_t t = blockIdx.x / slots;
-    const int slot = (int)(blockIdx.x % slots);
-    if (t >= p.tokens) return;
-    const int kind = slot < p.hq ? 0 : (slot < p.hq + p.hkv ? 1 : 2);  // q, k, v
-    const int h = kind == 0 ? slot : (kind == 1 ? slot - p.hq : slot - p.hq - p.hkv);
-    const int heads = kind == 0 ? p.hq : p.hkv;
-    const float *src = (kind == 0 ? p.q : (kind == 1 ? p.k : p.v)) + (t * heads + h) * D;
-    void *dst = kind == 0 ? p.q_out : (kind == 1 ? p.k_out : p.v_out);
-    const int64_t dst0 = kind == 0 ? (t * p.hq + h) * D : h * p.out_head_stride + t * D;
+    constexpr int RG = K <= 1 ? 2 : (K == 2 ? 4 : (K == 4 ? 2 : 1));
+    constexpr int KP = (K + 1) / 2;               // rotary pairs per lane
+    constexpr int WAVES = TABLE ? 4 : 8;
+    __shared__ float rowbuf[WAVES][64 * K];
+    __shared__ f32x2 rot[TABLE ? 1 : 64 * KP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int D = p->d, hq = p->hq, half = D / 2;
+    const RotarySpec spec{p->rot.kind, p->rot.rotated_dims, p->rot.theta, p->rot.factor, p->rot.low, p->rot.high, p->rot.original};
+    const int pairs = rotary_pairs(spec.kind, D, spec.rotated_dims);
+    const int64_t position = p->position + t;
+    const int end = first + rows < hq + 2 * hkv ? first + rows : hq + 2 * hkv;
 
-    // Every load first (the row, the norm weights, the rotary pairs), then the
-    // arithmetic: one memory round trip per launch instead of three.
-    constexpr int KMAX = 8;  // elements per lane, D <= 512
-    const float *w = kind == 0 ? p.q_norm : (kind == 1 ? p.k_norm : nullptr);
-    const int half = D / 2;
-    const int pairs = kind == 2 ? 0 : rotary_pairs(p.rot.kind, D, p.rot.rotated_dims);
-    float xv[KMAX], wv[KMAX], cv[KMAX / 2], sv[KMAX / 2];
-    for (int k = 0; k < KMAX; ++k) {
-        const int i = lane + 64 * k;
-        xv[k] = i < D ? src[i] : 0.0f;
-        wv[k] = w && i < D ? w[i] : 0.0f;
-    }
-    for (int k = 0; k < KMAX / 2; ++k) {
-        const int j = lane + 64 * k;
-        cv[k] = 1.0f;
-        sv[k] = 0.0f;
-        if (j < half && j < pairs) {
-            if constexpr (TABLE) {
-                const float *cs = p.rope + 2 * ((p.position + t - p.rope_pos0) * pairs + j);
-                cv[k] = cs[0];
-                sv[k] = cs[1];
-            } else {
-                rotary_cos_sin(p.rot, D, p.position + t, j, &cv[k], &sv[k]);
+    float x[RG][K], wq[K], wk[K];
+    f32x2 cs[KP];
+    auto source = [&](int slot) {
+        return slot < hq ? io.q + (t * hq + slot) * D
+                         : (slot < hq + hkv ? io.k + (t * hkv + slot - hq) * D : io.v + (t * hkv + slot - hq - hkv) * D);
+    };
+    auto load = [&](int slot0) {
+#pragma unroll
+        for (int i = 0; i < RG; ++i) {
+            const int slot = slot0 + i * waves;
+            if (slot < end) {
+                const float *src = source(slot);
+                for (int k = 0; k < K; ++k) x[i][k] = lane + 64 * k < D ? src[lane + 64 * k] : 0.0f;
             }
+        }
+    };
+    // Every load first (rows, norm weights, rotary pairs), then the arithmetic.
+    load(first + wave);
+    for (int k = 0; k < K; ++k) {
+        const int i = lane + 64 * k;
+        wq[k] = io.q_norm && i < D ? io.q_norm[i] : 0.0f;
+        wk[k] = io.k_norm && i < D ? io.k_norm[i] : 0.0f;
+    }
+    for (int k = 0; k < KP; ++k) {
+        const int j = lane + 64 * k;
+        cs[k] = f32x2{1.0f, 0.0f};
+        if constexpr (TABLE) {
+            if (j < pairs) cs[k] = *gload_ptr<f32x2>(p->rope + 2 * ((position - p->rope_pos0) * pairs + j));
+        }
+    }
+    if constexpr (!TABLE) {
+        if (pairs > 0) {
+            // The lower half of the workgroup takes the cosines, the upper the
+            // sines: each wave's chain holds one of them.
+            const int j = threadIdx.x & 255;
+            const bool sine = wave >= WAVES / 2;
+            if (j < pairs) rot[j][sine ? 1 : 0] = rotary_part(spec, D, position, j, sine);
+            __syncthreads();
+            for (int k = 0; k < KP; ++k)
+                if (lane + 64 * k < pairs) cs[k] = rot[lane + 64 * k];
         }
     }
 
     bool bad = false;
-    for (int k = 0; k < KMAX; ++k)
-        if (lane + 64 * k < D) bad |= !is_finite_f(xv[k]);
-    if (kind == 2) {
-        for (int k = 0; k < KMAX; ++k)
-            if (lane + 64 * k < D) store_out<DT>(dst, dst0 + lane + 64 * k, xv[k]);
-        raise_status(p.status, bad, ST_NONFINITE_INPUT);
-        return;
-    }
-    if (w) {
-        double ss = 0.0;
-        for (int k = 0; k < KMAX; ++k)
-            if (lane + 64 * k < D) {
-                const double x = (double)xv[k];
-                ss += x * x;
+    float *row = rowbuf[wave];
+    for (int slot0 = first + wave; slot0 < end; slot0 += RG * waves) {
+        if (slot0 != first + wave) load(slot0);
+        // The norm of every row of the group before any is stored.
+#pragma unroll
+        for (int i = 0; i < RG; ++i) {
+            const int slot = slot0 + i * waves;
+            if (slot >= end) continue;
+            for (int k = 0; k < K; ++k) bad |= lane + 64 * k < D && !is_finite_f(x[i][k]);
+            const bool is_q = slot < hq;
+            if (slot >= hq + hkv || !(is_q ? io.q_norm : io.k_norm)) continue;
+            double ss = 0.0;
+            for (int k = 0; k < K; ++k)
+                if (lane + 64 * k < D) {
+                    const double v = (double)x[i][k];
+                    ss += v * v;
+                }
+            ss = wave_sum_f64(ss);
+            const double inv = 1.0 / sqrt(ss / (double)D + (double)p->eps);
+            for (int k = 0; k < K; ++k) {
+                const float w = is_q ? wq[k] : wk[k];
+                const float y = (float)((double)x[i][k] * inv * (double)w);
+                bad |= lane + 64 * k < D && (!is_finite_f(y) || !is_finite_f(w));
+                x[i][k] = y;
             }
-        ss = wave_sum_f64(ss);
-        const double inv = 1.0 / sqrt(ss / (double)D + (double)p.eps);
-        for (int k = 0; k < KMAX; ++k)
-            if (lane + 64 * k < D) {
-                const float y = (float)((double)xv[k] * inv * (double)wv[k]);
-                bad |= !is_finite_f(y) || !is_finite_f(wv[k]);
-                xv[k] = y;
-            }
-    }
-    // The rotary pairs elements j and j + D/2, which may sit in other lanes:
-    // through LDS (one wave, whose LDS accesses complete in order).
-    for (int k = 0; k < KMAX; ++k)
-        if (lane + 64 * k < D) row[lane + 64 * k] = xv[k];
-    __syncthreads();
-    for (int k = 0; k < KMAX / 2; ++k) {
-        const int j = lane + 64 * k;
-        if (j >= half) break;
-        const float a = row[j], b = row[j + half];
-        float x = a, y = b;
-        if (j < pairs) {
-            const float c = cv[k], sn = sv[k];
-            const float ac = a * c, bs = b * sn, bc = b * c, as = a * sn;
-            x = ac - bs;
-            y = bc + as;
-            bad |= !is_finite_f(x) || !is_finite_f(y);
         }
-        store_out<DT>(dst, dst0 + j, x);
-        store_out<DT>(dst, dst0 + j + half, y);
+#pragma unroll
+        for (int i = 0; i < RG; ++i) {
+            const int slot = slot0 + i * waves;
+            if (slot >= end) continue;
+            if (slot >= hq + hkv) {
+                const int64_t dst = (int64_t)(slot - hq - hkv) * io.out_head_stride + t * D;
+                for (int k = 0; k < K; ++k)
+                    if (lane + 64 * k < D) store_out<DT>(io.v_out, dst + lane + 64 * k, x[i][k]);
+                continue;
+            }
+            const bool is_q = slot < hq;
+            void *out = is_q ? io.q_out : io.k_out;
+            const int64_t dst = is_q ? (t * hq + slot) * D : (int64_t)(slot - hq) * io.out_head_stride + t * D;
+            // The rotary pairs elements j and j + D/2, which may sit in other
+            // lanes: through LDS (the wave's own row, whose accesses complete
+            // in order).
+            for (int k = 0; k < K; ++k)
+                if (lane + 64 * k < D) row[lane + 64 * k] = x[i][k];
+            for (int k = 0; k < KP; ++k) {
+                const int j = lane + 64 * k;
+                if (j >= half) continue;
+                float a = row[j], b = row[j + half];
+                if (j < pairs) {
+                    const float c = cs[k][0], sn = cs[k][1];
+                    const float ac = a * c, bs = b * sn, bc = b * c, as = a * sn;
+                    a = ac - bs;
+                    b = bc + as;
+                    bad |= !is_finite_f(a) || !is_finite_f(b);
+                }
+                store_out<DT>(out, dst + j, a);
+                store_out<DT>(out, dst + j + half, b);
+            }
+        }
     }
-    raise_status(p.status, bad, ST_NONFINITE_INPUT);
+    raise_status(p->status, bad, ST_NONFINITE_INPUT);
+}
+
+// blocks_per_token workgroups of `rows` slots per token.
+template <int DT, int K, bool TABLE>
+__global__ __launch_bounds__(TABLE ? 256 : 512) void produce_qkv(ProduceParams args, int rows, int blocks_per_token) {
+    // Its fields arrive through dependent scalar loads: their lines (and the
+    // hidden arguments' start) first, in one round trip.
+    const_ptr<ProduceParams> p = warm_kernarg_ptr<ProduceParams, (sizeof(ProduceParams) + 8 + 63) / 64, 0>();
+    const uint32_t bpt = (uint32_t)blocks_per_token;
+    const ProduceLayer io{p->q, p->k, p->v, p->q_norm, p->k_norm, p->q_out, p->k_out, p->v_out, p->out_head_stride};
+    produce_rows<DT, K, TABLE>(p, io, p->hkv, blockIdx.x / bpt, (int)(blockIdx.x % bpt) * rows, rows);
+}
+
+// The chunk of several session layers, one after the other in the grid (the
+// rotary table is the session's).  A layer without K/V of its own has k_out
+// null: only its Q rows are made.
+template <int DT, int K>
+__global__ __launch_bounds__(256) void produce_qkv_layers(ProduceLayersArgs args, int rows, int blocks_per_token) {
+    const_ptr<ProduceLayersArgs> a = warm_kernarg_ptr<ProduceLayersArgs, 11, offsetof(ProduceLayersArgs, e) + DECODE_LAYERS_MAX * sizeof(ProduceLayer) - 4>();
+    const uint32_t bpt = (uint32_t)blocks_per_token, per = bpt * (uint32_t)a->p.tokens;
+    const uint32_t layer = blockIdx.x / per, b = blockIdx.x % per;
+    const_ptr<ProduceLayer> e = &a->e[layer];
+    const ProduceLayer io{e->q, e->k, e->v, e->q_norm, e->k_norm, e->q_out, e->k_out, e->v_out, e->out_head_stride};
+    produce_rows<DT, K, true>(&a->p, io, io.k_out ? a->p.hkv : 0, b / bpt, (int)(b % bpt) * rows, rows);
 }
 
 // (cos, sin) of every (position, pair) for rows [pos0, pos0 + rows): the
@@ -188,10 +245,8 @@ __global__ __launch_bounds__(256) void rotary_table(float *out, int64_t pos0, in
     if (i >= rows * pairs) return;
     const int64_t r = i / pairs;
     const int j = (int)(i % pairs);
-    float c, s;
-    rotary_cos_sin(rot, D, pos0 + r, j, &c, &s);
-    out[2 * i] = c;
-    out[2 * i + 1] = s;
+    out[2 * i] = rotary_part(rot, D, pos0 + r, j, false);
+    out[2 * i + 1] = rotary_part(rot, D, pos0 + r, j, true);
 }
 
 }  // namespace tkh
@@ -213,23 +268,60 @@ extern "C" hipError_t tkh_launch_rotary_table(float *out, int64_t pos0, int64_t 
     return hipGetLastError();
 }
 
-extern "C" hipError_t tkh_launch_produce(const tkh::ProduceParams *p, int dtype, hipStream_t stream) {
+// Slots per workgroup.  With a rotary table: two for each of its four waves.
+// Without one each workgroup evaluates its token's rotation, so it takes up to 32
+// slots (four for each of eight waves), unless the card is mostly idle anyway
+// (one round of one slot per wave on 256 CUs: 1 token of 32/8/128 6.3 us
+// against 8.1 with all 48), and all of them from 1,024 tokens on, where the FP64
+// work decides (48 slots: 128 tokens 6.5 us in two workgroups, 8.6 in one; 4,096
+// tokens 80 and 66).
+static int produce_slots(int64_t tokens, int slots, bool table) {
+    if (table || tokens * ((slots + 7) / 8) <= 256) return 8;
+    const int blocks = tokens >= 1024 ? 1 : (slots + 31) / 32;
+    return ((slots + blocks - 1) / blocks + 7) / 8 * 8;
+}
+
+template <int DT, int K>
+static hipError_t launch_produce(const tkh::ProduceParams *p, hipStream_t stream) {
     using namespace tkh;
-    const int64_t blocks = p->tokens * (p->hq + 2 * p->hkv);
-    if (blocks <= 0 || p->d > 512 || p->d % 2) return hipErrorInvalidValue;
-    dim3 grid((unsigned)blocks), block(64);
-    const bool table = p->rope != nullptr;
-    if (dtype == F32) {
-        if (table) hipLaunchKernelGGL((produce_qkv<F32, true>), grid, block, 0, stream, *p);
-        else hipLaunchKernelGGL((produce_qkv<F32, false>), grid, block, 0, stream, *p);
-    } else if (dtype == F16) {
-        if (table) hipLaunchKernelGGL((produce_qkv<F16, true>), grid, block, 0, stream, *p);
-        else hipLaunchKernelGGL((produce_qkv<F16, false>), grid, block, 0, stream, *p);
-    } else if (dtype == BF16) {
-        if (table) hipLaunchKernelGGL((produce_qkv<BF16, true>), grid, block, 0, stream, *p);
-        else hipLaunchKernelGGL((produce_qkv<BF16, false>), grid, block, 0, stream, *p);
-    } else {
-        return hipErrorInvalidValue;
-    }
+    const bool table = p->rope != nullptr || rotary_pairs(p->rot.kind, p->d, p->rot.rotated_dims) == 0;
+    const int slots = p->hq + 2 * p->hkv, rows = produce_slots(p->tokens, slots, table), bpt = (slots + rows - 1) / rows;
+    const dim3 grid((unsigned)(p->tokens * bpt));
+    if (table) hipLaunchKernelGGL((produce_qkv<DT, K, true>), grid, dim3(256), 0, stream, *p, rows, bpt);
+    else hipLaunchKernelGGL((produce_qkv<DT, K, false>), grid, dim3(512), 0, stream, *p, rows, bpt);
     return hipGetLastError();
+}
+
+// f(type tag, elements-per-lane tag) for a dtype and head size.
+template <class F> static hipError_t produce_build(int dtype, int d, F f) {
+    using namespace tkh;
+    auto of = [&](auto dt) {
+        if (d <= 64) return f(dt, std::integral_constant<int, 1>{});
+        if (d <= 128) return f(dt, std::integral_constant<int, 2>{});
+        if (d <= 256) return f(dt, std::integral_constant<int, 4>{});
+        return f(dt, std::integral_constant<int, 8>{});
+    };
+    if (dtype == F32) return of(std::integral_constant<int, F32>{});
+    if (dtype == F16) return of(std::integral_constant<int, F16>{});
+    if (dtype == BF16) return of(std::integral_constant<int, BF16>{});
+    return hipErrorInvalidValue;
+}
+
+extern "C" hipError_t tkh_launch_produce(const tkh::ProduceParams *p, int dtype, hipStream_t stream) {
+    if (p->tokens <= 0 || p->hq + 2 * p->hkv <= 0 || p->d > 512 || p->d % 2) return hipErrorInvalidValue;
+    return produce_build(dtype, p->d, [&](auto dt, auto k) {
+        return launch_produce<decltype(dt)::value, decltype(k)::value>(p, stream);
+    });
+}
+
+// The layers' chunk; the rows have a rotary table, or no rotary.
+extern "C" hipError_t tkh_launch_produce_layers(const tkh::ProduceLayersArgs *a, int dtype, hipStream_t stream) {
+    using namespace tkh;
+    const int slots = a->p.hq + 2 * a->p.hkv, rows = produce_slots(a->p.tokens, slots, true), bpt = (slots + rows - 1) / rows;
+    const dim3 grid((unsigned)(a->count * a->p.tokens * bpt)), block(256);
+    if (a->p.tokens <= 0 || a->count <= 0 || a->p.d > 512 || a->p.d % 2) return hipErrorInvalidValue;
+    return produce_build(dtype, a->p.d, [&](auto dt, auto k) {
+        hipLaunchKernelGGL((produce_qkv_layers<decltype(dt)::value, decltype(k)::value>), grid, block, 0, stream, *a, rows, bpt);
+        return hipGetLastError();
+    });
 }

@@ -94,11 +94,9 @@ tkh::RotarySpec rotary_spec(const tkh_producer_shape *sh) {
     return r;
 }
 
-uint32_t launch_producer(tkh_context *ctx, const tkh_producer_shape *sh, tkh_dtype dtype,
-                         const float *q, const float *k, const float *v, const float *qn,
-                         const float *kn, void *q_out, void *k_out, void *v_out,
-                         uint64_t head_stride, tkh_error *err, const float *rope = nullptr,
-                         uint64_t rope_pos0 = 0) {
+tkh::ProduceParams producer_params(tkh_context *ctx, const tkh_producer_shape *sh, const float *q, const float *k,
+                                   const float *v, const float *qn, const float *kn, void *q_out, void *k_out,
+                                   void *v_out, uint64_t head_stride, const float *rope, uint64_t rope_pos0) {
     tkh::ProduceParams p{};
     p.rope = rope;
     p.rope_pos0 = (int64_t)rope_pos0;
@@ -119,6 +117,16 @@ uint32_t launch_producer(tkh_context *ctx, const tkh_producer_shape *sh, tkh_dty
     p.rot = rotary_spec(sh);
     p.eps = sh->norm_epsilon;
     p.status = ctx->status_dev;
+    return p;
+}
+
+uint32_t launch_producer(tkh_context *ctx, const tkh_producer_shape *sh, tkh_dtype dtype,
+                         const float *q, const float *k, const float *v, const float *qn,
+                         const float *kn, void *q_out, void *k_out, void *v_out,
+                         uint64_t head_stride, tkh_error *err, const float *rope = nullptr,
+                         uint64_t rope_pos0 = 0) {
+    const tkh::ProduceParams p =
+        producer_params(ctx, sh, q, k, v, qn, kn, q_out, k_out, v_out, head_stride, rope, rope_pos0);
     HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     HIP_TRY(tkh_launch_produce(&p, (int)dtype, ctx->stream), "producer launch");
     return TKH_OK;
@@ -168,7 +176,8 @@ struct tkh_session {
     // Queued ring sessions: the end of the last chunk whose ring commit ran
     // with a clean status word (written by the gated commit on the device).
     uint64_t *committed_dev = nullptr;
-    void *q_scratch = nullptr;                 // [chunk, Hq, D] cache dtype
+    void *q_scratch = nullptr;                 // q_slots x [chunk, Hq, D] cache dtype
+    int q_slots = 1;                           // layers whose Q a chunk can hold at once
     float *rope = nullptr;                     // (cos, sin) per (position, pair), or null
     bool fused_decode = false;                 // decode steps fold the producer into attention
     std::vector<void *> stage_k, stage_v;      // sliding layers: [Hkv, chunk, D]
@@ -198,7 +207,9 @@ struct tkh_session {
         }
     } chunk;
     std::vector<tkh_kv *> ring_owners;  // the ring caches, for reset_batch
-    tkh_host::DecodeBatchOfLayers steps;       // a decode step's layers, when they are given together
+    // The layers of a step or a chunk, when they are given together.
+    tkh_host::DecodeBatchOfLayers steps;
+    tkh_host::ChunkBatchOfLayers layers;
 };
 
 namespace {
@@ -457,8 +468,10 @@ extern "C" uint32_t tkh_session_create(tkh_context *ctx, const tkh_session_optio
         s->chunk.ring_kv.reserve(s->producers);
         s->chunk.frames.reserve(s->producers);
         s->chunk.owner_frame.reserve(s->producers);
-        s->scratch_bytes = chunk * o->query_heads * D * es;
-        hipError_t e = hipMalloc(&s->q_scratch, chunk * o->query_heads * D * es);
+        // A slot per layer that is launched together (f32 chunks are not).
+        s->q_slots = o->storage == TKH_F32 ? 1 : (int)std::min<uint64_t>(o->layers, tkh::DECODE_LAYERS_MAX);
+        s->scratch_bytes = (uint64_t)s->q_slots * chunk * o->query_heads * D * es;
+        hipError_t e = hipMalloc(&s->q_scratch, s->scratch_bytes);
         if (e == hipSuccess) e = hipMalloc(&s->committed_dev, sizeof(uint64_t));
         if (e == hipSuccess) e = tkh_launch_fill_u64(s->committed_dev, 0, ctx->stream);
         // The rotary (cos, sin) of every session position, once.
@@ -615,10 +628,10 @@ void begin_chunk(tkh_session *s, uint64_t start, uint64_t count, bool position_i
 
 void abort_chunk(tkh_session *s) { s->chunk.clear(); }
 
-// `batch`: where a decode step of this layer may wait for other layers' (null:
-// launched at once).
-uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBatchOfLayers *batch,
-                    tkh_error *err) {
+// `together`: every layer's inputs are at hand, so this layer's launches may
+// wait for other layers' (flush_layers).
+uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, bool together, tkh_error *err) {
+    DecodeBatchOfLayers *batch = together ? &s->steps : nullptr;
     tkh_session::Chunk &c = s->chunk;
     const uint64_t start = c.start, count = c.count;
     const bool position_indexed = c.position_indexed;
@@ -644,13 +657,32 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
     sh.low_freq_factor = o.low_freq_factor;
     sh.high_freq_factor = o.high_freq_factor;
     sh.original_max_positions = o.original_max_positions;
+    void *q_rows = s->q_scratch;  // the chunk's produced Q
+    // The layer's producer, launched at once or with the other layers'.
+    auto produce = [&](const tkh_producer_shape &shape, const float *q, const float *k, const float *v, const float *qn,
+                       const float *kn, void *k_out, void *v_out, uint64_t head_stride, const float *context) -> uint32_t {
+        if (!together || s->q_slots == 1)
+            return launch_producer(ctx, &shape, o.storage, q, k, v, qn, kn, q_rows, k_out, v_out, head_stride, err, s->rope,
+                                   o.position_offset);
+        const tkh::ProduceParams p = producer_params(ctx, &shape, q, k, v, qn, kn, q_rows, k_out, v_out, head_stride, s->rope,
+                                                     o.position_offset);
+        s->layers.kv_heads = Hkv;
+        TRY(add_chunk_producer(ctx, &s->layers, p, o.storage, context, s->q_slots, &q_rows,
+                               o.prefill_chunk_size * Hq * D * es, err));
+        ctx->collect = &s->layers;
+        return TKH_OK;
+    };
+    struct Uncollect {
+        tkh_context *ctx;
+        ~Uncollect() { ctx->collect = nullptr; }
+    } uncollect{ctx};
     // Attention of the chunk's Q (in the Q scratch) over a linear cache's keys
     // [0, start + count): Model::run -> LayerKv::attend -> attention_cached
     // (src/model/mod.rs:645-662), or the window form with a score scale.
     auto attend_linear = [&](tkh_kv *kv, uint64_t window, float *context) -> uint32_t {
         if (o.score_scale == 0.0f) {
             tkh_cached_shape cs{count, Hq, Hkv, D, kv->capacity, start};
-            return tkh_attention_cached(ctx, &cs, o.storage, s->q_scratch, count * Hq * D, kv->k,
+            return tkh_attention_cached(ctx, &cs, o.storage, q_rows, count * Hq * D, kv->k,
                                         Hkv * kv->capacity * D, kv->v, Hkv * kv->capacity * D,
                                         context, count * Hq * D, nullptr, 0, nullptr, 0, err);
         }
@@ -667,7 +699,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
         ws.window = window;
         ws.scale = o.score_scale;
         ws.softcap = o.softcap;
-        return tkh_window_attention(ctx, &ws, o.storage, s->q_scratch, count * Hq * D, kv->k,
+        return tkh_window_attention(ctx, &ws, o.storage, q_rows, count * Hq * D, kv->k,
                                     Hkv * kv->capacity * D, kv->v, Hkv * kv->capacity * D, context,
                                     count * Hq * D, nullptr, 0, nullptr, 0, err);
     };
@@ -758,8 +790,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
         }
         tkh_producer_shape qs = sh;
         qs.kv_heads = 0;
-        TRY(launch_producer(ctx, &qs, o.storage, q, nullptr, nullptr, io.q_norm, nullptr,
-                            s->q_scratch, nullptr, nullptr, 0, err, s->rope, o.position_offset));
+        TRY(produce(qs, q, nullptr, nullptr, io.q_norm, nullptr, nullptr, nullptr, 0, context));
         if (!ring) {
             TRY(attend_linear(kv, window, context));
         } else {
@@ -767,7 +798,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
             tkh_span_shape span{};
             TRY(tkh_kv_view(kv, &owner_frame[owner], Hq, o.score_scale, segs, &span, err));
             span.softcap = o.softcap;
-            TRY(tkh_span_attention(ctx, &span, o.storage, s->q_scratch, count * Hq * D, segs,
+            TRY(tkh_span_attention(ctx, &span, o.storage, q_rows, count * Hq * D, segs,
                                    context, count * Hq * D, nullptr, 0, nullptr, 0, err));
         }
         return ok(err);
@@ -787,8 +818,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
         TRY(attention_cached_fused(ctx, &cs, o.storage, kv->k, kv->v, context, f, batch, err));
     } else if (!ring) {
         uint8_t *kb = (uint8_t *)kv->k + start * D * es, *vb = (uint8_t *)kv->v + start * D * es;
-        TRY(launch_producer(ctx, &sh, o.storage, q, k, v, io.q_norm, io.k_norm, s->q_scratch,
-                            kb, vb, kv->capacity * D, err, s->rope, o.position_offset));
+        TRY(produce(sh, q, k, v, io.q_norm, io.k_norm, kb, vb, kv->capacity * D, context));
         TRY(attend_linear(kv, window, context));
     } else {
         // Sliding layer: stage the chunk, attend over the ring's old spans
@@ -799,9 +829,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
                         (unsigned long long)l, (unsigned long long)kv->offset,
                         (unsigned long long)start);
         if (!fused_step)
-            TRY(launch_producer(ctx, &sh, o.storage, q, k, v, io.q_norm, io.k_norm, s->q_scratch,
-                                s->stage_k[owner], s->stage_v[owner], count * D, err, s->rope,
-                                o.position_offset));
+            TRY(produce(sh, q, k, v, io.q_norm, io.k_norm, s->stage_k[owner], s->stage_v[owner], count * D, context));
         tkh_kv_frame f{};
         f.k = s->stage_k[owner];
         f.v = s->stage_v[owner];
@@ -819,7 +847,7 @@ uint32_t eval_layer(tkh_session *s, uint64_t l, const tkh_layer_io &io, DecodeBa
                                                    (int64_t)D, (int64_t)(span.keys - 1), 0);
             TRY(span_attention_fused(ctx, &span, o.storage, segs, context, fd, batch, err));
         } else {
-            TRY(tkh_span_attention(ctx, &span, o.storage, s->q_scratch, count * Hq * D, segs,
+            TRY(tkh_span_attention(ctx, &span, o.storage, q_rows, count * Hq * D, segs,
                                    context, count * Hq * D, nullptr, 0, nullptr, 0, err));
         }
         ring_kv.push_back(kv);
@@ -860,14 +888,18 @@ uint32_t commit_chunk(tkh_session *s, tkh_error *err) {
 uint32_t evaluate_chunk(tkh_session *s, const tkh_layer_io *layers, uint64_t start,
                         uint64_t count, bool position_indexed, tkh_error *err) {
     begin_chunk(s, start, count, position_indexed);
-    // A decode step's layers go out in as few launches as their number allows:
-    // alone, each is a latency-bound launch and a merge on a mostly idle card.
-    // Six 8/4/256 layers at about 2,050 keys (five of window 1,024): six
-    // launches of 7.5 us and six merges of 3.0 became one of 14.9 and one of 4.3.
+    // The layers go out in as few launches as their number allows: alone, each
+    // is latency-bound launches and a merge on a mostly idle card.  Six 8/4/256
+    // layers, five of window 1,024, at about 2,050 keys: a step's six launches of
+    // 7.5 us and six merges of 3.0 became one of 14.9 and one of 4.0; a 128-token
+    // chunk's six producers, attention launches and merges (4.0 + 15.7 + 4.5 us
+    // each) one of 7.3, one of 39 and one of 11.
     s->steps.args.count = 0;
+    s->layers.clear();
     uint32_t rc = TKH_OK;
-    for (uint64_t l = 0; l < s->opt.layers && rc == TKH_OK; ++l) rc = eval_layer(s, l, layers[l], &s->steps, err);
+    for (uint64_t l = 0; l < s->opt.layers && rc == TKH_OK; ++l) rc = eval_layer(s, l, layers[l], true, err);
     if (rc == TKH_OK) rc = flush_decode_layers(s->ctx, &s->steps, err);
+    if (rc == TKH_OK) rc = flush_chunk_layers(s->ctx, &s->layers, err);
     if (rc != TKH_OK) {
         abort_chunk(s);
         return rc;
@@ -905,7 +937,7 @@ extern "C" uint32_t tkh_session_chunk_layer(tkh_session *s, uint64_t layer, cons
                     (unsigned long long)c.next_layer, (unsigned long long)layer);
     if (!io) return invalid("layer inputs", err);
     if (s->ctx) {
-        const uint32_t rc = eval_layer(s, layer, *io, nullptr, err);
+        const uint32_t rc = eval_layer(s, layer, *io, false, err);
         if (rc != TKH_OK) {
             abort_chunk(s);
             return rc;
