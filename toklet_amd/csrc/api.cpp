@@ -24,8 +24,9 @@
 #include "host.hpp"
 
 extern "C" int tkh_tile_head(int head_dim);
-extern "C" int tkh_tile_keys(int head_dim);
-extern "C" int tkh_tile_row_waves(int head_dim);
+extern "C" int tkh_tile_keys(int dtype, int head_dim);
+extern "C" int tkh_tile_row_waves(int dtype, int head_dim);
+extern "C" int tkh_tile_share(int dtype, int head_dim);
 extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStream_t stream,
                                       hipEvent_t start, hipEvent_t stop);
 extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
@@ -707,7 +708,7 @@ uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
 // combine launch when the keys are split and a probability launch when asked.
 uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_error *err) {
     const int64_t D = plan.head_dim, Hq = plan.query_heads, Hkv = plan.kv_heads, G = Hq / Hkv;
-    const int64_t DP = tkh_tile_head((int)D), KT = tkh_tile_keys((int)D);
+    const int64_t DP = tkh_tile_head((int)D), KT = tkh_tile_keys((int)plan.dtype, (int)D);
     // One partial per output row must fit the workspace, split or not.
     {
         size_t need = 0;
@@ -738,13 +739,13 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     // long, for at most tile_groups workgroups in all: two fit on a CU, and a few
     // more than that many take a second round (128-token FP32 chunk at offset
     // 1920, 14/2/64: 532 workgroups 29 us, the last 20 of them starting 17 us late).
-    const int waves = tkh_tile_row_waves((int)D);
+    const int waves = tkh_tile_row_waves((int)plan.dtype, (int)D);
     const int rw = std::min(waves, max_rows <= 16 ? 1 : (max_rows <= 32 ? 2 : 4));
     int64_t base = 0;
     for (auto &p : group) base += Hkv * (((int64_t)p.queries * G + 16 * rw - 1) / (16 * rw));
     int64_t splits = std::max<int64_t>(1, ctx->tile_groups / base);
     splits = std::min<int64_t>(splits, std::max<int64_t>(1, max_span / KT));
-    int kw = max_span > KT ? (int)std::min<int64_t>(waves / rw, KT / 16) : 1;
+    int kw = max_span > KT ? std::min(waves / rw, tkh_tile_share((int)plan.dtype, (int)D)) : 1;
     splits = std::min<int64_t>(splits, 64 / kw);
     auto fits = [&](int64_t s) {
         return s == 1 || (size_t)rows * s * (DP + 2) * sizeof(float) <= split_region_bytes(ctx);

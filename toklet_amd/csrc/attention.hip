@@ -85,6 +85,169 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// What a workgroup and one of its waves cover.
+struct TileWork {
+    int kvh, split, splits;      // KV head, key split and splits of the problem
+    int m_kv, prow, ks;          // packed rows of the KV head, this lane's, and the wave's share of the keys
+    int t_row, h_row;            // its token and query head (a valid row's)
+    bool active, rvalid;         // the wave has rows; the lane's row exists
+    int64_t lo;                  // first logical key of the workgroup's range
+    int n;                       // its keys; relative to `lo` from here on:
+    int rlo, rhi;                // keys the lane's row sees
+    int wlo, whi;                // ... some row of the wave sees
+    int vlo, vhi;                // ... some row of the workgroup sees
+};
+
+// Wave group `wg` (of the rw x kw that share the workgroup) and lane row j.
+__device__ __forceinline__ TileWork tile_work(const TileArgs &a, int wg, int j, const_ptr<Problem> *problem) {
+    const Params &p = a.p;
+    TileWork w;
+    const int G = p.group;
+    const bool full_diag = p.diag_mode == 1;
+    // XCD-major tile order (dispatch slot b runs on XCD b % 8): the row blocks
+    // of one KV head, which read the same keys, share an XCD's L2.
+    int64_t tile;
+    {
+        const uint32_t nb = gridDim.x, per = (nb + 7) / 8;
+        const uint32_t x = blockIdx.x % 8, k = blockIdx.x / 8;
+        const uint32_t full = nb % 8 == 0 ? 8 : nb % 8;
+        tile = (int64_t)(x < full ? x * per + k : full * per + (x - full) * (per - 1) + k);
+    }
+    const_ptr<Problem> pr = problem_ptr(p, tile);
+    *problem = pr;
+    const uint32_t local = (uint32_t)(tile - pr->tile_base), nrb = (uint32_t)pr->row_blocks;
+    const uint32_t ns = (uint32_t)pr->splits;
+    const int rb = (int)(local % nrb);
+    w.split = (int)(local / nrb % ns);
+    w.splits = (int)ns;
+    w.kvh = (int)(local / (nrb * ns));
+    const int64_t k_pos0 = pr->k_pos0, keys = pr->keys, q_pos0 = pr->q_pos0;
+    const int m_kv = w.m_kv = pr->queries * G;
+    const int rw = a.rw, rg = wg % rw;
+    w.ks = wg / rw;
+    const int row0 = (rb * rw + rg) * 16;    // the wave's first packed row
+    w.active = w.ks < a.kw && row0 < m_kv;
+    w.prow = row0 + j;
+    w.rvalid = w.ks < a.kw && w.prow < m_kv;
+    const int rrow = w.prow < m_kv ? w.prow : m_kv - 1;
+    w.t_row = (int)((uint32_t)rrow / (uint32_t)G);
+    w.h_row = w.kvh * G + (int)((uint32_t)rrow % (uint32_t)G);
+
+    // The split's keys; the workgroup's rows see [v_lo, v_hi) of them.  The
+    // full diagnostics score every key, so they walk the whole split.
+    const int64_t base_lo = full_diag ? 0 : pr->vis_lo, base_hi = full_diag ? keys : pr->vis_hi;
+    const int64_t s_lo = base_lo + (int64_t)w.split * pr->split_keys;
+    const int64_t s_hi = s_lo + pr->split_keys < base_hi ? s_lo + pr->split_keys : base_hi;
+    int64_t r_lo, r_hi, v_lo, v_hi, w_lo, w_hi, tmp;
+    visible_range(p, k_pos0, keys, q_pos0 + w.t_row, &r_lo, &r_hi);
+    const int wg_first = rb * rw * 16, wg_last = min(wg_first + rw * 16, m_kv) - 1;
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wg_first / (uint32_t)G, &v_lo, &tmp);
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wg_last / (uint32_t)G, &tmp, &v_hi);
+    v_lo = v_lo > s_lo ? v_lo : s_lo;
+    v_hi = v_hi < s_hi ? v_hi : s_hi;
+    const int wv_first = min(row0, m_kv - 1), wv_last = min(row0 + 15, m_kv - 1);
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_first / (uint32_t)G, &w_lo, &tmp);
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_last / (uint32_t)G, &tmp, &w_hi);
+    const int64_t lo = full_diag ? s_lo : v_lo, hi = full_diag ? s_hi : v_hi;
+    const int n = hi > lo ? (int)(hi - lo) : 0;
+    auto rel = [&](int64_t x) { return (int)(x < lo ? 0 : (x > lo + n ? n : x - lo)); };
+    w.lo = lo;
+    w.n = n;
+    w.rlo = w.rvalid ? rel(r_lo) : 0;
+    w.rhi = w.rvalid ? rel(r_hi) : 0;
+    w.wlo = rel(w_lo);
+    w.whi = w.active ? rel(w_hi) : 0;
+    w.vlo = rel(v_lo);
+    w.vhi = rel(v_hi);
+    return w;
+}
+
+// The dots of a staged tile's blocks as masked scores in the exp2 domain, lane
+// row j against keys 16 b + 4 g + r (relative t0 on), with the diagnostics'
+// scores stored by the waves that have `store`.  Returns the lane's maximum.
+template <int NB>
+__device__ __forceinline__ float finish_scores(const Params &p, const TileWork &w, const_ptr<Problem> pr, int t0, int g,
+                                               bool store, const bool (&scored)[NB], f32x4 (&st)[NB], bool &bad) {
+    const float scale = p.scale, cap = p.softcap;
+    const bool full_diag = p.diag_mode == 1;
+    const bool last_row = w.h_row == p.query_heads - 1 && w.t_row == pr->queries - 1;
+    const bool diag = p.diag_mode != 0 && store && w.rvalid && (full_diag || last_row);
+    float *const xs = p.scores ? p.scores : p.probs;  // raw scores (attn_tile_probs turns them into probabilities)
+    float tmax = NEG_INF;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (!scored[b]) {
+            st[b] = f32x4{NEG_INF, NEG_INF, NEG_INF, NEG_INF};
+            continue;
+        }
+        f32x4 x;
+        for (int r = 0; r < 4; ++r) x[r] = st[b][r] * scale;
+        if (cap != 0.0f)
+            for (int r = 0; r < 4; ++r) x[r] = softcap_f(x[r], cap);
+        const int key = t0 + 16 * b + 4 * g;
+        for (int r = 0; r < 4; ++r) {
+            const bool vis = key + r >= w.rlo && key + r < w.rhi;
+            bad |= vis && !is_finite_f(x[r]);
+            st[b][r] = vis ? x[r] * LOG2E : NEG_INF;
+            tmax = fmaxf(tmax, st[b][r]);
+        }
+        if (diag) {
+            const int first = full_diag ? 0 : w.rlo, end = full_diag ? w.n : w.rhi;
+            float *xr = xs + (full_diag ? ((int64_t)w.h_row * pr->queries + w.t_row) * pr->keys : 0) + w.lo + key;
+            if (key >= first && key + 4 <= end) *reinterpret_cast<f32x4u *>(xr) = x;
+            else
+                for (int r = 0; r < 4; ++r)
+                    if (key + r >= first && key + r < end) xr[r] = x[r];
+        }
+    }
+    return tmax;
+}
+
+// Where a lane's row of unnormalised context goes: divided by its mass into the
+// output, or into its partial with (max, mass) beside it.  `lead`: this lane
+// stores the row's (max, mass).
+struct TileOut {
+    bool direct, write;
+    bool bad_mass = false, bad_out = false;
+    float inv;
+    float *row;
+    int D;
+    __device__ __forceinline__ TileOut(const TileArgs &a, const TileWork &w, const_ptr<Problem> pr, int dp, bool lead, float m,
+                                       float l) {
+        const Params &p = a.p;
+        const int S = w.splits * a.kw;
+        const int64_t part = pr->slot_base + ((int64_t)w.kvh * w.m_kv + w.prow) * S + w.split * a.kw + w.ks;
+        D = p.head_dim;
+        direct = S == 1;
+        write = direct || m != NEG_INF;  // a partial whose split shows the row no key is never read
+        inv = direct ? 1.0f / l : 1.0f;
+        row = direct ? pr->out + ((int64_t)w.t_row * p.query_heads + w.h_row) * D : p.part_o + part * dp;
+        if (!w.rvalid) return;
+        bad_mass = direct && (!(l > 0.0f) || !is_finite_f(l));
+        if (lead && (!direct || p.diag_mode != 0)) {
+            const f32x2 ml = {m, l};
+            *gstore_ptr<f32x2>(p.part_ml + 2 * part) = ml;
+        }
+    }
+    __device__ __forceinline__ void emit(int d, f32x4 o, bool &bad) {
+        for (int e = 0; e < 4; ++e) {
+            bad |= d + e < D && !is_finite_f(o[e]);
+            o[e] *= inv;
+            bad_out |= d + e < D && !is_finite_f(o[e]);
+        }
+        if (!write) return;
+        if (d + 4 <= D) *reinterpret_cast<f32x4u *>(row + d) = o;
+        else
+            for (int e = 0; e < 4; ++e)
+                if (d + e < D) row[d + e] = o[e];
+    }
+    __device__ __forceinline__ void report(const Params &p, bool bad) const {
+        raise_status(p, bad, ST_NONFINITE_INPUT);
+        raise_status(p, bad_mass, ST_BAD_MASS);
+        raise_status(p, direct && bad_out, ST_NONFINITE_OUTPUT);
+    }
+};
+
 }  // namespace
 
 // What bounds it: v_mfma_f32_16x16x4 (32 cycles for 2,048 FLOP, 157 TFLOP/s
@@ -131,54 +294,14 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     const int G = p.group, Hq = p.query_heads, D = p.head_dim;
     const bool full_diag = p.diag_mode == 1;
 
-    // XCD-major tile order (dispatch slot b runs on XCD b % 8): the row blocks
-    // of one KV head, which read the same keys, share an XCD's L2.
-    int64_t tile;
-    {
-        const uint32_t nb = gridDim.x, per = (nb + 7) / 8;
-        const uint32_t x = blockIdx.x % 8, k = blockIdx.x / 8;
-        const uint32_t full = nb % 8 == 0 ? 8 : nb % 8;
-        tile = (int64_t)(x < full ? x * per + k : full * per + (x - full) * (per - 1) + k);
-    }
-    const_ptr<Problem> pr = problem_ptr(p, tile);
-    const uint32_t local = (uint32_t)(tile - pr->tile_base), nrb = (uint32_t)pr->row_blocks;
-    const uint32_t ns = (uint32_t)pr->splits;
-    const int rb = (int)(local % nrb), split = (int)(local / nrb % ns), kvh = (int)(local / (nrb * ns));
-    const int64_t k_pos0 = pr->k_pos0, keys = pr->keys, q_pos0 = pr->q_pos0;
-    const int m_kv = pr->queries * G, nseg = pr->nseg;
-
-    const int rw = a.rw, kw = a.kw;
+    const_ptr<Problem> pr;
+    const TileWork w = tile_work(a, wave / FS, j, &pr);
+    const int kw = a.kw, ks = w.ks, kvh = w.kvh, m_kv = w.m_kv, nseg = pr->nseg, n = w.n;
     const int fs = wave % FS, f0 = fs * DW;  // the wave's features start at f0
-    const int rg = wave / FS % rw, ks = wave / FS / rw;
-    const int row0 = (rb * rw + rg) * 16;    // the wave's first packed row
-    const bool active = ks < kw && row0 < m_kv;
-    const int prow = row0 + j;
-    const bool rvalid = ks < kw && prow < m_kv;
-    const int rrow = prow < m_kv ? prow : m_kv - 1;
-    const int t_row = (int)((uint32_t)rrow / (uint32_t)G), h_row = kvh * G + (int)((uint32_t)rrow % (uint32_t)G);
-
-    // The split's keys; the workgroup's rows see [v_lo, v_hi) of them.  The
-    // full diagnostics score every key, so they walk the whole split.
-    const int64_t base_lo = full_diag ? 0 : pr->vis_lo, base_hi = full_diag ? keys : pr->vis_hi;
-    const int64_t s_lo = base_lo + (int64_t)split * pr->split_keys;
-    const int64_t s_hi = s_lo + pr->split_keys < base_hi ? s_lo + pr->split_keys : base_hi;
-    int64_t r_lo, r_hi, v_lo, v_hi, w_lo, w_hi, tmp;
-    visible_range(p, k_pos0, keys, q_pos0 + t_row, &r_lo, &r_hi);
-    const int wg_first = rb * rw * 16, wg_last = min(wg_first + rw * 16, m_kv) - 1;
-    visible_range(p, k_pos0, keys, q_pos0 + wg_first / G, &v_lo, &tmp);
-    visible_range(p, k_pos0, keys, q_pos0 + wg_last / G, &tmp, &v_hi);
-    v_lo = v_lo > s_lo ? v_lo : s_lo;
-    v_hi = v_hi < s_hi ? v_hi : s_hi;
-    const int wv_first = min(row0, m_kv - 1), wv_last = min(row0 + 15, m_kv - 1);
-    visible_range(p, k_pos0, keys, q_pos0 + wv_first / G, &w_lo, &tmp);
-    visible_range(p, k_pos0, keys, q_pos0 + wv_last / G, &tmp, &w_hi);
-    const int64_t lo = full_diag ? s_lo : v_lo, hi = full_diag ? s_hi : v_hi;
-    const int n = hi > lo ? (int)(hi - lo) : 0;
-    // Relative to `lo` from here on.
-    auto rel = [&](int64_t x) { return (int)(x < lo ? 0 : (x > lo + n ? n : x - lo)); };
-    const int rlo = rvalid ? rel(r_lo) : 0, rhi = rvalid ? rel(r_hi) : 0;
-    const int wlo = rel(w_lo), whi = active ? rel(w_hi) : 0;
-    const int vlo = rel(v_lo), vhi = rel(v_hi);
+    const bool active = w.active, rvalid = w.rvalid;
+    const int t_row = w.t_row, h_row = w.h_row, rlo = w.rlo, rhi = w.rhi, wlo = w.wlo, whi = w.whi;
+    const int vlo = w.vlo, vhi = w.vhi;
+    const int64_t lo = w.lo, keys = pr->keys;
 
     // Features past the head are zeros in Q, K and V.  A vector load of one
     // reads the row's last chunk instead, so that no load is under a branch: the
@@ -234,9 +357,6 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
         }
     };
 
-    const float scale = p.scale, cap = p.softcap;
-    const bool last_row = h_row == Hq - 1 && t_row == pr->queries - 1;
-    float *const xs = p.scores ? p.scores : p.probs;  // raw scores (attn_tile_probs turns them into probabilities)
     f32x4 acc[FB][4];
     for (int fb = 0; fb < FB; ++fb)
         for (int e = 0; e < 4; ++e) acc[fb][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -285,30 +405,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
                     for (int r = 0; r < 4; ++r) st[b][r] += d[w * NB * 64][r];
             }
         }
-        float tmax = NEG_INF;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (!scored[b]) continue;
-            f32x4 x;
-            for (int r = 0; r < 4; ++r) x[r] = st[b][r] * scale;
-            if (cap != 0.0f)
-                for (int r = 0; r < 4; ++r) x[r] = softcap_f(x[r], cap);
-            const int key = t0 + 16 * b + 4 * g;
-            for (int r = 0; r < 4; ++r) {
-                const bool vis = key + r >= rlo && key + r < rhi;
-                bad |= vis && !is_finite_f(x[r]);
-                st[b][r] = vis ? x[r] * LOG2E : NEG_INF;
-                tmax = fmaxf(tmax, st[b][r]);
-            }
-            if (fs == 0 && p.diag_mode != 0 && rvalid && (full_diag || last_row)) {
-                const int first = full_diag ? 0 : rlo, end = full_diag ? n : rhi;
-                float *xr = xs + (full_diag ? ((int64_t)h_row * pr->queries + t_row) * keys : 0) + lo + key;
-                if (key >= first && key + 4 <= end) *reinterpret_cast<f32x4u *>(xr) = x;
-                else
-                    for (int r = 0; r < 4; ++r)
-                        if (key + r >= first && key + r < end) xr[r] = x[r];
-            }
-        }
+        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, bad);
         // The tile's maximum over the row's four lanes; O and l move with it.
         tmax = row4_max(tmax);
         const float m_new = fmaxf(m_run, tmax);
@@ -341,39 +438,332 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     }
 
     l_run = row4_sum(l_run);
-    const bool direct = ns == 1 && kw == 1;
-    bool bad_mass = false, bad_out = false;
-    if (rvalid) {
-        const int64_t part = pr->slot_base + ((int64_t)kvh * m_kv + prow) * (ns * kw) + split * kw + ks;
-        if (g == 0 && fs == 0 && (!direct || p.diag_mode != 0)) {
-            const f32x2 ml = {m_run, l_run};
-            *gstore_ptr<f32x2>(p.part_ml + 2 * part) = ml;
-        }
-        const float inv = direct ? 1.0f / l_run : 1.0f;
-        bad_mass = direct && (!(l_run > 0.0f) || !is_finite_f(l_run));
-        float *orow = direct ? pr->out + ((int64_t)t_row * Hq + h_row) * D : p.part_o + part * DP;
+    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
+    if (rvalid)
         for (int fb = 0; fb < FB; ++fb)
+            for (int r = 0; r < 4; ++r)
+                out.emit(f0 + 64 * fb + 16 * g + 4 * r, f32x4{acc[fb][0][r], acc[fb][1][r], acc[fb][2][r], acc[fb][3][r]}, bad);
+    out.report(p, bad);
+}
+
+// ---------------------------------------------------------------------------
+// attn_split: the same walk on the 16-bit matrix cores (v_mfma_f32_16x16x32,
+// sixteen times the FP32 rate), with FP32 operands split into 16-bit planes whose
+// products lose nothing FP32 arithmetic keeps.
+//
+//  * bf16 and f16 storage: Q, K and V are planes as they are.  A probability is
+//    split into three bf16 planes (each the rounding of what the last left, so
+//    their sum is the FP32 value), or two f16 ones of 2^11 P (22 bits; the factor
+//    keeps small probabilities' second plane in f16's range).
+//  * F32 storage: Q, K, V and P are three bf16 planes each, and a product of two
+//    values is the six plane products down to 2^-16 (the three left out are below
+//    2^-24, FP32's own rounding).
+//
+// Lane (j, g) holds query row j.  Q.K: A = K plane (key j of a 16-key block,
+// features 32 s + 8 g .. + 7), B = Q.  P.V over 32 keys: the MFMA's k index
+// 8 g + 4 b + r stands for key 16 b + 4 g + r, where the scores already sit, so P
+// needs no exchange; A = V transposed, feature 16 fb + j, staged with its keys in
+// that order.  A thread transposes four keys by four features in registers on the
+// way to LDS.  The 16 rows of an operand read fall on distinct banks: K rows are
+// padded by 16 bytes, V rows (whose size decides whether two workgroups of
+// 512-wide heads fit a CU) have their 16-byte chunks XOR-swizzled by row.
+__host__ __device__ constexpr int split_keys(int DP) { return DP <= 64 ? 64 : 32; }
+__host__ __device__ constexpr int split_feature_waves(int DP) { return DP <= 256 ? 1 : 2; }
+
+namespace {
+
+template <int DT> struct Planes { static constexpr int store = 1, prob = 3; };
+template <> struct Planes<F32> { static constexpr int store = 3, prob = 3; };
+template <> struct Planes<F16> { static constexpr int store = 1, prob = 2; };
+constexpr float PROB_SCALE_F16 = 0x1p11f;
+
+template <int DT> __device__ __forceinline__ f32x4 mfma32k(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (DT == F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Two floats rounded to bf16 and packed; they keep what the rounding left.  (Cut
+// off instead, values either side of a power of two have leading planes 0.4%
+// apart, and sums that cancel in FP32 no longer do plane by plane.)  LIMIT: a
+// value that would round to infinity takes the largest bf16 first.
+template <bool LIMIT> __device__ __forceinline__ uint32_t plane2(float &a, float &b) {
+    constexpr float top = 0x1.fep127f;
+    const f32x2 v = {LIMIT ? __builtin_amdgcn_fmed3f(a, -top, top) : a, LIMIT ? __builtin_amdgcn_fmed3f(b, -top, top) : b};
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+    a -= __builtin_bit_cast(float, w << 16);
+    b -= __builtin_bit_cast(float, w & 0xffff0000u);
+    return w;
+}
+
+// Eight stored elements as planes of an MFMA operand.
+template <int DT>
+__device__ __forceinline__ void planes8(typename Raw4<DT>::T lo, typename Raw4<DT>::T hi, u32x4 (&out)[Planes<DT>::store]) {
+    if constexpr (DT == F32) {
+        const f32x4 x = widen4<DT>(lo), y = widen4<DT>(hi);
+        float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+        for (int e = 0; e < 4; ++e) {
+            out[0][e] = plane2<true>(v[2 * e], v[2 * e + 1]);
+            out[1][e] = plane2<false>(v[2 * e], v[2 * e + 1]);
+            out[2][e] = plane2<false>(v[2 * e], v[2 * e + 1]);
+        }
+    } else {
+        out[0] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+}
+
+// A lane's probabilities of 32 keys (two score blocks) as planes.
+template <int DT>
+__device__ __forceinline__ void prob_planes(const f32x4 &a, const f32x4 &b, u32x4 (&out)[Planes<DT>::prob]) {
+    f32x4 x = a, y = b;
+    if constexpr (DT == F16) {
+        auto half2 = [](float u, float v) {
+            const f16x2 h = {(_Float16)u, (_Float16)v};
+            return __builtin_bit_cast(uint32_t, h);
+        };
+        for (int e = 0; e < 4; ++e) {
+            x[e] *= PROB_SCALE_F16;
+            y[e] *= PROB_SCALE_F16;
+        }
+        for (int pl = 0; pl < 2; ++pl) {
+            out[pl] = u32x4{half2(x[0], x[1]), half2(x[2], x[3]), half2(y[0], y[1]), half2(y[2], y[3])};
+            for (int e = 0; e < 4; ++e) {
+                x[e] -= (float)(_Float16)x[e];
+                y[e] -= (float)(_Float16)y[e];
+            }
+        }
+    } else {
+        float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+        for (int pl = 0; pl < 3; ++pl)
+            for (int e = 0; e < 4; ++e) out[pl][e] = plane2<false>(v[2 * e], v[2 * e + 1]);
+    }
+}
+
+}  // namespace
+
+template <int DT, int DP, bool VEC>
+__global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
+    warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
+    constexpr int KT = split_keys(DP), NB = KT / 16, NG = KT / 32, FS = split_feature_waves(DP);
+    constexpr int DW = DP / FS, QS = DW / 32, FB = DW / 16;   // a wave's features, Q.K steps, P.V blocks
+    constexpr int SP = Planes<DT>::store, PP = Planes<DT>::prob;
+    constexpr int KROW = DP * 2 + 16, VROW = KT * 2;          // staged row bytes: K per key, V per feature
+    constexpr int KPL = KT * KROW, VPL = DP * VROW;           // bytes per plane
+    constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / 16 / 256;  // a thread's 8-feature K chunks, 4 x 4 V blocks
+    static_assert(NK >= 1 && NV >= 1, "staging covers the tile");
+    __shared__ __attribute__((aligned(16))) uint8_t kt[SP * KPL];
+    __shared__ __attribute__((aligned(16))) uint8_t vt[SP * VPL];
+    __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? 4 * NB * 64 : 1];  // partial scores
+    using Raw = typename Raw4<DT>::T;
+    const Params &p = a.p;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int j = lane & 15, g = lane >> 4;
+    const int D = p.head_dim;
+    const bool full_diag = p.diag_mode == 1;
+    const_ptr<Problem> pr;
+    const TileWork w = tile_work(a, wave / FS, j, &pr);
+    const int fs = wave % FS, f0 = fs * DW;  // the wave's features start at f0
+    const int nseg = pr->nseg, n = w.n;
+    // Byte offset of 16-byte chunk c of V row f.
+    auto v_at = [](int f, int c) { return f * VROW + ((c ^ (KT == 32 ? f >> 2 & 3 : f >> 1 & 7)) << 4); };
+
+    // Features past the head are zeros in Q, K and V (attn_tile's loads).
+    const int last = D - 4;
+    auto feature = [&](int d) { return VEC ? min(d, last) : d; };
+    const Raw none{};
+    u32x4 q[QS][SP];
+    {
+        const int64_t at = (int64_t)w.t_row * pr->q_row_stride + (int64_t)w.h_row * D;
+        Raw lo[QS], hi[QS];
+        for (int s = 0; s < QS; ++s) {
+            const int d = f0 + 32 * s + 8 * g;
+            lo[s] = load4<DT, VEC>(pr->q, at + feature(d), D - d);
+            hi[s] = load4<DT, VEC>(pr->q, at + feature(d + 4), D - d - 4);
+        }
+        for (int s = 0; s < QS; ++s) {
+            const int d = f0 + 32 * s + 8 * g;
+            planes8<DT>(!VEC || d <= last ? lo[s] : none, !VEC || d + 4 <= last ? hi[s] : none, q[s]);
+        }
+    }
+
+    // K chunk m of a thread: row i / (DP / 8), features 8 (i % (DP / 8)).  V block
+    // m: key quad i % 8 of its 32-key group, features 4 (i / 8 % (DP / 4)).
+    constexpr int CPR = DP / 8, FPR = DP / 4;
+    Raw kreg[NK][2], vreg[NV][4];
+    auto fetch_rows = [&](int t0, auto at) {
+#pragma unroll
+        for (int m = 0; m < NK; ++m) {
+            const int i = tid + 256 * m, d = 8 * (i % CPR);
+            const void *kb, *vb;
+            const int64_t off = at(w.lo + min(t0 + i / CPR, n - 1), &kb, &vb);
+            kreg[m][0] = load4<DT, VEC>(kb, off + feature(d), D - d);
+            kreg[m][1] = load4<DT, VEC>(kb, off + feature(d + 4), D - d - 4);
+        }
+#pragma unroll
+        for (int m = 0; m < NV; ++m) {
+            const int i = tid + 256 * m, d = 4 * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
             for (int r = 0; r < 4; ++r) {
-                const int d = f0 + 64 * fb + 16 * g + 4 * r;
-                f32x4 o;
+                const void *kb, *vb;
+                const int64_t off = at(w.lo + min(t0 + k0 + r, n - 1), &kb, &vb);
+                vreg[m][r] = load4<DT, VEC>(vb, off + feature(d), D - d);
+            }
+        }
+    };
+    auto fetch = [&](int t0) {
+        if (nseg == 1) {
+            const void *kb = pr->seg[0].k, *vb = pr->seg[0].v;
+            const int64_t rs = pr->seg[0].row_stride, head = (int64_t)w.kvh * pr->seg[0].head_stride;
+            fetch_rows(t0, [&](int64_t key, const void **k, const void **v) {
+                *k = kb;
+                *v = vb;
+                return head + key * rs;
+            });
+        } else {
+            fetch_rows(t0, [&](int64_t key, const void **k, const void **v) { return seg_select(pr, key, w.kvh, k, v); });
+        }
+    };
+    auto stage = [&](int t0) {
+#pragma unroll
+        for (int m = 0; m < NK; ++m) {
+            const int i = tid + 256 * m, d = 8 * (i % CPR);
+            u32x4 pl[SP];
+            planes8<DT>(!VEC || d <= last ? kreg[m][0] : none, !VEC || d + 4 <= last ? kreg[m][1] : none, pl);
+            for (int s = 0; s < SP; ++s) *reinterpret_cast<u32x4 *>(kt + s * KPL + i / CPR * KROW + 2 * d) = pl[s];
+        }
+#pragma unroll
+        for (int m = 0; m < NV; ++m) {
+            const int i = tid + 256 * m, qd = i % 8, d = 4 * (i / 8 % FPR), t = i / (8 * FPR);
+            const int k0 = t0 + 32 * t + 4 * qd;
+            Raw x[4];
+            for (int r = 0; r < 4; ++r)
+                x[r] = (!VEC || d <= last) && k0 + r >= w.vlo && k0 + r < w.vhi ? vreg[m][r] : none;
+            // Row f holds the group's keys as 8-byte pieces: g = qd % 4 first, then b = qd / 4.
+            auto to = [&](int e) { return vt + v_at(d + e, 4 * t + (qd & 3)) + 8 * (qd >> 2); };
+            if constexpr (DT == F32) {
+                f32x4 y[4];
+                for (int r = 0; r < 4; ++r) y[r] = widen4<DT>(x[r]);
                 for (int e = 0; e < 4; ++e) {
-                    o[e] = acc[fb][e][r];
-                    bad |= d + e < D && !is_finite_f(o[e]);
-                    o[e] *= inv;
-                    bad_out |= d + e < D && !is_finite_f(o[e]);
+                    float v[4] = {y[0][e], y[1][e], y[2][e], y[3][e]};
+                    for (int s = 0; s < 3; ++s) {
+                        using Quad = typename Raw4<F16>::T;
+                        const Quad o = s == 0 ? Quad{plane2<true>(v[0], v[1]), plane2<true>(v[2], v[3])}
+                                              : Quad{plane2<false>(v[0], v[1]), plane2<false>(v[2], v[3])};
+                        *reinterpret_cast<Quad *>(to(e) + s * VPL) = o;
+                    }
                 }
-                // A partial whose split shows the row no key is never read.
-                if (d + 4 <= D) {
-                    if (direct || m_run != NEG_INF) *reinterpret_cast<f32x4u *>(orow + d) = o;
-                } else {
-                    for (int e = 0; e < 4; ++e)
-                        if (d + e < D) orow[d + e] = o[e];
+            } else {
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t pick = e & 1 ? 0x07060302u : 0x05040100u;
+                    const uint32_t o0 = __builtin_amdgcn_perm(x[1][e >> 1], x[0][e >> 1], pick);
+                    const uint32_t o1 = __builtin_amdgcn_perm(x[3][e >> 1], x[2][e >> 1], pick);
+                    *reinterpret_cast<Raw *>(to(e)) = Raw{o0, o1};
                 }
             }
+        }
+    };
+
+    f32x4 acc[FB];
+    for (int fb = 0; fb < FB; ++fb) acc[fb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = NEG_INF, l_run = 0.0f;
+    bool bad = false;
+
+    if (n > 0) fetch(0);
+    for (int t0 = 0; t0 < n; t0 += KT) {
+        __syncthreads();
+        stage(t0);
+        __syncthreads();
+        if (t0 + KT < n) fetch(t0 + KT);
+        f32x4 st[NB];
+        bool seen[NB], scored[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int k0 = t0 + 16 * b;
+            seen[b] = w.active && k0 < w.whi && k0 + 16 > w.wlo;
+            scored[b] = seen[b] || (full_diag && w.active && k0 < n);
+            f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;  // the leading planes, the rest (or two chains)
+            if (scored[b]) {
+                const uint8_t *kr = kt + (16 * b + j) * KROW + 2 * f0 + 16 * g;
+#pragma unroll
+                for (int s = 0; s < QS; ++s) {
+                    u32x4 k[SP];
+                    for (int pl = 0; pl < SP; ++pl) k[pl] = *reinterpret_cast<const u32x4 *>(kr + pl * KPL + 64 * s);
+                    if constexpr (SP == 3) {
+                        s0 = mfma32k<DT>(k[0], q[s][0], s0);
+                        s1 = mfma32k<DT>(k[2], q[s][0], s1);
+                        s1 = mfma32k<DT>(k[0], q[s][2], s1);
+                        s1 = mfma32k<DT>(k[1], q[s][1], s1);
+                        s1 = mfma32k<DT>(k[1], q[s][0], s1);
+                        s1 = mfma32k<DT>(k[0], q[s][1], s1);
+                    } else if (s % 2 == 0) {
+                        s0 = mfma32k<DT>(k[0], q[s][0], s0);
+                    } else {
+                        s1 = mfma32k<DT>(k[0], q[s][0], s1);
+                    }
+                }
+            }
+            for (int r = 0; r < 4; ++r) st[b][r] = s0[r] + s1[r];
+            if constexpr (FS > 1) dots[(wave * NB + b) * 64 + lane] = st[b];
+        }
+        if constexpr (FS > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const f32x4 *d = dots + (wave - fs) * NB * 64 + b * 64 + lane;
+                st[b] = d[0];
+                for (int x = 1; x < FS; ++x)
+                    for (int r = 0; r < 4; ++r) st[b][r] += d[x * NB * 64][r];
+            }
+        }
+        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, bad);
+        tmax = row4_max(tmax);
+        const float m_new = fmaxf(m_run, tmax);
+        const float base = m_new == NEG_INF ? 0.0f : m_new;
+        if (__ballot(m_new > m_run) != 0) {
+            const float corr = __builtin_amdgcn_exp2f(m_run - base);
+            l_run *= corr;
+            for (int fb = 0; fb < FB; ++fb)
+                for (int r = 0; r < 4; ++r) acc[fb][r] *= corr;
+            m_run = m_new;
+        }
+#pragma unroll
+        for (int t = 0; t < NG; ++t) {
+            if (!seen[2 * t] && !seen[2 * t + 1]) continue;
+            for (int b = 2 * t; b < 2 * t + 2; ++b)
+                for (int r = 0; r < 4; ++r) {
+                    st[b][r] = __builtin_amdgcn_exp2f(st[b][r] - base);
+                    l_run += st[b][r];
+                }
+            u32x4 pb[PP];
+            prob_planes<DT>(st[2 * t], st[2 * t + 1], pb);
+            const uint8_t *vr = vt + v_at(f0 + j, 4 * t + g);  // the swizzle repeats every 16 rows
+#pragma unroll
+            for (int fb = 0; fb < FB; ++fb) {
+                u32x4 v[SP];
+                for (int pl = 0; pl < SP; ++pl) v[pl] = *reinterpret_cast<const u32x4 *>(vr + pl * VPL + 16 * fb * VROW);
+                f32x4 o = acc[fb];
+                if constexpr (SP == 3) {
+                    o = mfma32k<DT>(v[2], pb[0], o);
+                    o = mfma32k<DT>(v[0], pb[2], o);
+                    o = mfma32k<DT>(v[1], pb[1], o);
+                    o = mfma32k<DT>(v[1], pb[0], o);
+                    o = mfma32k<DT>(v[0], pb[1], o);
+                } else {
+                    for (int pl = PP - 1; pl > 0; --pl) o = mfma32k<DT>(v[0], pb[pl], o);
+                }
+                acc[fb] = mfma32k<DT>(v[0], pb[0], o);
+            }
+        }
     }
-    raise_status(p, bad, ST_NONFINITE_INPUT);
-    raise_status(p, bad_mass, ST_BAD_MASS);
-    raise_status(p, direct && bad_out, ST_NONFINITE_OUTPUT);
+
+    l_run = row4_sum(l_run);
+    if constexpr (DT == F16)
+        for (int fb = 0; fb < FB; ++fb)
+            for (int r = 0; r < 4; ++r) acc[fb][r] *= 1.0f / PROB_SCALE_F16;
+    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
+    if (w.rvalid)
+        for (int fb = 0; fb < FB; ++fb) out.emit(f0 + 16 * fb + 4 * g, acc[fb], bad);
+    out.report(p, bad);
 }
 
 // Merged (max, mass) of a row's S partials.
@@ -482,13 +872,27 @@ __global__ __launch_bounds__(256) void attn_tile_probs(TileArgs a) {
 
 }  // namespace tkh
 
-// Head sizes the kernel is built for (the smallest that holds `head_dim`), the
-// keys of its staged tile, and the row groups a workgroup has waves for.
+// Head sizes the kernels are built for (the smallest that holds `head_dim`).
 extern "C" int tkh_tile_head(int head_dim) {
     return head_dim <= 64 ? 64 : (head_dim <= 128 ? 128 : (head_dim <= 256 ? 256 : 512));
 }
-extern "C" int tkh_tile_keys(int head_dim) { return tkh::tile_keys(tkh_tile_head(head_dim)); }
-extern "C" int tkh_tile_row_waves(int head_dim) { return 4 / tkh::tile_feature_waves(tkh_tile_head(head_dim)); }
+// attn_split takes every 16-bit launch and FP32 ones up to 128, whose six plane
+// products cost 6/16 of FP32 MFMAs; three planes of wider FP32 tiles do not leave
+// room for two workgroups in LDS, and those stay on attn_tile.
+static bool tile_splits(int dtype, int head_dim) { return dtype != tkh::F32 || tkh_tile_head(head_dim) <= 128; }
+// Keys of a staged tile, row groups a workgroup has waves for, and how many of
+// its waves may share a row group's keys.
+extern "C" int tkh_tile_keys(int dtype, int head_dim) {
+    const int dp = tkh_tile_head(head_dim);
+    return tile_splits(dtype, head_dim) ? tkh::split_keys(dp) : tkh::tile_keys(dp);
+}
+extern "C" int tkh_tile_row_waves(int dtype, int head_dim) {
+    const int dp = tkh_tile_head(head_dim);
+    return 4 / (tile_splits(dtype, head_dim) ? tkh::split_feature_waves(dp) : tkh::tile_feature_waves(dp));
+}
+extern "C" int tkh_tile_share(int dtype, int head_dim) {
+    return tile_splits(dtype, head_dim) ? 1 : tkh_tile_keys(dtype, head_dim) / 16;
+}
 
 // start/stop, when not null, are recorded around the kernel by the dispatch
 // itself (hipExtLaunchKernelGGL), so profiled durations exclude the host gap
@@ -498,15 +902,16 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
     using namespace tkh;
     const int dp = tkh_tile_head(a->p.head_dim);
     dim3 grid((unsigned)a->p.total_tiles), block(256);
-#define TKH_TILE(DT, DP)                                                                               \
-    if (dtype == DT && dp == DP) {                                                                     \
-        if (a->vec) hipExtLaunchKernelGGL((attn_tile<DT, DP, true>), grid, block, 0, stream, start, stop, 0, *a); \
-        else hipExtLaunchKernelGGL((attn_tile<DT, DP, false>), grid, block, 0, stream, start, stop, 0, *a);       \
-        return hipGetLastError();                                                                      \
+#define TKH_TILE(KERNEL, DT, DP)                                                                        \
+    if (dtype == DT && dp == DP) {                                                                      \
+        if (a->vec) hipExtLaunchKernelGGL((KERNEL<DT, DP, true>), grid, block, 0, stream, start, stop, 0, *a); \
+        else hipExtLaunchKernelGGL((KERNEL<DT, DP, false>), grid, block, 0, stream, start, stop, 0, *a);       \
+        return hipGetLastError();                                                                       \
     }
-    TKH_TILE(F32, 64) TKH_TILE(F32, 128) TKH_TILE(F32, 256) TKH_TILE(F32, 512)
-    TKH_TILE(F16, 64) TKH_TILE(F16, 128) TKH_TILE(F16, 256) TKH_TILE(F16, 512)
-    TKH_TILE(BF16, 64) TKH_TILE(BF16, 128) TKH_TILE(BF16, 256) TKH_TILE(BF16, 512)
+    TKH_TILE(attn_split, F32, 64) TKH_TILE(attn_split, F32, 128) TKH_TILE(attn_tile, F32, 256) TKH_TILE(attn_tile, F32, 512)
+    TKH_TILE(attn_split, F16, 64) TKH_TILE(attn_split, F16, 128) TKH_TILE(attn_split, F16, 256) TKH_TILE(attn_split, F16, 512)
+    TKH_TILE(attn_split, BF16, 64) TKH_TILE(attn_split, BF16, 128) TKH_TILE(attn_split, BF16, 256)
+    TKH_TILE(attn_split, BF16, 512)
 #undef TKH_TILE
     return hipErrorInvalidValue;
 }
