@@ -31,7 +31,6 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
                                       hipEvent_t start, hipEvent_t stop);
 extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
                                             hipEvent_t start, hipEvent_t stop);
-extern "C" hipError_t tkh_launch_tile_probs(const tkh::TileArgs *a, hipStream_t stream);
 extern "C" hipError_t tkh_launch_kv_append(int src, int dst, const void *k, const void *v,
                                            void *kc, void *vc, int64_t tokens, int heads,
                                            int dims, int64_t capacity, int64_t offset,
@@ -732,6 +731,7 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
         for (int i = 0; i < p.nseg; ++i) {
             at |= (uintptr_t)p.seg[i].k | (uintptr_t)p.seg[i].v;
             strides |= p.seg[i].head_stride | p.seg[i].row_stride;
+            vec = vec && p.seg[i].row_stride < INT32_MAX / 4 / 64;  // a tile's offsets in 32 bits
         }
         vec = vec && at % chunk == 0 && strides % 4 == 0;
     }
@@ -788,18 +788,14 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     args.kw = kw;
     args.vec = vec ? 1 : 0;
 
-    const bool merge = splits * kw > 1;
+    const bool split = splits * kw > 1, second = split || plan.probs;
     hipEvent_t *ev = nullptr;
-    if (ctx->profiling) TRY(profile_slot(ctx, &ev, merge, err));
+    if (ctx->profiling) TRY(profile_slot(ctx, &ev, second, err));
     hipError_t e = tkh_launch_tile(&args, (int)plan.dtype, ctx->stream, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
     if (e != hipSuccess) return device_error(e, "attention launch", err);
-    if (merge) {
-        e = tkh_launch_tile_merge(&args, rows, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);
+    if (second) {
+        e = tkh_launch_tile_merge(&args, split ? rows : 0, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);
         if (e != hipSuccess) return device_error(e, "combine launch", err);
-    }
-    if (plan.probs) {
-        e = tkh_launch_tile_probs(&args, ctx->stream);
-        if (e != hipSuccess) return device_error(e, "probability launch", err);
     }
     return TKH_OK;
 }

@@ -7,10 +7,11 @@
 //  * attn_tile<DT, DP>: any head_dim D <= DP.  A workgroup is four waves over
 //    16 packed rows each (query x head of the GQA group) of one (problem, KV
 //    head), optionally one key split of it.
+//  * attn_split<DT, DP>: the same on the 16-bit matrix cores, FP32 values as
+//    16-bit planes.
 //  * attn_tile_merge: combines split-K partials (max, mass, unnormalised
-//    context) and writes the context.
-//  * attn_tile_probs: the diagnostics' probabilities from the stored scores
-//    and each row's merged (max, mass).
+//    context) and writes the context; makes the diagnostics' probabilities from
+//    the stored scores and each row's merged (max, mass).
 //
 // Scores are kept in the exp2 domain (score * log2 e) so the softmax uses
 // v_exp_f32 directly.  Masked keys contribute exactly zero.
@@ -58,12 +59,11 @@ template <int DT> __device__ __forceinline__ f32x4 widen4(typename Raw4<DT>::T w
 // Elements [off, off + 4) of a row of which the first n exist.  VEC (every row
 // starts on a whole chunk and ends with one): one vector load, the caller
 // keeps `off` inside the row.  Otherwise one by one, the rest zeros.
-template <int DT, bool VEC>
-__device__ __forceinline__ typename Raw4<DT>::T load4(const void *base, int64_t off, int n) {
+template <int DT, bool VEC, class Off>
+__device__ __forceinline__ typename Raw4<DT>::T load4(const void *base, Off off, int n) {
     using T = typename Raw4<DT>::T;
     if constexpr (VEC) {
-        if constexpr (DT == F32) return *gload_ptr<T>(reinterpret_cast<const float *>(base) + off);
-        else return *gload_ptr<T>(reinterpret_cast<const uint16_t *>(base) + off);
+        return *gload_ptr<T>(reinterpret_cast<const uint8_t *>(base) + off * ElemSize<DT>::value);
     }
     T w{};
     for (int e = 0; e < 4; ++e)
@@ -95,6 +95,7 @@ struct TileWork {
     int n;                       // its keys; relative to `lo` from here on:
     int rlo, rhi;                // keys the lane's row sees
     int wlo, whi;                // ... some row of the wave sees
+    int flo, fhi;                // ... every row of the wave sees
     int vlo, vhi;                // ... some row of the workgroup sees
 };
 
@@ -138,7 +139,7 @@ __device__ __forceinline__ TileWork tile_work(const TileArgs &a, int wg, int j, 
     const int64_t base_lo = full_diag ? 0 : pr->vis_lo, base_hi = full_diag ? keys : pr->vis_hi;
     const int64_t s_lo = base_lo + (int64_t)w.split * pr->split_keys;
     const int64_t s_hi = s_lo + pr->split_keys < base_hi ? s_lo + pr->split_keys : base_hi;
-    int64_t r_lo, r_hi, v_lo, v_hi, w_lo, w_hi, tmp;
+    int64_t r_lo, r_hi, v_lo, v_hi, w_lo, w_hi, f_lo, f_hi, tmp;
     visible_range(p, k_pos0, keys, q_pos0 + w.t_row, &r_lo, &r_hi);
     const int wg_first = rb * rw * 16, wg_last = min(wg_first + rw * 16, m_kv) - 1;
     visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wg_first / (uint32_t)G, &v_lo, &tmp);
@@ -146,8 +147,8 @@ __device__ __forceinline__ TileWork tile_work(const TileArgs &a, int wg, int j, 
     v_lo = v_lo > s_lo ? v_lo : s_lo;
     v_hi = v_hi < s_hi ? v_hi : s_hi;
     const int wv_first = min(row0, m_kv - 1), wv_last = min(row0 + 15, m_kv - 1);
-    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_first / (uint32_t)G, &w_lo, &tmp);
-    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_last / (uint32_t)G, &tmp, &w_hi);
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_first / (uint32_t)G, &w_lo, &f_hi);
+    visible_range(p, k_pos0, keys, q_pos0 + (uint32_t)wv_last / (uint32_t)G, &f_lo, &w_hi);
     const int64_t lo = full_diag ? s_lo : v_lo, hi = full_diag ? s_hi : v_hi;
     const int n = hi > lo ? (int)(hi - lo) : 0;
     auto rel = [&](int64_t x) { return (int)(x < lo ? 0 : (x > lo + n ? n : x - lo)); };
@@ -157,22 +158,34 @@ __device__ __forceinline__ TileWork tile_work(const TileArgs &a, int wg, int j, 
     w.rhi = w.rvalid ? rel(r_hi) : 0;
     w.wlo = rel(w_lo);
     w.whi = w.active ? rel(w_hi) : 0;
+    w.flo = rel(f_lo);
+    w.fhi = rel(f_hi);
     w.vlo = rel(v_lo);
     w.vhi = rel(v_hi);
     return w;
 }
 
-// The dots of a staged tile's blocks as masked scores in the exp2 domain, lane
-// row j against keys 16 b + 4 g + r (relative t0 on), with the diagnostics'
-// scores stored by the waves that have `store`.  Returns the lane's maximum.
+// A row's exponents: the softmax weight of a score is 2^(y * mul - m * mul), where
+// y is the raw dot product (mul = scale * log2 e) or, with a softcap, the capped
+// or stored score (mul = log2 e), and m the row's maximum y.  Formed by one fma,
+// the difference is rounded once however large the scores are.
+__device__ __forceinline__ bool scores_scaled(const Params &p) { return p.softcap != 0.0f || p.diag_mode != 0; }
+__device__ __forceinline__ float exp_mul(const Params &p) { return scores_scaled(p) ? LOG2E : p.scale * LOG2E; }
+
+// The dots of a staged tile's blocks as y values with masked keys at -inf: lane
+// row j against keys 16 b + 4 g + r (relative, t0 on).  Stores the diagnostics'
+// scores in the waves that have `store`.  Blocks that every row of the
+// wave sees need no comparison (a row past the last has the last row's dots, which
+// nothing stores).  Returns the lane's maximum; amax
+// collects the largest |y|, NaN included.
 template <int NB>
 __device__ __forceinline__ float finish_scores(const Params &p, const TileWork &w, const_ptr<Problem> pr, int t0, int g,
-                                               bool store, const bool (&scored)[NB], f32x4 (&st)[NB], bool &bad) {
+                                               bool store, const bool (&scored)[NB], f32x4 (&st)[NB], float &amax) {
     const float scale = p.scale, cap = p.softcap;
-    const bool full_diag = p.diag_mode == 1;
+    const bool full_diag = p.diag_mode == 1, scaled = scores_scaled(p);
     const bool last_row = w.h_row == p.query_heads - 1 && w.t_row == pr->queries - 1;
     const bool diag = p.diag_mode != 0 && store && w.rvalid && (full_diag || last_row);
-    float *const xs = p.scores ? p.scores : p.probs;  // raw scores (attn_tile_probs turns them into probabilities)
+    float *const xs = p.scores ? p.scores : p.probs;  // raw scores (attn_tile_merge turns them into probabilities)
     float tmax = NEG_INF;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -180,18 +193,13 @@ __device__ __forceinline__ float finish_scores(const Params &p, const TileWork &
             st[b] = f32x4{NEG_INF, NEG_INF, NEG_INF, NEG_INF};
             continue;
         }
-        f32x4 x;
-        for (int r = 0; r < 4; ++r) x[r] = st[b][r] * scale;
+        if (scaled)
+            for (int r = 0; r < 4; ++r) st[b][r] *= scale;
         if (cap != 0.0f)
-            for (int r = 0; r < 4; ++r) x[r] = softcap_f(x[r], cap);
-        const int key = t0 + 16 * b + 4 * g;
-        for (int r = 0; r < 4; ++r) {
-            const bool vis = key + r >= w.rlo && key + r < w.rhi;
-            bad |= vis && !is_finite_f(x[r]);
-            st[b][r] = vis ? x[r] * LOG2E : NEG_INF;
-            tmax = fmaxf(tmax, st[b][r]);
-        }
+            for (int r = 0; r < 4; ++r) st[b][r] = softcap_f(st[b][r], cap);
+        const int k0 = t0 + 16 * b, key = k0 + 4 * g;
         if (diag) {
+            const f32x4 x = st[b];
             const int first = full_diag ? 0 : w.rlo, end = full_diag ? w.n : w.rhi;
             float *xr = xs + (full_diag ? ((int64_t)w.h_row * pr->queries + w.t_row) * pr->keys : 0) + w.lo + key;
             if (key >= first && key + 4 <= end) *reinterpret_cast<f32x4u *>(xr) = x;
@@ -199,6 +207,16 @@ __device__ __forceinline__ float finish_scores(const Params &p, const TileWork &
                 for (int r = 0; r < 4; ++r)
                     if (key + r >= first && key + r < end) xr[r] = x[r];
         }
+        if (k0 >= w.flo && k0 + 16 <= w.fhi) {
+            for (int r = 0; r < 4; ++r) amax = __builtin_elementwise_maximum(amax, __builtin_fabsf(st[b][r]));
+        } else {
+            for (int r = 0; r < 4; ++r) {
+                const bool vis = key + r >= w.rlo && key + r < w.rhi;
+                amax = __builtin_elementwise_maximum(amax, vis ? __builtin_fabsf(st[b][r]) : 0.0f);
+                st[b][r] = vis ? st[b][r] : NEG_INF;
+            }
+        }
+        for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, st[b][r]);
     }
     return tmax;
 }
@@ -360,8 +378,9 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     f32x4 acc[FB][4];
     for (int fb = 0; fb < FB; ++fb)
         for (int e = 0; e < 4; ++e) acc[fb][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = NEG_INF, l_run = 0.0f;
-    bool bad = false;
+    // m_run: the row's maximum y, m_exp = m_run * mul (0 before the first).
+    const float mul = exp_mul(p);
+    float m_run = NEG_INF, m_exp = 0.0f, l_run = 0.0f, amax = 0.0f;
 
     if (n > 0) fetch(0);
     for (int t0 = 0; t0 < n; t0 += KT) {
@@ -405,13 +424,14 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
                     for (int r = 0; r < 4; ++r) st[b][r] += d[w * NB * 64][r];
             }
         }
-        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, bad);
+        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, amax);
         // The tile's maximum over the row's four lanes; O and l move with it.
         tmax = row4_max(tmax);
         const float m_new = fmaxf(m_run, tmax);
-        const float base = m_new == NEG_INF ? 0.0f : m_new;
         if (__ballot(m_new > m_run) != 0) {
-            const float corr = __builtin_amdgcn_exp2f(m_run - base);
+            const float moved = m_new == NEG_INF ? 0.0f : m_new * mul;
+            const float corr = m_run == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m_exp - moved);
+            m_exp = moved;
             l_run *= corr;
             for (int fb = 0; fb < FB; ++fb)
                 for (int e = 0; e < 4; ++e)
@@ -422,7 +442,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
         for (int b = 0; b < NB; ++b) {
             if (!seen[b]) continue;
             for (int r = 0; r < 4; ++r) {
-                const float e = __builtin_amdgcn_exp2f(st[b][r] - base);
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(st[b][r], mul, -m_exp));
                 st[b][r] = e;
                 l_run += e;
             }
@@ -438,7 +458,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     }
 
     l_run = row4_sum(l_run);
-    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
+    bool bad = !(amax < -NEG_INF);
+    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run == NEG_INF ? NEG_INF : m_exp, l_run);
     if (rvalid)
         for (int fb = 0; fb < FB; ++fb)
             for (int r = 0; r < 4; ++r)
@@ -572,18 +593,13 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     const int last = D - 4;
     auto feature = [&](int d) { return VEC ? min(d, last) : d; };
     const Raw none{};
-    u32x4 q[QS][SP];
+    Raw qlo[QS], qhi[QS];
     {
         const int64_t at = (int64_t)w.t_row * pr->q_row_stride + (int64_t)w.h_row * D;
-        Raw lo[QS], hi[QS];
         for (int s = 0; s < QS; ++s) {
             const int d = f0 + 32 * s + 8 * g;
-            lo[s] = load4<DT, VEC>(pr->q, at + feature(d), D - d);
-            hi[s] = load4<DT, VEC>(pr->q, at + feature(d + 4), D - d - 4);
-        }
-        for (int s = 0; s < QS; ++s) {
-            const int d = f0 + 32 * s + 8 * g;
-            planes8<DT>(!VEC || d <= last ? lo[s] : none, !VEC || d + 4 <= last ? hi[s] : none, q[s]);
+            qlo[s] = load4<DT, VEC>(pr->q, at + feature(d), D - d);
+            qhi[s] = load4<DT, VEC>(pr->q, at + feature(d + 4), D - d - 4);
         }
     }
 
@@ -591,12 +607,13 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     // m: key quad i % 8 of its 32-key group, features 4 (i / 8 % (DP / 4)).
     constexpr int CPR = DP / 8, FPR = DP / 4;
     Raw kreg[NK][2], vreg[NV][4];
-    auto fetch_rows = [&](int t0, auto at) {
+    // at(row) -> (K, V) addresses of the tile's row, whose elements follow.
+    auto fetch_rows = [&](auto at) {
 #pragma unroll
         for (int m = 0; m < NK; ++m) {
             const int i = tid + 256 * m, d = 8 * (i % CPR);
             const void *kb, *vb;
-            const int64_t off = at(w.lo + min(t0 + i / CPR, n - 1), &kb, &vb);
+            const auto off = at(i / CPR, &kb, &vb);
             kreg[m][0] = load4<DT, VEC>(kb, off + feature(d), D - d);
             kreg[m][1] = load4<DT, VEC>(kb, off + feature(d + 4), D - d - 4);
         }
@@ -605,24 +622,41 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
             const int i = tid + 256 * m, d = 4 * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
             for (int r = 0; r < 4; ++r) {
                 const void *kb, *vb;
-                const int64_t off = at(w.lo + min(t0 + k0 + r, n - 1), &kb, &vb);
+                const auto off = at(k0 + r, &kb, &vb);
                 vreg[m][r] = load4<DT, VEC>(vb, off + feature(d), D - d);
             }
         }
     };
+    constexpr int ES = ElemSize<DT>::value;
     auto fetch = [&](int t0) {
-        if (nseg == 1) {
-            const void *kb = pr->seg[0].k, *vb = pr->seg[0].v;
-            const int64_t rs = pr->seg[0].row_stride, head = (int64_t)w.kvh * pr->seg[0].head_stride;
-            fetch_rows(t0, [&](int64_t key, const void **k, const void **v) {
-                *k = kb;
-                *v = vb;
-                return head + key * rs;
-            });
+        const int left = n - 1 - t0;  // rows past the last repeat it
+        if (VEC && nseg == 1) {
+            // A tile's rows span less than 2 GiB (launch_tile): a uniform base and
+            // 32-bit offsets.
+            const int64_t first = ((int64_t)w.kvh * pr->seg[0].head_stride + (w.lo + t0) * pr->seg[0].row_stride) * ES;
+            const uint8_t *kb = reinterpret_cast<const uint8_t *>(pr->seg[0].k) + first;
+            const uint8_t *vb = reinterpret_cast<const uint8_t *>(pr->seg[0].v) + first;
+            const uint32_t rs = (uint32_t)pr->seg[0].row_stride;
+            auto rows = [&](auto row_of) {
+                fetch_rows([&](int r, const void **k, const void **v) {
+                    *k = kb;
+                    *v = vb;
+                    return row_of(r) * rs;
+                });
+            };
+            if (left >= KT - 1) rows([](int r) { return (uint32_t)r; });
+            else rows([&](int r) { return (uint32_t)min(r, left); });
         } else {
-            fetch_rows(t0, [&](int64_t key, const void **k, const void **v) { return seg_select(pr, key, w.kvh, k, v); });
+            fetch_rows([&](int r, const void **k, const void **v) { return seg_select(pr, w.lo + t0 + min(r, left), w.kvh, k, v); });
         }
     };
+    // The first tile is on its way before Q is waited for.
+    if (n > 0) fetch(0);
+    u32x4 q[QS][SP];
+    for (int s = 0; s < QS; ++s) {
+        const int d = f0 + 32 * s + 8 * g;
+        planes8<DT>(!VEC || d <= last ? qlo[s] : none, !VEC || d + 4 <= last ? qhi[s] : none, q[s]);
+    }
     auto stage = [&](int t0) {
 #pragma unroll
         for (int m = 0; m < NK; ++m) {
@@ -665,10 +699,10 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
 
     f32x4 acc[FB];
     for (int fb = 0; fb < FB; ++fb) acc[fb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = NEG_INF, l_run = 0.0f;
-    bool bad = false;
+    // m_run: the row's maximum y, m_exp = m_run * mul (0 before the first).
+    const float mul = exp_mul(p);
+    float m_run = NEG_INF, m_exp = 0.0f, l_run = 0.0f, amax = 0.0f;
 
-    if (n > 0) fetch(0);
     for (int t0 = 0; t0 < n; t0 += KT) {
         __syncthreads();
         stage(t0);
@@ -715,12 +749,13 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
                     for (int r = 0; r < 4; ++r) st[b][r] += d[x * NB * 64][r];
             }
         }
-        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, bad);
+        float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, amax);
         tmax = row4_max(tmax);
         const float m_new = fmaxf(m_run, tmax);
-        const float base = m_new == NEG_INF ? 0.0f : m_new;
         if (__ballot(m_new > m_run) != 0) {
-            const float corr = __builtin_amdgcn_exp2f(m_run - base);
+            const float moved = m_new == NEG_INF ? 0.0f : m_new * mul;
+            const float corr = m_run == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m_exp - moved);
+            m_exp = moved;
             l_run *= corr;
             for (int fb = 0; fb < FB; ++fb)
                 for (int r = 0; r < 4; ++r) acc[fb][r] *= corr;
@@ -731,7 +766,7 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
             if (!seen[2 * t] && !seen[2 * t + 1]) continue;
             for (int b = 2 * t; b < 2 * t + 2; ++b)
                 for (int r = 0; r < 4; ++r) {
-                    st[b][r] = __builtin_amdgcn_exp2f(st[b][r] - base);
+                    st[b][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[b][r], mul, -m_exp));
                     l_run += st[b][r];
                 }
             u32x4 pb[PP];
@@ -760,19 +795,41 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     if constexpr (DT == F16)
         for (int fb = 0; fb < FB; ++fb)
             for (int r = 0; r < 4; ++r) acc[fb][r] *= 1.0f / PROB_SCALE_F16;
-    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
+    bool bad = !(amax < -NEG_INF);
+    TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run == NEG_INF ? NEG_INF : m_exp, l_run);
     if (w.rvalid)
         for (int fb = 0; fb < FB; ++fb) out.emit(f0 + 16 * fb + 4 * g, acc[fb], bad);
     out.report(p, bad);
 }
 
-// Merged (max, mass) of a row's S partials.
-__device__ __forceinline__ void merged_stats(const float *ml, int S, float &M, float &L) {
-    M = NEG_INF;
-    for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * s]);
-    L = 0.0f;
-    for (int s = 0; s < S; ++s)
-        if (ml[2 * s] != NEG_INF) L += __builtin_amdgcn_exp2f(ml[2 * s] - M) * ml[2 * s + 1];
+// The probabilities of one diagnostics row by one wave, from the scores the
+// attention kernel stored (in the probability buffer itself when the caller asked
+// for no scores): masked keys are exactly +0.  The row's partials are merged by the
+// lanes (at most 64 of them).
+__device__ __forceinline__ void probs_row(const TileArgs &a, int64_t row_index) {
+    const Params &p = a.p;
+    const Problem &pr = p.single;  // diagnostics are single-problem calls
+    const int G = p.group, Hq = p.query_heads, lane = threadIdx.x & 63;
+    const bool full = p.diag_mode == 1;
+    const int64_t hr = full ? row_index : (int64_t)Hq * pr.queries - 1;
+    const int h = (int)(hr / pr.queries), t = (int)(hr % pr.queries);
+    const int m_kv = pr.queries * G, S = pr.splits * a.kw;
+    const int64_t local = (int64_t)(h / G) * m_kv + (int64_t)t * G + h % G;
+    const float *ml = p.part_ml + 2 * (pr.slot_base + local * S);
+    f32x2 mine = {NEG_INF, 0.0f};
+    if (lane < S) mine = *gload_ptr<f32x2>(ml + 2 * lane);
+    int64_t lo, hi;
+    visible_range(p, pr, pr.q_pos0 + t, &lo, &hi);
+    const int64_t row = full ? hr * pr.keys : 0, end = full ? pr.keys : hi;
+    const float *xs = (p.scores ? p.scores : p.probs) + row;
+    const float M = wave_max(mine[0]);
+    const float L = wave_sum(mine[0] == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(mine[0] - M) * mine[1]);
+    const float inv = 1.0f / L;
+#pragma unroll 4
+    for (int64_t key = (full ? 0 : lo) + lane; key < end; key += 64) {
+        const float x = xs[key];
+        p.probs[row + key] = key >= lo && key < hi ? __builtin_amdgcn_exp2f(__builtin_fmaf(x, LOG2E, -M)) * inv : 0.0f;
+    }
 }
 
 __device__ __forceinline__ int find_row_problem(const Params &p, int64_t row) {
@@ -784,11 +841,19 @@ __device__ __forceinline__ int find_row_problem(const Params &p, int64_t row) {
     return lo;
 }
 
-// Split-K combine: one thread per four features of a row, so a launch has
-// rows x D / 4 threads and a thread's partials (16 splits at a time) are all
-// in flight together; the time is one memory round trip.
-__global__ __launch_bounds__(256) void attn_tile_merge(TileArgs a, int64_t total_rows, int dp) {
+// Split-K combine, in the first merge_blocks workgroups: one thread per four
+// features of a row, so a launch has rows x D / 4 threads and a thread's partials
+// (16 splits at a time) are all in flight together; the time is one memory round
+// trip.  The workgroups after those make the diagnostics' probabilities, a wave per
+// row: 300 tokens of 16/8/128 took 5 us and, as a launch of its own whose threads
+// each went through a row's partials one by one, 11 us; together they take 9.6.
+__global__ __launch_bounds__(256) void attn_tile_merge(TileArgs a, int64_t total_rows, int dp, uint32_t merge_blocks) {
     const Params &p = a.p;
+    if (blockIdx.x >= merge_blocks) {
+        const int64_t r = (int64_t)(blockIdx.x - merge_blocks) * 4 + (threadIdx.x >> 6);
+        if (r < (p.diag_mode == 1 ? (int64_t)p.query_heads * p.single.queries : 1)) probs_row(a, r);
+        return;
+    }
     const int D = p.head_dim, Hq = p.query_heads, G = p.group;
     const uint32_t per = (uint32_t)(D + 3) / 4;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -845,31 +910,6 @@ __global__ __launch_bounds__(256) void attn_tile_merge(TileArgs a, int64_t total
     raise_status(p, bad_out, ST_NONFINITE_OUTPUT);
 }
 
-// The probabilities of one diagnostics row per workgroup, from the scores
-// attn_tile stored (in the probability buffer itself when the caller asked for
-// no scores): masked keys are exactly +0.
-__global__ __launch_bounds__(256) void attn_tile_probs(TileArgs a) {
-    const Params &p = a.p;
-    const Problem &pr = p.single;  // diagnostics are single-problem calls
-    const int G = p.group, Hq = p.query_heads;
-    const bool full = p.diag_mode == 1;
-    const int64_t hr = full ? (int64_t)blockIdx.x : (int64_t)Hq * pr.queries - 1;
-    const int h = (int)(hr / pr.queries), t = (int)(hr % pr.queries);
-    const int m_kv = pr.queries * G, S = pr.splits * a.kw;
-    const int64_t local = (int64_t)(h / G) * m_kv + (int64_t)t * G + h % G;
-    float M, L;
-    merged_stats(p.part_ml + 2 * (pr.slot_base + local * S), S, M, L);
-    const float inv = 1.0f / L;
-    int64_t lo, hi;
-    visible_range(p, pr, pr.q_pos0 + t, &lo, &hi);
-    const int64_t row = full ? hr * pr.keys : 0, end = full ? pr.keys : hi;
-    const float *xs = (p.scores ? p.scores : p.probs) + row;
-    for (int64_t key = (full ? 0 : lo) + threadIdx.x; key < end; key += 256) {
-        const float x = xs[key];
-        p.probs[row + key] = key >= lo && key < hi ? __builtin_amdgcn_exp2f(x * LOG2E - M) * inv : 0.0f;
-    }
-}
-
 }  // namespace tkh
 
 // Head sizes the kernels are built for (the smallest that holds `head_dim`).
@@ -916,19 +956,15 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
     return hipErrorInvalidValue;
 }
 
+// The combine of `total_rows` rows (0: the keys were not split) and the
+// probabilities, when the call asks for them.
 extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
                                             hipEvent_t start, hipEvent_t stop) {
     using namespace tkh;
-    const int64_t threads = total_rows * ((a->p.head_dim + 3) / 4);
-    dim3 grid((unsigned)((threads + 255) / 256)), block(256);
+    const int64_t merge = (total_rows * ((a->p.head_dim + 3) / 4) + 255) / 256;
+    const int64_t rows = !a->p.probs ? 0 : (a->p.diag_mode == 1 ? (int64_t)a->p.query_heads * a->p.single.queries : 1);
+    dim3 grid((unsigned)(merge + (rows + 3) / 4)), block(256);
     hipExtLaunchKernelGGL(attn_tile_merge, grid, block, 0, stream, start, stop, 0, *a, total_rows,
-                          tkh_tile_head(a->p.head_dim));
-    return hipGetLastError();
-}
-
-extern "C" hipError_t tkh_launch_tile_probs(const tkh::TileArgs *a, hipStream_t stream) {
-    using namespace tkh;
-    const int64_t rows = a->p.diag_mode == 1 ? (int64_t)a->p.query_heads * a->p.single.queries : 1;
-    hipLaunchKernelGGL(attn_tile_probs, dim3((unsigned)rows), dim3(256), 0, stream, *a);
+                          tkh_tile_head(a->p.head_dim), (uint32_t)merge);
     return hipGetLastError();
 }
