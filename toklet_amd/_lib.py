@@ -106,6 +106,7 @@ class LayerIo(ctypes.Structure):
 P = ctypes.POINTER
 E = P(Error)
 
+# Device pointers are all void pointers here: a tensor's data_ptr() passes as it is.
 SIGNATURES = {
     "tkh_abi_version": (u32, []),
     "tkh_context_create": (u32, [ctypes.c_int, vp, ctypes.c_size_t, ctypes.c_int, P(vp), E]),
@@ -115,22 +116,22 @@ SIGNATURES = {
     "tkh_context_profile": (u32, [vp, ctypes.c_int, E]),
     "tkh_context_profile_read": (u32, [vp, P(Profile), E]),
     "tkh_attention_cached": (u32, [vp, P(CachedShape), ctypes.c_int, vp, u64, vp, u64, vp, u64,
-                                   fptr, u64, fptr, u64, fptr, u64, E]),
+                                   vp, u64, vp, u64, vp, u64, E]),
     "tkh_attention_cached_static": (u32, [ctypes.c_int, vp, P(CachedShape), ctypes.c_int, vp, u64,
-                                          vp, u64, vp, u64, fptr, u64, P(u32), E]),
-    "tkh_attention": (u32, [vp, P(AttentionShape), ctypes.c_int, vp, u64, vp, u64, vp, u64, fptr,
-                            u64, fptr, u64, fptr, u64, E]),
+                                          vp, u64, vp, u64, vp, u64, vp, E]),
+    "tkh_attention": (u32, [vp, P(AttentionShape), ctypes.c_int, vp, u64, vp, u64, vp, u64, vp,
+                            u64, vp, u64, vp, u64, E]),
     "tkh_window_attention": (u32, [vp, P(WindowShape), ctypes.c_int, vp, u64, vp, u64, vp, u64,
-                                   fptr, u64, fptr, u64, fptr, u64, E]),
-    "tkh_span_attention": (u32, [vp, P(SpanShape), ctypes.c_int, vp, u64, P(Segment), fptr, u64,
-                                 fptr, u64, fptr, u64, E]),
-    "tkh_project_greedy": (u32, [vp, u64, u64, u64, fptr, u64, fptr, u64, fptr, u64, P(u32), u64,
+                                   vp, u64, vp, u64, vp, u64, E]),
+    "tkh_span_attention": (u32, [vp, P(SpanShape), ctypes.c_int, vp, u64, P(Segment), vp, u64,
+                                 vp, u64, vp, u64, E]),
+    "tkh_project_greedy": (u32, [vp, u64, u64, u64, vp, u64, vp, u64, vp, u64, vp, u64,
                                  E]),
-    "tkh_logit_softcap": (u32, [vp, fptr, u64, f32, E]),
+    "tkh_logit_softcap": (u32, [vp, vp, u64, f32, E]),
     "tkh_decode_batch": (u32, [vp, u64, u64, u64, u64, ctypes.c_int, vp, vp, vp, P(u64), P(u64),
-                               P(u64), f32, fptr, E]),
+                               P(u64), f32, vp, E]),
     "tkh_prefill_batch": (u32, [vp, u64, u64, u64, u64, u64, ctypes.c_int, vp, vp, vp, P(u64),
-                                P(u64), P(u64), f32, fptr, E]),
+                                P(u64), P(u64), f32, vp, E]),
     "tkh_kv_planned_bytes": (u32, [u64, u64, u64, u32, u64, ctypes.c_int, u64, P(u64), E]),
     "tkh_kv_create": (u32, [vp, u64, u64, u64, u64, u32, u64, ctypes.c_int, P(vp), E]),
     "tkh_kv_destroy": (None, [vp]),

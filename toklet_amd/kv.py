@@ -65,6 +65,7 @@ class _Owner:
                err)
         self.handle = handle
         self.storage = storage
+        self._flat = None
         _lib.track(self, _lib.KV_OWNER)
 
     def info(self) -> _lib.KvInfo:
@@ -78,6 +79,17 @@ class _Owner:
         shape = (i.heads, i.capacity, i.dims)
         return (device_tensor(i.k, shape, self.storage, self.ctx.device),
                 device_tensor(i.v, shape, self.storage, self.ctx.device))
+
+    def _storage(self):
+        """(k, v) flat views of the whole storage and its base addresses: fixed for the
+        owner's life, so they are made once (wrapping an address as a tensor costs
+        several launches' worth of host time)."""
+        if self._flat is None:
+            i = self.info()
+            n = (i.heads * i.capacity * i.dims,)
+            self._flat = (device_tensor(i.k, n, self.storage, self.ctx.device),
+                          device_tensor(i.v, n, self.storage, self.ctx.device), int(i.k), int(i.v))
+        return self._flat
 
     @property
     def offset(self) -> int:
@@ -93,6 +105,7 @@ class _Owner:
 
     def close(self):
         if getattr(self, "handle", None):
+            self._flat = None
             _lib.load().tkh_kv_destroy(self.handle)
             self.handle = None
 
@@ -200,15 +213,26 @@ class KvView:
     def segments(self) -> List[AttentionKvSegment]:
         segs, _ = self._raw(1, 1.0)
         out = []
-        dt = self.cache.storage
-        for s in segs:
+        k, v, k0, v0 = self.cache._storage()
+        es = k.element_size()
+        for i, s in enumerate(segs):
+            n = s.k_len
             if s.keys == 0:
                 out.append(AttentionKvSegment(None, None, 0, 0, int(s.key_start)))
-                continue
-            k = device_tensor(s.k, (s.k_len,), dt, self.cache.ctx.device)
-            v = device_tensor(s.v, (s.v_len,), dt, self.cache.ctx.device)
-            out.append(AttentionKvSegment(k, v, int(s.keys), int(s.head_stride), int(s.key_start)))
+            elif i == 2:  # the staged rows
+                out.append(AttentionKvSegment(self._staged(self.prepared.k, s.k, n), self._staged(self.prepared.v, s.v, n),
+                                              int(s.keys), int(s.head_stride), int(s.key_start)))
+            else:
+                kb, vb = (s.k - k0) // es, (s.v - v0) // es
+                out.append(AttentionKvSegment(k[kb:kb + n], v[vb:vb + n], int(s.keys), int(s.head_stride),
+                                              int(s.key_start)))
         return out
+
+    def _staged(self, rows: torch.Tensor, ptr: int, n: int) -> torch.Tensor:
+        """The caller's staged rows as the flat tensor the frame describes."""
+        if rows.dtype is self.cache.storage and rows.is_contiguous() and rows.data_ptr() == ptr and rows.numel() == n:
+            return rows.view(-1)
+        return device_tensor(ptr, (n,), self.cache.storage, self.cache.ctx.device)
 
     def attention_shape(self, query_heads: int, scale: float) -> SpanAttentionShape:
         _, s = self._raw(query_heads, scale)

@@ -156,30 +156,35 @@ class SpanAttentionShape:
     softcap: float = 0.0
 
 
+# A call through these bindings costs about as much as a launch, so the argument
+# helpers avoid building ctypes objects: addresses go as plain integers.
 def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p()
+    return None if t is None else t.data_ptr()
 
 
 def _fptr(t: Optional[torch.Tensor]):
     if t is None:
-        return ctypes.cast(None, _lib.fptr)
-    if t.dtype != torch.float32:
+        return None
+    if t.dtype is not torch.float32:
         raise TypeError("outputs are float32 tensors")
-    return ctypes.cast(t.data_ptr(), _lib.fptr)
+    return t.data_ptr()
 
 
 def _n(t: Optional[torch.Tensor]) -> int:
-    return t.numel() if t is not None else 0
+    return 0 if t is None else t.numel()
 
 
 def dtype_of(*tensors: torch.Tensor) -> int:
-    dts = {t.dtype for t in tensors if t is not None}
-    if len(dts) != 1:
-        raise TypeError(f"q/k/v must share one dtype, got {dts}")
-    (dt,) = dts
-    if dt not in _DTYPES:
+    dt = None
+    for t in tensors:
+        if t is not None and t.dtype is not dt:
+            if dt is not None:
+                raise TypeError(f"q/k/v must share one dtype, got {({x.dtype for x in tensors if x is not None})}")
+            dt = t.dtype
+    code = _DTYPES.get(dt)
+    if code is None:
         raise TypeError(f"unsupported dtype {dt}")
-    return _DTYPES[dt]
+    return code
 
 
 def _window(window):
@@ -211,7 +216,7 @@ def attention_cached_static(device: int, q, k, v, context, shape: CachedAttentio
                          shape.capacity, shape.offset)
     if stream is None:
         stream = torch.cuda.current_stream(device)
-    st = ctypes.cast(status.data_ptr(), ctypes.POINTER(ctypes.c_uint32)) if status is not None else None
+    st = _ptr(status)
     rc = _lib.load().tkh_attention_cached_static(
         device, ctypes.c_void_p(stream.cuda_stream), ctypes.byref(s), dtype_of(q, k, v), _ptr(q),
         _n(q), _ptr(k), _n(k), _ptr(v), _n(v), _fptr(context), _n(context), st, ctypes.byref(err))
@@ -251,7 +256,7 @@ def span_attention(ctx: Context, q, segments: Sequence[AttentionKvSegment], cont
     segs = (_lib.Segment * 3)()
     tensors = [q] + [t for sg in segments for t in (sg.k, sg.v) if t is not None]
     for i, sg in enumerate(segments):
-        segs[i] = _lib.Segment(_ptr(sg.k).value, _n(sg.k), _ptr(sg.v).value, _n(sg.v), sg.keys,
+        segs[i] = _lib.Segment(_ptr(sg.k), _n(sg.k), _ptr(sg.v), _n(sg.v), sg.keys,
                                sg.head_stride, sg.key_start)
     hw, w = _window(shape.window)
     s = _lib.SpanShape(shape.queries, shape.keys, shape.query_heads, shape.kv_heads,
@@ -275,10 +280,9 @@ def project_greedy(ctx: Context, context: torch.Tensor, weights: torch.Tensor,
     vocab = weights.shape[0]
     if tokens.dtype != torch.int32:
         raise TypeError("tokens is an int32 tensor (uint32 ids)")
-    tok = ctypes.cast(tokens.data_ptr(), ctypes.POINTER(ctypes.c_uint32))
     rc = _lib.load().tkh_project_greedy(
         ctx.handle, rows, hidden, vocab, _fptr(context), _n(context), _fptr(weights), _n(weights),
-        _fptr(logits), _n(logits), tok, _n(tokens), ctypes.byref(err))
+        _fptr(logits), _n(logits), _ptr(tokens), _n(tokens), ctypes.byref(err))
     _check(rc, err)
 
 
