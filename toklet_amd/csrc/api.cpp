@@ -719,8 +719,7 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     }
     tkh::TileArgs args{};
     int64_t max_rows = 0, max_span = 0, rows = 0;
-    bool vec = D % 4 == 0;
-    const uintptr_t chunk = 4 * (uintptr_t)esize(plan.dtype);
+    int vec = D % 8 == 0 ? 8 : (D % 4 == 0 ? 4 : 1);
     for (auto &p : group) {
         visible_union(plan, p);
         max_rows = std::max<int64_t>(max_rows, p.queries * G);
@@ -731,9 +730,10 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
         for (int i = 0; i < p.nseg; ++i) {
             at |= (uintptr_t)p.seg[i].k | (uintptr_t)p.seg[i].v;
             strides |= p.seg[i].head_stride | p.seg[i].row_stride;
-            vec = vec && p.seg[i].row_stride < INT32_MAX / 4 / 64;  // a tile's offsets in 32 bits
+            if (p.seg[i].row_stride >= INT32_MAX / 4 / 64) vec = 1;  // a tile's offsets in 32 bits
         }
-        vec = vec && at % chunk == 0 && strides % 4 == 0;
+        while (vec > 1 && (at % (vec * (uintptr_t)std::min(esize(plan.dtype), 16 / vec)) != 0 || strides % vec != 0))
+            vec = vec == 8 ? 4 : 1;
     }
     // Row groups per workgroup, then key splits, each at least a staged tile
     // long, for at most tile_groups workgroups in all: two fit on a CU, and a few
@@ -786,7 +786,7 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     prm.diag_mode = plan.diag_mode;
     args.rw = rw;
     args.kw = kw;
-    args.vec = vec ? 1 : 0;
+    args.vec = vec;
 
     const bool split = splits * kw > 1, second = split || plan.probs;
     hipEvent_t *ev = nullptr;

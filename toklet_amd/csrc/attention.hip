@@ -563,7 +563,8 @@ __device__ __forceinline__ void prob_planes(const f32x4 &a, const f32x4 &b, u32x
 
 }  // namespace
 
-template <int DT, int DP, bool VEC>
+// VE: elements that start and end every row in whole vectors (1: element loads).
+template <int DT, int DP, int VE>
 __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
     constexpr int KT = split_keys(DP), NB = KT / 16, NG = KT / 32, FS = split_feature_waves(DP);
@@ -571,7 +572,13 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     constexpr int SP = Planes<DT>::store, PP = Planes<DT>::prob;
     constexpr int KROW = DP * 2 + 16, VROW = KT * 2;          // staged row bytes: K per key, V per feature
     constexpr int KPL = KT * KROW, VPL = DP * VROW;           // bytes per plane
-    constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / 16 / 256;  // a thread's 8-feature K chunks, 4 x 4 V blocks
+    constexpr bool VEC = VE > 1;
+    // A thread's K chunks of eight features and V blocks of four keys by VF
+    // features; with whole 16-byte vectors of 16-bit elements a wide tile's
+    // blocks take eight: half the load instructions (300 tokens of 16/8/128 with
+    // diagnostics 39.7 -> 37.1 us a call, 128 queries of 8/1/512 59.7 -> 57.1).
+    constexpr int VF = VE == 8 && DP >= 256 ? 8 : 4;
+    constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / (4 * VF) / 256;
     static_assert(NK >= 1 && NV >= 1, "staging covers the tile");
     __shared__ __attribute__((aligned(16))) uint8_t kt[SP * KPL];
     __shared__ __attribute__((aligned(16))) uint8_t vt[SP * VPL];
@@ -590,23 +597,31 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     auto v_at = [](int f, int c) { return f * VROW + ((c ^ (KT == 32 ? f >> 2 & 3 : f >> 1 & 7)) << 4); };
 
     // Features past the head are zeros in Q, K and V (attn_tile's loads).
-    const int last = D - 4;
-    auto feature = [&](int d) { return VEC ? min(d, last) : d; };
     const Raw none{};
-    Raw qlo[QS], qhi[QS];
+    auto whole = [&](int d, int width) { return VE == 1 || d + width <= D; };
+    auto load_four = [&](const void *base, auto off, int d) {
+        return load4<DT, VEC>(base, off + (VEC ? min(d, D - 4) : d), D - d);
+    };
+    auto load_eight = [&](const void *base, auto off, int d, Raw (&to)[2]) {
+        if constexpr (VE == 8) {
+            const u32x4 x = *gload_ptr<u32x4>(reinterpret_cast<const uint8_t *>(base) + (off + min(d, D - 8)) * 2);
+            to[0] = Raw{x[0], x[1]};
+            to[1] = Raw{x[2], x[3]};
+        } else {
+            to[0] = load_four(base, off, d);
+            to[1] = load_four(base, off, d + 4);
+        }
+    };
+    Raw qraw[QS][2];
     {
         const int64_t at = (int64_t)w.t_row * pr->q_row_stride + (int64_t)w.h_row * D;
-        for (int s = 0; s < QS; ++s) {
-            const int d = f0 + 32 * s + 8 * g;
-            qlo[s] = load4<DT, VEC>(pr->q, at + feature(d), D - d);
-            qhi[s] = load4<DT, VEC>(pr->q, at + feature(d + 4), D - d - 4);
-        }
+        for (int s = 0; s < QS; ++s) load_eight(pr->q, at, f0 + 32 * s + 8 * g, qraw[s]);
     }
 
     // K chunk m of a thread: row i / (DP / 8), features 8 (i % (DP / 8)).  V block
-    // m: key quad i % 8 of its 32-key group, features 4 (i / 8 % (DP / 4)).
-    constexpr int CPR = DP / 8, FPR = DP / 4;
-    Raw kreg[NK][2], vreg[NV][4];
+    // m: key quad i % 8 of its 32-key group, features VF (i / 8 % (DP / VF)).
+    constexpr int CPR = DP / 8, FPR = DP / VF;
+    Raw kreg[NK][2], vreg[NV][4][VF / 4];
     // at(row) -> (K, V) addresses of the tile's row, whose elements follow.
     auto fetch_rows = [&](auto at) {
 #pragma unroll
@@ -614,16 +629,16 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
             const int i = tid + 256 * m, d = 8 * (i % CPR);
             const void *kb, *vb;
             const auto off = at(i / CPR, &kb, &vb);
-            kreg[m][0] = load4<DT, VEC>(kb, off + feature(d), D - d);
-            kreg[m][1] = load4<DT, VEC>(kb, off + feature(d + 4), D - d - 4);
+            load_eight(kb, off, d, kreg[m]);
         }
 #pragma unroll
         for (int m = 0; m < NV; ++m) {
-            const int i = tid + 256 * m, d = 4 * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
+            const int i = tid + 256 * m, d = VF * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
             for (int r = 0; r < 4; ++r) {
                 const void *kb, *vb;
                 const auto off = at(k0 + r, &kb, &vb);
-                vreg[m][r] = load4<DT, VEC>(vb, off + feature(d), D - d);
+                if constexpr (VF == 8) load_eight(vb, off, d, vreg[m][r]);
+                else vreg[m][r][0] = load_four(vb, off, d);
             }
         }
     };
@@ -655,43 +670,46 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     u32x4 q[QS][SP];
     for (int s = 0; s < QS; ++s) {
         const int d = f0 + 32 * s + 8 * g;
-        planes8<DT>(!VEC || d <= last ? qlo[s] : none, !VEC || d + 4 <= last ? qhi[s] : none, q[s]);
+        planes8<DT>(whole(d, 4) ? qraw[s][0] : none, whole(d + 4, 4) ? qraw[s][1] : none, q[s]);
     }
     auto stage = [&](int t0) {
 #pragma unroll
         for (int m = 0; m < NK; ++m) {
             const int i = tid + 256 * m, d = 8 * (i % CPR);
             u32x4 pl[SP];
-            planes8<DT>(!VEC || d <= last ? kreg[m][0] : none, !VEC || d + 4 <= last ? kreg[m][1] : none, pl);
+            planes8<DT>(whole(d, 4) ? kreg[m][0] : none, whole(d + 4, 4) ? kreg[m][1] : none, pl);
             for (int s = 0; s < SP; ++s) *reinterpret_cast<u32x4 *>(kt + s * KPL + i / CPR * KROW + 2 * d) = pl[s];
         }
 #pragma unroll
         for (int m = 0; m < NV; ++m) {
-            const int i = tid + 256 * m, qd = i % 8, d = 4 * (i / 8 % FPR), t = i / (8 * FPR);
+            const int i = tid + 256 * m, qd = i % 8, d0 = VF * (i / 8 % FPR), t = i / (8 * FPR);
             const int k0 = t0 + 32 * t + 4 * qd;
-            Raw x[4];
-            for (int r = 0; r < 4; ++r)
-                x[r] = (!VEC || d <= last) && k0 + r >= w.vlo && k0 + r < w.vhi ? vreg[m][r] : none;
-            // Row f holds the group's keys as 8-byte pieces: g = qd % 4 first, then b = qd / 4.
-            auto to = [&](int e) { return vt + v_at(d + e, 4 * t + (qd & 3)) + 8 * (qd >> 2); };
-            if constexpr (DT == F32) {
-                f32x4 y[4];
-                for (int r = 0; r < 4; ++r) y[r] = widen4<DT>(x[r]);
-                for (int e = 0; e < 4; ++e) {
-                    float v[4] = {y[0][e], y[1][e], y[2][e], y[3][e]};
-                    for (int s = 0; s < 3; ++s) {
-                        using Quad = typename Raw4<F16>::T;
-                        const Quad o = s == 0 ? Quad{plane2<true>(v[0], v[1]), plane2<true>(v[2], v[3])}
-                                              : Quad{plane2<false>(v[0], v[1]), plane2<false>(v[2], v[3])};
-                        *reinterpret_cast<Quad *>(to(e) + s * VPL) = o;
+            for (int half = 0; half < VF / 4; ++half) {
+                const int d = d0 + 4 * half;
+                Raw x[4];
+                for (int r = 0; r < 4; ++r)
+                    x[r] = whole(d, 4) && k0 + r >= w.vlo && k0 + r < w.vhi ? vreg[m][r][half] : none;
+                // Row f holds the group's keys as 8-byte pieces: g = qd % 4 first, then b = qd / 4.
+                auto to = [&](int e) { return vt + v_at(d + e, 4 * t + (qd & 3)) + 8 * (qd >> 2); };
+                if constexpr (DT == F32) {
+                    f32x4 y[4];
+                    for (int r = 0; r < 4; ++r) y[r] = widen4<DT>(x[r]);
+                    for (int e = 0; e < 4; ++e) {
+                        float v[4] = {y[0][e], y[1][e], y[2][e], y[3][e]};
+                        for (int s = 0; s < 3; ++s) {
+                            using Quad = typename Raw4<F16>::T;
+                            const Quad o = s == 0 ? Quad{plane2<true>(v[0], v[1]), plane2<true>(v[2], v[3])}
+                                                  : Quad{plane2<false>(v[0], v[1]), plane2<false>(v[2], v[3])};
+                            *reinterpret_cast<Quad *>(to(e) + s * VPL) = o;
+                        }
                     }
-                }
-            } else {
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t pick = e & 1 ? 0x07060302u : 0x05040100u;
-                    const uint32_t o0 = __builtin_amdgcn_perm(x[1][e >> 1], x[0][e >> 1], pick);
-                    const uint32_t o1 = __builtin_amdgcn_perm(x[3][e >> 1], x[2][e >> 1], pick);
-                    *reinterpret_cast<Raw *>(to(e)) = Raw{o0, o1};
+                } else {
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t pick = e & 1 ? 0x07060302u : 0x05040100u;
+                        const uint32_t o0 = __builtin_amdgcn_perm(x[1][e >> 1], x[0][e >> 1], pick);
+                        const uint32_t o1 = __builtin_amdgcn_perm(x[3][e >> 1], x[2][e >> 1], pick);
+                        *reinterpret_cast<Raw *>(to(e)) = Raw{o0, o1};
+                    }
                 }
             }
         }
@@ -942,17 +960,26 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
     using namespace tkh;
     const int dp = tkh_tile_head(a->p.head_dim);
     dim3 grid((unsigned)a->p.total_tiles), block(256);
-#define TKH_TILE(KERNEL, DT, DP)                                                                        \
-    if (dtype == DT && dp == DP) {                                                                      \
-        if (a->vec) hipExtLaunchKernelGGL((KERNEL<DT, DP, true>), grid, block, 0, stream, start, stop, 0, *a); \
-        else hipExtLaunchKernelGGL((KERNEL<DT, DP, false>), grid, block, 0, stream, start, stop, 0, *a);       \
-        return hipGetLastError();                                                                       \
+#define TKH_LAUNCH(...) hipExtLaunchKernelGGL((__VA_ARGS__), grid, block, 0, stream, start, stop, 0, *a)
+#define TKH_TILE(DP)                                                                    \
+    if (dtype == F32 && dp == DP) {                                                     \
+        if (a->vec >= 4) TKH_LAUNCH(attn_tile<F32, DP, true>);                          \
+        else TKH_LAUNCH(attn_tile<F32, DP, false>);                                     \
+        return hipGetLastError();                                                       \
     }
-    TKH_TILE(attn_split, F32, 64) TKH_TILE(attn_split, F32, 128) TKH_TILE(attn_tile, F32, 256) TKH_TILE(attn_tile, F32, 512)
-    TKH_TILE(attn_split, F16, 64) TKH_TILE(attn_split, F16, 128) TKH_TILE(attn_split, F16, 256) TKH_TILE(attn_split, F16, 512)
-    TKH_TILE(attn_split, BF16, 64) TKH_TILE(attn_split, BF16, 128) TKH_TILE(attn_split, BF16, 256)
-    TKH_TILE(attn_split, BF16, 512)
+#define TKH_SPLIT(DT, DP)                                                               \
+    if (dtype == DT && dp == DP) {                                                      \
+        if (DT != F32 && a->vec >= 8) TKH_LAUNCH(attn_split<DT, DP, DT != F32 ? 8 : 4>); \
+        else if (a->vec >= 4) TKH_LAUNCH(attn_split<DT, DP, 4>);                        \
+        else TKH_LAUNCH(attn_split<DT, DP, 1>);                                         \
+        return hipGetLastError();                                                       \
+    }
+    TKH_SPLIT(F32, 64) TKH_SPLIT(F32, 128) TKH_TILE(256) TKH_TILE(512)
+    TKH_SPLIT(F16, 64) TKH_SPLIT(F16, 128) TKH_SPLIT(F16, 256) TKH_SPLIT(F16, 512)
+    TKH_SPLIT(BF16, 64) TKH_SPLIT(BF16, 128) TKH_SPLIT(BF16, 256) TKH_SPLIT(BF16, 512)
+#undef TKH_SPLIT
 #undef TKH_TILE
+#undef TKH_LAUNCH
     return hipErrorInvalidValue;
 }
 

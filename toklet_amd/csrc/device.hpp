@@ -290,7 +290,7 @@ struct TileArgs {
     Params p;             // first: the single-problem path reads it at the kernel-argument base
     int32_t rw;           // 16-row groups per workgroup (1, 2 or 4)
     int32_t kw;           // waves sharing a row group's keys, each with a partial of its own
-    int32_t vec;          // every row starts on a whole 4-element chunk: vector loads
+    int32_t vec;          // elements whose whole vectors make up every row (8, 4, or 1: no vector loads)
 };
 static_assert(sizeof(PrefillArgs) <= 4096, "kernel arguments");
 static_assert(sizeof(DecodeArgs) <= 4096, "kernel arguments");
