@@ -1090,6 +1090,37 @@ uint32_t tkh_host::add_chunk_producer(tkh_context *ctx, ChunkBatchOfLayers *batc
     return TKH_OK;
 }
 
+// Puts the layers whose workgroups take the most keys first: workgroups start in
+// order, and a long one that starts last runs on a card that has emptied (figures
+// at pf_locate).
+static void longest_first(tkh::PrefillLayersArgs &a, int64_t wgs, int64_t merge_blocks) {
+    struct Part {
+        int layer;
+        int64_t keys, wgs, merge_blocks;
+    } part[tkh::DECODE_LAYERS_MAX];
+    for (int i = 0; i < a.count; ++i) {
+        const tkh::Problem &p = a.e[i].pr;
+        const bool last = i + 1 == a.count;
+        part[i] = {i, std::min<int64_t>(p.split_keys, p.vis_hi - p.vis_lo), (last ? wgs : a.first[i + 1]) - a.first[i],
+                   (last ? merge_blocks : a.merge_first[i + 1]) - a.merge_first[i]};
+    }
+    auto longer = [](const Part &x, const Part &y) { return x.keys != y.keys ? x.keys > y.keys : x.layer < y.layer; };
+    if (std::is_sorted(part, part + a.count, longer)) return;
+    std::sort(part, part + a.count, longer);
+    tkh::PrefillLayer given[tkh::DECODE_LAYERS_MAX];
+    std::copy(a.e, a.e + a.count, given);
+    int64_t first = 0, merge = 0;
+    for (int i = 0; i < a.count; ++i) {
+        a.e[i] = given[part[i].layer];
+        a.e[i].pr.tile_base = first;
+        a.e[i].pr.part_base = merge;
+        a.first[i] = (int32_t)first;
+        a.merge_first[i] = (int32_t)merge;
+        first += part[i].wgs;
+        merge += part[i].merge_blocks;
+    }
+}
+
 // The batched layers' producers, then the attention calls that joined, then the
 // merge of those that are split: three launches.
 uint32_t tkh_host::flush_chunk_layers(tkh_context *ctx, ChunkBatchOfLayers *batch, tkh_error *err) {
@@ -1123,6 +1154,7 @@ uint32_t tkh_host::flush_chunk_layers(tkh_context *ctx, ChunkBatchOfLayers *batc
     hipEvent_t *ev = nullptr;
     if (ctx->profiling) TRY(profile_slot(ctx, &ev, merge_blocks > 0, err));
     a.count = layers;
+    longest_first(a, wgs, merge_blocks);
     hipError_t e = tkh_launch_prefill_layers(&a, batch->dtype, D, wgs, ctx->stream, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
     if (e == hipSuccess && merge_blocks > 0)
         e = tkh_launch_prefill_merge_layers(&a, D, merge_blocks, ctx->stream, ev ? ev[2] : nullptr, ev ? ev[3] : nullptr);

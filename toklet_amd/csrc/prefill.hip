@@ -340,12 +340,30 @@ template <bool LAYERS> using prefill_args = std::conditional_t<LAYERS, PrefillLa
 template <int D, bool LAYERS>
 __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, int &split, int &kvh, int &sidx) {
     // XCD-major tile order: dispatch slot b runs on XCD b % 8; give each XCD
-    // a contiguous range of logical tiles.
+    // a contiguous range of logical tiles.  With several layers, a contiguous
+    // range of every layer's own: over the launch as a whole the layers of the
+    // longest splits would fall to one or two XCDs, and the others wait for them
+    // (128 tokens of six 8/4/256 layers at 2,048 keys, five of window 1,024: 51.8
+    // us, 44.2 with each layer over every XCD and the longest layers first).
     int64_t tile;
+    int layer = 0;
     {
-        const uint32_t nb = gridDim.x;
+        uint32_t b = blockIdx.x, nb = gridDim.x;
+        if constexpr (LAYERS) {
+            const_ptr<PrefillLayersArgs> la = (const_ptr<PrefillLayersArgs>)__builtin_amdgcn_kernarg_segment_ptr();
+            uint32_t base = 0, end = nb;
+            for (int i = DECODE_LAYERS_MAX - 1; i > 0; --i) {
+                const uint32_t first = i < la->count ? (uint32_t)la->first[i] : nb;
+                const bool in = b >= first;  // the last layer that starts at or before b
+                layer = in && base == 0 ? i : layer;
+                base = in && base == 0 ? first : base;
+                end = in ? end : first;
+            }
+            b -= base;
+            nb = end - base;
+        }
         const uint32_t per = (nb + 7) / 8;
-        const uint32_t x = blockIdx.x % 8, k = blockIdx.x / 8;
+        const uint32_t x = b % 8, k = b / 8;
         const uint32_t full = nb % 8 == 0 ? 8 : nb % 8;  // XCDs that receive `per` blocks
         tile = (int64_t)(x < full ? x * per + k : full * per + (x - full) * (per - 1) + k);
     }
@@ -389,9 +407,6 @@ __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, 
             const_ptr<Problem> pr;
             if constexpr (LAYERS) {
                 const_ptr<PrefillLayersArgs> la = (const_ptr<PrefillLayersArgs>)args;
-                int layer = 0;
-                for (int i = 1; i < DECODE_LAYERS_MAX; ++i)
-                    layer = i < la->count && (int)tile >= la->first[i] ? i : layer;
                 const_ptr<PrefillLayer> e = &la->e[uniform32(layer)];
                 pr = &e->pr;
                 pv.has_window = e->has_window;
@@ -413,7 +428,7 @@ __device__ __forceinline__ void pf_locate(const Params &p, PfView &pv, int &rb, 
             pv.row_blocks = pr->row_blocks;
             pv.splits = pr->splits;
             pv.split_keys = pr->split_keys;
-            uint32_t local = (uint32_t)(tile - pv.tile_base);
+            uint32_t local = (uint32_t)(LAYERS ? tile : tile - pv.tile_base);
             const uint32_t nrb = (uint32_t)pv.row_blocks, ns = (uint32_t)pv.splits;
             rb = (int)(local % nrb);
             local /= nrb;
