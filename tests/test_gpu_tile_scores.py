@@ -94,3 +94,19 @@ def test_scales_at_the_ends(torch_mod, orc, D, diag):
         worst = np.max(np.abs(got[0] - ref[0]) - 1e-4 * np.abs(ref[0]))
         log(f"D={D} diag {diag} scale {scale:.3g}: worst excess {worst:.2e}")
         assert np.all(np.isfinite(got[0])) and worst <= 1e-5
+
+
+@pytest.mark.parametrize("diag", [False, True])
+@pytest.mark.parametrize("dt,D", [("f32", 64), ("f32", 256), ("bf16", 96)])
+def test_scores_past_the_largest_are_refused(torch_mod, orc, dt, D, diag):
+    """Finite operands whose scaled score is not: refused whichever sign it has, also
+    where a larger finite score would leave it no weight."""
+    from toklet_amd import ops
+
+    q = np.ones((QUERIES, HQ, D), np.float32)
+    for sign in (-1.0, 1.0):
+        k = np.zeros((HKV, 40, D), np.float32)
+        k[:, 7] = sign * 1e9
+        with pytest.raises(ops.TkhError) as e:
+            _run(torch_mod, orc, q, stored(k, dt), np.ones_like(k), dt, 1e30, diag=diag, check=False)
+        assert e.value.name == "NonFinite"

@@ -187,7 +187,7 @@ __device__ __forceinline__ float finite_max(float m) { return m == NEG_INF ? 0.0
 // scores in the waves that have `store`.  Blocks that every row of the
 // wave sees need no comparison (a row past the last has the last row's dots, which
 // nothing stores).  Returns the lane's maximum; amax
-// collects the largest |y|, NaN included.
+// collects the largest |y|, NaN included (finite_scores).
 template <int NB>
 __device__ __forceinline__ float finish_scores(const Params &p, const TileWork &w, const_ptr<Problem> pr, int t0, int g,
                                                bool store, const bool (&scored)[NB], f32x4 (&st)[NB], float &amax) {
@@ -229,6 +229,12 @@ __device__ __forceinline__ float finish_scores(const Params &p, const TileWork &
         for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, st[b][r]);
     }
     return tmax;
+}
+
+// Whether every score a lane saw is finite: the scaled one, also where y is the raw
+// dot (rounding keeps the order, so the largest tells).
+__device__ __forceinline__ bool finite_scores(const Params &p, float amax) {
+    return is_finite_f(scores_scaled(p) ? amax : amax * p.scale);
 }
 
 // Where a lane's row of unnormalised context goes: divided by its mass into the
@@ -466,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     }
 
     l_run = row4_sum(l_run);
-    bool bad = !(amax < -NEG_INF);
+    bool bad = !finite_scores(p, amax);
     TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
     if (rvalid)
         for (int fb = 0; fb < FB; ++fb)
@@ -819,7 +825,7 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     if constexpr (DT == F16)
         for (int fb = 0; fb < FB; ++fb)
             for (int r = 0; r < 4; ++r) acc[fb][r] *= 1.0f / PROB_SCALE_F16;
-    bool bad = !(amax < -NEG_INF);
+    bool bad = !finite_scores(p, amax);
     TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
     if (w.rvalid)
         for (int fb = 0; fb < FB; ++fb) out.emit(f0 + 16 * fb + 4 * g, acc[fb], bad);
