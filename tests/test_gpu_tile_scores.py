@@ -1,7 +1,8 @@
 """The FP32-exact attention kernels (attention.hip) over the range of finite
 scores: rows whose maximum is far from zero, held by several keys in different
 tiles and splits, so that the context is the mean of those keys' V exactly
-whatever rounds below them; and scales at the ends of FP32."""
+whatever rounds below them; light keys beside a heavy one that has nothing to add;
+and scales at the ends of FP32."""
 
 import numpy as np
 import pytest
@@ -75,6 +76,32 @@ def test_row_maximum_weighs_one(torch_mod, orc, dt, D, keys, diag):
                 # An FP32 dot of D products (and the softcap's tanh): D ulps at most.
                 assert np.all(np.abs(got[1] - ref[1]) <= D * 2.0 ** -23 * np.abs(ref[1]))
                 assert np.max(np.abs(got[2] - ref[2])) <= 1e-5
+
+
+@pytest.mark.parametrize("diag", [False, True])
+@pytest.mark.parametrize("D", [64, 96, 256, 512])
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+def test_light_keys_keep_their_bits(torch_mod, orc, dt, D, diag):
+    """A heavy key whose V is zero, and keys e^-25 and e^-60 as heavy: their sum is
+    all of the context, so a weight that lost bits or fell to zero shows at full
+    size.  Weights are 2^t with t rounded to FP32 (at most 87, half an ulp 2^-18)
+    and V, P and sums as FP32 keeps them: within 1e-5 of the result."""
+    if not _exact_kernels(dt, D, diag):
+        pytest.skip("another kernel's call")
+    rng = np.random.default_rng(D)
+    keys = 70
+    for nats in (25.0, 60.0):
+        v = np.zeros((HKV, keys, D), np.float32)
+        k = np.zeros((HKV, keys, D), np.float32)
+        k[:, 1:, 0] = -4.0
+        v[:, 1:] = rng.uniform(100.0, 400.0, (HKV, keys - 1, D))
+        q = np.zeros((QUERIES, HQ, D), np.float32)
+        q[:, :, 0] = nats / 4.0
+        q, k, v = (stored(x, dt) for x in (q, k, v))
+        got, ref = _run(torch_mod, orc, q, k, v, dt, 1.0, diag=diag)
+        worst = np.max(np.abs(got[0] / ref[0].astype(np.float64) - 1.0))
+        log(f"{dt} D={D} diag {diag} {nats} nats: relative error {worst:.2e}")
+        assert worst <= 1e-5
 
 
 @pytest.mark.parametrize("diag", [False, True])

@@ -27,6 +27,7 @@ extern "C" int tkh_tile_head(int head_dim);
 extern "C" int tkh_tile_keys(int dtype, int head_dim);
 extern "C" int tkh_tile_row_waves(int dtype, int head_dim);
 extern "C" int tkh_tile_share(int dtype, int head_dim);
+extern "C" int tkh_tile_resident(int dtype, int head_dim);
 extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStream_t stream,
                                       hipEvent_t start, hipEvent_t stop);
 extern "C" hipError_t tkh_launch_tile_merge(const tkh::TileArgs *a, int64_t total_rows, hipStream_t stream,
@@ -743,7 +744,7 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     const int rw = std::min(waves, max_rows <= 16 ? 1 : (max_rows <= 32 ? 2 : 4));
     int64_t base = 0;
     for (auto &p : group) base += Hkv * (((int64_t)p.queries * G + 16 * rw - 1) / (16 * rw));
-    int64_t splits = std::max<int64_t>(1, ctx->tile_groups / base);
+    int64_t splits = std::max<int64_t>(1, ctx->tile_groups * tkh_tile_resident((int)plan.dtype, (int)D) / 2 / base);
     splits = std::min<int64_t>(splits, std::max<int64_t>(1, max_span / KT));
     int kw = max_span > KT ? std::min(waves / rw, tkh_tile_share((int)plan.dtype, (int)D)) : 1;
     splits = std::min<int64_t>(splits, 64 / kw);

@@ -486,13 +486,20 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 // sixteen times the FP32 rate), with FP32 operands split into 16-bit planes whose
 // products lose nothing FP32 arithmetic keeps.
 //
-//  * bf16 and f16 storage: Q, K and V are planes as they are.  A probability is
-//    split into three bf16 planes (each the rounding of what the last left, so
-//    their sum is the FP32 value), or two f16 ones of 2^11 P (22 bits; the factor
-//    keeps small probabilities' second plane in f16's range).
-//  * F32 storage: Q, K, V and P are three bf16 planes each, and a product of two
-//    values is the six plane products down to 2^-16 (the three left out are below
-//    2^-24, FP32's own rounding).
+//  * Probabilities are three bf16 planes, each the rounding of what the last left:
+//    their sum is the FP32 value, over all of FP32's normal range.
+//  * bf16 storage: Q, K and V are planes as they are.
+//  * f16 storage: Q and K are, on the f16 form of the MFMA; V's 11 bits are two bf16
+//    planes, exactly, and the product left out is below 2^-26 of the whole.  (Two
+//    f16 planes of 2^11 P, two MFMAs where these take five, kept 22 bits of a weight
+//    of 1 and none of one of 2^-36: 69 keys e^-25 as heavy as one whose V is zero
+//    summed to 23% of their context.  They took 23.2 us for 128 queries over 2048
+//    keys at 12/4/96, 24.2 for 300 tokens of 16/8/128 with diagnostics and 40.5 for
+//    128 queries over 1025 keys at 8/1/512; these 26.1, 25.7 and 44.0.)
+//  * F32 storage: Q, K and V are three bf16 planes each, and a product of two
+//    values is the six plane products down to 2^-18 of it; the three left out are
+//    below 2^-25 of it together, half of FP32's own rounding.  Planes hold an
+//    element below 2^-110 to 2^-133, bf16's smallest number.
 //
 // Lane (j, g) holds query row j.  Q.K: A = K plane (key j of a 16-key block,
 // features 32 s + 8 g .. + 7), B = Q.  P.V over 32 keys: the MFMA's k index
@@ -507,10 +514,11 @@ __host__ __device__ constexpr int split_feature_waves(int DP) { return DP <= 256
 
 namespace {
 
-template <int DT> struct Planes { static constexpr int store = 1, prob = 3; };
-template <> struct Planes<F32> { static constexpr int store = 3, prob = 3; };
-template <> struct Planes<F16> { static constexpr int store = 1, prob = 2; };
-constexpr float PROB_SCALE_F16 = 0x1p11f;
+// Planes of Q and K, of V, and of a probability.
+constexpr int PROB_PLANES = 3;
+template <int DT> struct Planes { static constexpr int qk = 1, v = 1; };
+template <> struct Planes<F32> { static constexpr int qk = 3, v = 3; };
+template <> struct Planes<F16> { static constexpr int qk = 1, v = 2; };
 
 template <int DT> __device__ __forceinline__ f32x4 mfma32k(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (DT == F16)
@@ -534,7 +542,7 @@ template <bool LIMIT> __device__ __forceinline__ uint32_t plane2(float &a, float
 
 // Eight stored elements as planes of an MFMA operand.
 template <int DT>
-__device__ __forceinline__ void planes8(typename Raw4<DT>::T lo, typename Raw4<DT>::T hi, u32x4 (&out)[Planes<DT>::store]) {
+__device__ __forceinline__ void planes8(typename Raw4<DT>::T lo, typename Raw4<DT>::T hi, u32x4 (&out)[Planes<DT>::qk]) {
     if constexpr (DT == F32) {
         const f32x4 x = widen4<DT>(lo), y = widen4<DT>(hi);
         float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
@@ -549,30 +557,10 @@ __device__ __forceinline__ void planes8(typename Raw4<DT>::T lo, typename Raw4<D
 }
 
 // A lane's probabilities of 32 keys (two score blocks) as planes.
-template <int DT>
-__device__ __forceinline__ void prob_planes(const f32x4 &a, const f32x4 &b, u32x4 (&out)[Planes<DT>::prob]) {
-    f32x4 x = a, y = b;
-    if constexpr (DT == F16) {
-        auto half2 = [](float u, float v) {
-            const f16x2 h = {(_Float16)u, (_Float16)v};
-            return __builtin_bit_cast(uint32_t, h);
-        };
-        for (int e = 0; e < 4; ++e) {
-            x[e] *= PROB_SCALE_F16;
-            y[e] *= PROB_SCALE_F16;
-        }
-        for (int pl = 0; pl < 2; ++pl) {
-            out[pl] = u32x4{half2(x[0], x[1]), half2(x[2], x[3]), half2(y[0], y[1]), half2(y[2], y[3])};
-            for (int e = 0; e < 4; ++e) {
-                x[e] -= (float)(_Float16)x[e];
-                y[e] -= (float)(_Float16)y[e];
-            }
-        }
-    } else {
-        float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-        for (int pl = 0; pl < 3; ++pl)
-            for (int e = 0; e < 4; ++e) out[pl][e] = plane2<false>(v[2 * e], v[2 * e + 1]);
-    }
+__device__ __forceinline__ void prob_planes(const f32x4 &x, const f32x4 &y, u32x4 (&out)[PROB_PLANES]) {
+    float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    for (int pl = 0; pl < PROB_PLANES; ++pl)
+        for (int e = 0; e < 4; ++e) out[pl][e] = plane2<false>(v[2 * e], v[2 * e + 1]);
 }
 
 }  // namespace
@@ -583,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
     constexpr int KT = split_keys(DP), NB = KT / 16, NG = KT / 32, FS = split_feature_waves(DP);
     constexpr int DW = DP / FS, QS = DW / 32, FB = DW / 16;   // a wave's features, Q.K steps, P.V blocks
-    constexpr int SP = Planes<DT>::store, PP = Planes<DT>::prob;
+    constexpr int SP = Planes<DT>::qk, VP = Planes<DT>::v;
     constexpr int KROW = DP * 2 + 16, VROW = KT * 2;          // staged row bytes: K per key, V per feature
     constexpr int KPL = KT * KROW, VPL = DP * VROW;           // bytes per plane
     constexpr bool VEC = VE > 1;
@@ -595,7 +583,7 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / (4 * VF) / 256;
     static_assert(NK >= 1 && NV >= 1, "staging covers the tile");
     __shared__ __attribute__((aligned(16))) uint8_t kt[SP * KPL];
-    __shared__ __attribute__((aligned(16))) uint8_t vt[SP * VPL];
+    __shared__ __attribute__((aligned(16))) uint8_t vt[VP * VPL];
     __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? 4 * NB * 64 : 1];  // partial scores
     using Raw = typename Raw4<DT>::T;
     const Params &p = a.p;
@@ -705,12 +693,12 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
                     x[r] = whole(d, 4) && k0 + r >= w.vlo && k0 + r < w.vhi ? vreg[m][r][half] : none;
                 // Row f holds the group's keys as 8-byte pieces: g = qd % 4 first, then b = qd / 4.
                 auto to = [&](int e) { return vt + v_at(d + e, 4 * t + (qd & 3)) + 8 * (qd >> 2); };
-                if constexpr (DT == F32) {
+                if constexpr (VP > 1) {
                     f32x4 y[4];
                     for (int r = 0; r < 4; ++r) y[r] = widen4<DT>(x[r]);
                     for (int e = 0; e < 4; ++e) {
                         float v[4] = {y[0][e], y[1][e], y[2][e], y[3][e]};
-                        for (int s = 0; s < 3; ++s) {
+                        for (int s = 0; s < VP; ++s) {
                             using Quad = typename Raw4<F16>::T;
                             const Quad o = s == 0 ? Quad{plane2<true>(v[0], v[1]), plane2<true>(v[2], v[3])}
                                                   : Quad{plane2<false>(v[0], v[1]), plane2<false>(v[2], v[3])};
@@ -799,32 +787,32 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
                     st[b][r] = weight(st[b][r], m_ref, mul);
                     l_run += st[b][r];
                 }
-            u32x4 pb[PP];
-            prob_planes<DT>(st[2 * t], st[2 * t + 1], pb);
+            u32x4 pb[PROB_PLANES];
+            prob_planes(st[2 * t], st[2 * t + 1], pb);
             const uint8_t *vr = vt + v_at(f0 + j, 4 * t + g);  // the swizzle repeats every 16 rows
 #pragma unroll
             for (int fb = 0; fb < FB; ++fb) {
-                u32x4 v[SP];
-                for (int pl = 0; pl < SP; ++pl) v[pl] = *reinterpret_cast<const u32x4 *>(vr + pl * VPL + 16 * fb * VROW);
-                f32x4 o = acc[fb];
-                if constexpr (SP == 3) {
-                    o = mfma32k<DT>(v[2], pb[0], o);
-                    o = mfma32k<DT>(v[0], pb[2], o);
-                    o = mfma32k<DT>(v[1], pb[1], o);
-                    o = mfma32k<DT>(v[1], pb[0], o);
-                    o = mfma32k<DT>(v[0], pb[1], o);
-                } else {
-                    for (int pl = PP - 1; pl > 0; --pl) o = mfma32k<DT>(v[0], pb[pl], o);
+                u32x4 v[VP];
+                for (int pl = 0; pl < VP; ++pl) v[pl] = *reinterpret_cast<const u32x4 *>(vr + pl * VPL + 16 * fb * VROW);
+                // The smallest products first.  With V in planes their sum is added to
+                // the context once (rounded once, not once a product).
+                f32x4 o = VP > 1 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : acc[fb];
+                if constexpr (VP == 3) o = mfma32k<BF16>(v[2], pb[0], o);
+                o = mfma32k<BF16>(v[0], pb[2], o);
+                if constexpr (VP > 1) {
+                    o = mfma32k<BF16>(v[1], pb[1], o);
+                    o = mfma32k<BF16>(v[1], pb[0], o);
                 }
-                acc[fb] = mfma32k<DT>(v[0], pb[0], o);
+                o = mfma32k<BF16>(v[0], pb[1], o);
+                o = mfma32k<BF16>(v[0], pb[0], o);
+                if constexpr (VP > 1)
+                    for (int r = 0; r < 4; ++r) acc[fb][r] += o[r];
+                else acc[fb] = o;
             }
         }
     }
 
     l_run = row4_sum(l_run);
-    if constexpr (DT == F16)
-        for (int fb = 0; fb < FB; ++fb)
-            for (int r = 0; r < 4; ++r) acc[fb][r] *= 1.0f / PROB_SCALE_F16;
     bool bad = !finite_scores(p, amax);
     TileOut out(a, w, pr, DP, g == 0 && fs == 0, m_run, l_run);
     if (w.rvalid)
@@ -961,6 +949,9 @@ extern "C" int tkh_tile_row_waves(int dtype, int head_dim) {
     const int dp = tkh_tile_head(head_dim);
     return 4 / (tile_splits(dtype, head_dim) ? tkh::split_feature_waves(dp) : tkh::tile_feature_waves(dp));
 }
+// Workgroups a CU holds: the 105 KiB of 512-wide f16 tiles leave room for one (128
+// queries over 1025 keys at 8/1/512, kernels alone: 53.9 us split for two, 44.0 for one).
+extern "C" int tkh_tile_resident(int dtype, int head_dim) { return dtype == tkh::F16 && tkh_tile_head(head_dim) == 512 ? 1 : 2; }
 extern "C" int tkh_tile_share(int dtype, int head_dim) {
     return tile_splits(dtype, head_dim) ? 1 : tkh_tile_keys(dtype, head_dim) / 16;
 }
