@@ -453,17 +453,17 @@ uint32_t launch_decode(tkh_context *ctx, const Plan &plan, Problems group,
     if (group.size() == 1) prm.single = group[0];
     prm.nproblems = (int32_t)group.size();
     prm.total_tiles = wgs;
-    if (split && ++ctx->epoch == 0) {
-        // The epoch wrapped: clear every flag so no stale one can match again.
+    if (split && ++ctx->epoch > tkh::DECODE_EPOCHS) {
+        // Counted from 1 again: clear every flag so no stale one can match again.
         HIP_TRY(tkh_launch_zero_u64(reinterpret_cast<uint64_t *>(decode_region(ctx)),
                                     (int64_t)(decode_region_bytes(ctx) / sizeof(uint64_t)), ctx->stream),
                 "decode workspace clear");
         ctx->epoch = 1;
     }
-    prm.epoch = ctx->epoch;
+    prm.epoch = tkh::decode_flag(ctx->epoch);
     // The merging split waits for this launch's epoch; the test hook makes it
     // wait for one that no split stores, to exercise the bounded wait.
-    prm.wait_epoch = ctx->epoch + (ctx->test_flag_skew ? 1u : 0u);
+    prm.wait_epoch = prm.epoch + (ctx->test_flag_skew ? 1u : 0u);
     prm.split_wait_ticks = ctx->split_wait_ticks;
     // Much work streams at the HBM limit, where nontemporal loads raise the
     // rate (configs[2] 200 -> 184 us, 16 sessions at 8192 keys 96 -> 86 us);
@@ -1025,9 +1025,9 @@ uint64_t first_visible(uint64_t key_start, uint64_t position, bool has_window, u
 
 }  // namespace
 
-// The batched layers' launch, and the merge of those that are split.  The flags
-// of the decode region's layout are not used: the merge launch orders the
-// partials, which take the region from its start.
+// The batched layers' launch, and the merge of those that are split.  The merge
+// launch orders the partials, so there are no flags and the partials take the
+// decode region from its start (what they leave cannot pass for a flag: decode_flag).
 uint32_t tkh_host::flush_decode_layers(tkh_context *ctx, DecodeBatchOfLayers *batch, tkh_error *err) {
     tkh::DecodeLayersArgs &a = batch->args;
     if (a.count == 0) return TKH_OK;
@@ -1168,6 +1168,10 @@ extern "C" {
 
 uint32_t tkh_abi_version(void) { return TKH_ABI_VERSION; }
 
+// The flag values, for the test of what they cannot be taken for.
+uint32_t tkh_decode_flag(uint32_t epoch) { return tkh::decode_flag(epoch); }
+uint32_t tkh_decode_epochs(void) { return tkh::DECODE_EPOCHS; }
+
 uint32_t tkh_context_create(int device, void *stream, size_t workspace_bytes, int synchronous,
                             tkh_context **out, tkh_error *err) {
     if (!out) return invalid("context output", err);
@@ -1198,7 +1202,7 @@ uint32_t tkh_context_create(int device, void *stream, size_t workspace_bytes, in
         return cleanup(e, "status");
     if ((e = hipMalloc(&ctx->workspace, ctx->workspace_bytes)) != hipSuccess)
         return cleanup(e, "workspace");
-    // Decode tags start at 0, which no launch epoch equals.
+    // Decode flags start at 0, which no launch's flag equals.
     if ((e = hipMemset(decode_region(ctx), 0, decode_region_bytes(ctx))) != hipSuccess)
         return cleanup(e, "workspace");
     ctx->batch_store = new (std::nothrow) tkh::Problem[kSlotProblems];
@@ -1353,7 +1357,7 @@ StaticDevice g_static[kStaticMaxDevices];
 
 // Once per device, with that device current: the array's address, the
 // planner settings, and a cleared array (status 0; decode flags 0, which no
-// launch epoch equals).
+// launch's flag equals).
 uint32_t static_device(int device, hipStream_t stream, StaticDevice **out, tkh_error *err) {
     if (device < 0 || device >= kStaticMaxDevices) return invalid("device ordinal", err);
     StaticDevice &sd = g_static[device];

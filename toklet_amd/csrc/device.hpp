@@ -124,6 +124,14 @@ struct FusedDecode {
     int64_t new_row;       // cache row its K/V go to (new_key for a linear cache, 0 for a ring's stage)
 };
 
+// A split's completion flag for the launches counted 1 .. DECODE_EPOCHS.  The words
+// that hold a launch's flags may have held another's partials (a launch with fewer
+// slots, or one whose merge needs no flags), so a flag is a signalling NaN, which no
+// arithmetic leaves behind: a small whole number could be a stale denormal float,
+// and its split would be merged before it is written.
+constexpr uint32_t DECODE_EPOCHS = 0x3ffffe;
+__host__ __device__ constexpr uint32_t decode_flag(uint32_t epoch) { return 0xff800000u + epoch; }
+
 struct Params {
     const Problem *problems;
     int32_t nproblems;
@@ -150,7 +158,7 @@ struct Params {
     int32_t diag_mode;      // 0 none, 1 full [Hq, queries, keys], 2 last row [keys]
     int32_t stream_nt;      // decode: K/V stream read with nontemporal loads (1) or plain (0)
     uint32_t *flags;        // decode split-K completion flags, one per partial slot
-    uint32_t epoch;         // decode split-K: this launch's flag value (never 0; flags start at 0)
+    uint32_t epoch;         // decode split-K: this launch's flag value (decode_flag; flags start at 0)
     uint32_t wait_epoch;    // the flag value the merging split waits for (= epoch)
     uint64_t split_wait_ticks;  // bound of that wait, s_memrealtime ticks
     int32_t merge_launch;   // decode split-K: every split stores its partial; attn_decode_merge combines

@@ -145,7 +145,7 @@ struct tkh_context {
     int decode_disable = 0;
     bool decode_merge_launch = true;  // single-problem, latency-bound decode: combine in a second launch
     bool decode_merge_batch = false;  // compact-batch decode: combine in a second launch
-    uint32_t epoch = 0;          // last decode split-K epoch handed out
+    uint32_t epoch = 0;          // last decode split-K epoch handed out (1 .. DECODE_EPOCHS)
     uint64_t split_wait_ticks = 50000000;  // bound of a decode merge's wait for its splits
     bool test_flag_skew = false; // test hook: merges wait for a flag value no split stores
     int prefill_groups = 128;    // below this many row-block workgroups (128-row units), split the keys
@@ -169,9 +169,9 @@ struct tkh_context {
     double prof_attention_ms = 0, prof_combine_ms = 0;
 };
 
-// The workspace halves: split-K partials of the prefill and generic kernels
-// in the lower half, the decode kernel's tagged partials in the upper half
-// (kept apart so no other kernel's bits can pass for a decode tag).
+// The workspace halves: split-K partials of the prefill and FP32-exact kernels in
+// the lower half, the decode kernel's flags and partials in the upper half (cleared
+// at creation, so a word is 0, a flag or an FP32 partial there: decode_flag).
 inline size_t split_region_bytes(const tkh_context *ctx) { return ctx->workspace_bytes / 2; }
 inline size_t decode_region_offset(const tkh_context *ctx) {
     return (ctx->workspace_bytes / 2 + 255) / 256 * 256;
