@@ -122,3 +122,27 @@ def test_tile_over_ring_spans(torch_mod, orc, dt, D, W):
         ring.commit(frame)
         pos += n
     ctx.close()
+
+
+@pytest.mark.parametrize("hq,hkv,D,queries,keys,dt", [
+    (3, 1, 80, 1, 100, "bf16"),   # 9 partials: their pairs end inside a 16-byte vector
+    (3, 1, 512, 3, 170, "f32"),
+])
+def test_odd_partial_counts(torch_mod, orc, hq, hkv, D, queries, keys, dt):
+    """Odd numbers of rows and splits: the merge's vectors behind the (max, mass)
+    pairs."""
+    from toklet_amd import ops
+
+    torch = torch_mod
+    rng = np.random.default_rng(keys)
+    q = stored(rng.standard_normal((queries, hq, D)), dt)
+    k, v = (stored(rng.standard_normal((hkv, keys, D)), dt) for _ in range(2))
+    ref, _, _ = orc.window_attention(q, k.reshape(-1), v.reshape(-1), queries, keys, keys, hq, hkv, D, keys - queries, 0,
+                                     None, D ** -0.5)
+    ctx = ops.Context(0)
+    out = torch.full((queries * hq * D,), np.nan, dtype=torch.float32, device="cuda")
+    ops.window_attention(ctx, dev(q, dt), dev(k, dt), dev(v, dt), out, None, None,
+                         ops.WindowAttentionShape(queries, keys, keys, hq, hkv, D, keys - queries, 0, None, D ** -0.5))
+    log(f"{hq}/{hkv}/{D} {dt} {queries} x {keys}")
+    _close(host(out), ref, "context")
+    ctx.close()

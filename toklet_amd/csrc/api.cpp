@@ -748,8 +748,11 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     splits = std::min<int64_t>(splits, std::max<int64_t>(1, max_span / KT));
     int kw = max_span > KT ? std::min(waves / rw, tkh_tile_share((int)plan.dtype, (int)D)) : 1;
     splits = std::min<int64_t>(splits, 64 / kw);
+    // The (max, mass) pairs of s partials a row, in whole 16-byte vectors: the merge
+    // reads the contexts behind them four features at a time.
+    auto ml_floats = [&](int64_t s) { return ((size_t)rows * s * 2 + 3) / 4 * 4; };
     auto fits = [&](int64_t s) {
-        return s == 1 || (size_t)rows * s * (DP + 2) * sizeof(float) <= split_region_bytes(ctx);
+        return s == 1 || (ml_floats(s) + (size_t)rows * s * DP) * sizeof(float) <= split_region_bytes(ctx);
     };
     while (!fits(splits * kw)) {
         if (splits > 1) splits = (splits + 1) / 2;
@@ -781,7 +784,7 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
     prm.nproblems = (int32_t)group.size();
     prm.total_tiles = tiles;
     prm.part_ml = reinterpret_cast<float *>(ctx->workspace);
-    prm.part_o = prm.part_ml + 2 * (size_t)rows * splits * kw;
+    prm.part_o = prm.part_ml + ml_floats(splits * kw);
     prm.scores = plan.scores;
     prm.probs = plan.probs;
     prm.diag_mode = plan.diag_mode;
