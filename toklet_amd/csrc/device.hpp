@@ -589,6 +589,15 @@ __device__ __forceinline__ void visible_range(const Params &p, const Problem &pr
     visible_range(p, pr.k_pos0, pr.keys, pos, lo, hi);
 }
 
+// Orders the LDS accesses of one wave's lanes: what a lane stored before, any lane
+// of the wave reads after.  The hardware keeps a wave's LDS accesses in order, so
+// this only keeps the compiler from moving them and costs no instruction.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ void raise_status(uint32_t *status, bool bad, uint32_t bit) {
     if (__builtin_amdgcn_read_exec() != 0) {
         uint64_t m = __ballot(bad);

@@ -96,7 +96,7 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
     constexpr int RG = K <= 1 ? 2 : (K == 2 ? 4 : (K == 4 ? 2 : 1));
     constexpr int KP = (K + 1) / 2;               // rotary pairs per lane
     constexpr int WAVES = TABLE ? 4 : 8;
-    __shared__ float rowbuf[WAVES][64 * K];
+    __shared__ float rowbuf[WAVES][RG][64 * K];
     __shared__ f32x2 rot[TABLE ? 1 : 64 * KP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int D = p->d, hq = p->hq, half = D / 2;
@@ -105,7 +105,7 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
     const int64_t position = p->position + t;
     const int end = first + rows < hq + 2 * hkv ? first + rows : hq + 2 * hkv;
 
-    float x[RG][K], wq[K], wk[K];
+    float x[RG][K] = {}, wq[K], wk[K];
     f32x2 cs[KP];
     auto source = [&](int slot) {
         return slot < hq ? io.q + (t * hq + slot) * D
@@ -149,7 +149,6 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
     }
 
     bool bad = false;
-    float *row = rowbuf[wave];
     for (int slot0 = first + wave; slot0 < end; slot0 += RG * waves) {
         if (slot0 != first + wave) load(slot0);
         // The norm of every row of the group before any is stored.
@@ -175,6 +174,12 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
                 x[i][k] = y;
             }
         }
+        // The rotary pairs elements j and j + D/2, which may sit in other lanes:
+        // through LDS (the wave's own rows).
+#pragma unroll
+        for (int i = 0; i < RG; ++i)
+            for (int k = 0; k < K; ++k) rowbuf[wave][i][lane + 64 * k] = x[i][k];
+        wave_lds_order();
 #pragma unroll
         for (int i = 0; i < RG; ++i) {
             const int slot = slot0 + i * waves;
@@ -188,11 +193,7 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
             const bool is_q = slot < hq;
             void *out = is_q ? io.q_out : io.k_out;
             const int64_t dst = is_q ? (t * hq + slot) * D : (int64_t)(slot - hq) * io.out_head_stride + t * D;
-            // The rotary pairs elements j and j + D/2, which may sit in other
-            // lanes: through LDS (the wave's own row, whose accesses complete
-            // in order).
-            for (int k = 0; k < K; ++k)
-                if (lane + 64 * k < D) row[lane + 64 * k] = x[i][k];
+            const float *row = rowbuf[wave][i];
             for (int k = 0; k < KP; ++k) {
                 const int j = lane + 64 * k;
                 if (j >= half) continue;
@@ -208,6 +209,7 @@ __device__ __forceinline__ void produce_rows(const_ptr<ProduceParams> p, const P
                 store_out<DT>(out, dst + j + half, b);
             }
         }
+        wave_lds_order();  // the next group's rows take their place
     }
     raise_status(p->status, bad, ST_NONFINITE_INPUT);
 }
