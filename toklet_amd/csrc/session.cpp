@@ -229,6 +229,11 @@ void free_session(tkh_session *s) {
     delete s;
 }
 
+// What the Q scratch of layers that are launched together may take: a thousandth of
+// the card.  Sharing launches pays up to the longest chunks (4,096 tokens of six
+// 8/4/256 layers 1.70 ms, 1.83 in slots for two; at 32/8/128 1.67 either way).
+constexpr uint64_t Q_SCRATCH_BYTES = 256 << 20;
+
 // Session::validate (src/session.rs:292-318): capacity, then every token id.
 uint32_t validate_tokens(const tkh_session *s, const uint32_t *tokens, uint64_t count,
                          uint64_t base, tkh_error *err) {
@@ -468,10 +473,9 @@ extern "C" uint32_t tkh_session_create(tkh_context *ctx, const tkh_session_optio
         s->chunk.ring_kv.reserve(s->producers);
         s->chunk.frames.reserve(s->producers);
         s->chunk.owner_frame.reserve(s->producers);
-        // A slot per layer that is launched together (f32 chunks are not).
-        s->q_slots = o->storage == TKH_F32 ? 1 : (int)std::min<uint64_t>(o->layers, tkh::DECODE_LAYERS_MAX);
-        s->scratch_bytes = (uint64_t)s->q_slots * chunk * o->query_heads * D * es;
-        hipError_t e = hipMalloc(&s->q_scratch, s->scratch_bytes);
+        const uint64_t slot = chunk * o->query_heads * D * es;
+        s->scratch_bytes = slot;
+        hipError_t e = hipMalloc(&s->q_scratch, slot);
         if (e == hipSuccess) e = hipMalloc(&s->committed_dev, sizeof(uint64_t));
         if (e == hipSuccess) e = tkh_launch_fill_u64(s->committed_dev, 0, ctx->stream);
         // The rotary (cos, sin) of every session position, once.
@@ -496,6 +500,22 @@ extern "C" uint32_t tkh_session_create(tkh_context *ctx, const tkh_session_optio
         if (e != hipSuccess) {
             free_session(s);
             return device_error(e, "session allocation", err);
+        }
+        // A Q slot per layer that is launched together (f32 chunks are not), as far
+        // as Q_SCRATCH_BYTES and then the memory go: one slot is all that a session
+        // needs, so the others never fail its creation.
+        const uint64_t slots =
+            o->storage == TKH_F32 ? 1 : std::min({o->layers, (uint64_t)tkh::DECODE_LAYERS_MAX, Q_SCRATCH_BYTES / slot});
+        if (slots > 1) {
+            void *wider = nullptr;
+            if (hipMalloc(&wider, slots * slot) == hipSuccess) {
+                hipFree(s->q_scratch);
+                s->q_scratch = wider;
+                s->q_slots = (int)slots;
+                s->scratch_bytes += (slots - 1) * slot;
+            } else {
+                (void)hipGetLastError();  // not the next call's
+            }
         }
     }
     *out = s;
