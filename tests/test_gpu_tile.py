@@ -146,3 +146,26 @@ def test_odd_partial_counts(torch_mod, orc, hq, hkv, D, queries, keys, dt):
     log(f"{hq}/{hkv}/{D} {dt} {queries} x {keys}")
     _close(host(out), ref, "context")
     ctx.close()
+
+
+# Head sizes that end inside a 256- or 512-wide build, where a wave that shares the
+# features has some or none of them, and rows that rule out vector loads there.
+WIDE = [
+    (4, 2, 130, 20, 90, None, 0.0, "f32", 0),
+    (4, 2, 132, 20, 90, 31, 30.0, "f32", 0),
+    (6, 2, 320, 17, 150, None, 0.0, "f32", 0),
+    (8, 1, 500, 9, 333, None, 0.0, "f32", 0),
+    (4, 2, 256, 20, 150, None, 0.0, "f32", 1),
+    (8, 1, 512, 9, 300, 70, 0.0, "f32", 1),
+    (4, 2, 200, 20, 150, None, 0.0, "bf16", 0),
+    (4, 2, 200, 20, 150, 31, 50.0, "f16", 1),
+    (6, 2, 260, 17, 333, None, 0.0, "f16", 0),
+    (6, 2, 260, 17, 333, None, 0.0, "bf16", 3),
+    (5, 1, 388, 3, 200, None, 0.0, "bf16", 4),     # whole vectors of four, not of eight
+]
+
+
+@pytest.mark.parametrize("diag", [False, True])
+@pytest.mark.parametrize("case", WIDE, ids=lambda c: "-".join(str(x) for x in c))
+def test_wide_builds_match_oracle(torch_mod, orc, case, diag):
+    test_tile_matches_oracle(torch_mod, orc, case, diag)
