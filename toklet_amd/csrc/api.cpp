@@ -5,7 +5,10 @@
 // toklet::cpu::Error before anything is launched.  A call then becomes a
 // list of device "problems" (device.hpp), a flat tile space split along the
 // key axis when the grid would otherwise be too small for 256 CUs, one
-// attention launch and one combine launch that publishes the context.
+// attention launch and, where keys are split across workgroups, one that combines
+// their partials (the streaming decode kernel may combine them itself).  Contexts
+// are written whatever the status word says; after TKH_NON_FINITE they are
+// unspecified.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -704,8 +707,8 @@ uint32_t launch_prefill(tkh_context *ctx, const Plan &plan, Problems group,
     return TKH_OK;
 }
 
-// FP32 storage, other head sizes and diagnostics: the FP32 tile kernel, then a
-// combine launch when the keys are split and a probability launch when asked.
+// FP32 storage, other head sizes and diagnostics: the FP32-exact kernels, then one
+// launch that combines the partials of split keys and makes the probabilities.
 uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_error *err) {
     const int64_t D = plan.head_dim, Hq = plan.query_heads, Hkv = plan.kv_heads, G = Hq / Hkv;
     const int64_t DP = tkh_tile_head((int)D), KT = tkh_tile_keys((int)plan.dtype, (int)D);
@@ -737,8 +740,8 @@ uint32_t launch_tile(tkh_context *ctx, const Plan &plan, Problems group, tkh_err
             vec = vec == 8 ? 4 : 1;
     }
     // Row groups per workgroup, then key splits, each at least a staged tile
-    // long, for at most tile_groups workgroups in all: two fit on a CU, and a few
-    // more than that many take a second round (128-token FP32 chunk at offset
+    // long, for at most tile_groups workgroups in all (half of them where a CU holds
+    // one workgroup and not two): a few more than fit at once take a second round (128-token FP32 chunk at offset
     // 1920, 14/2/64: 532 workgroups 29 us, the last 20 of them starting 17 us late).
     const int waves = tkh_tile_row_waves((int)plan.dtype, (int)D);
     const int rw = std::min(waves, max_rows <= 16 ? 1 : (max_rows <= 32 ? 2 : 4));
@@ -1016,7 +1019,7 @@ void init_tuning(tkh_context *ctx, int device) {
     ctx->prefill16 = env_int("TKH_PREFILL16", 1);
     ctx->prefill16_groups = std::max(1, env_int("TKH_PREFILL16_GROUPS", 64));
     ctx->prefill16_waves = env_int("TKH_PREFILL16_WAVES", 4) == 8 ? 8 : 4;
-    ctx->tile_groups = std::max(1, env_int("TKH_TILE_GROUPS", 512));
+    ctx->tile_groups = std::max(1, env_int("TKH_TILE_GROUPS", 2 * ctx->cus));
 }
 
 // First visible key (absolute) of a query at `position` (window_attention.rs:105-107).
@@ -1343,7 +1346,7 @@ namespace {
 
 // The device memory of tkh_attention_cached_static: the status word (the first
 // 256 bytes), then a workspace laid out as a context's (split-K partials of
-// the prefill and generic kernels, then the decode kernel's completion flags
+// the prefill and FP32-exact kernels, then the decode kernel's completion flags
 // and partials).  Each GPU the library runs on holds its own copy, at its own
 // address, until the process ends.
 constexpr size_t kStaticStatusBytes = 256;

@@ -4,11 +4,11 @@
 // at head_dim 64/128/256 take the MFMA prefill and streaming decode kernels
 // instead.
 //
-//  * attn_tile<DT, DP>: any head_dim D <= DP.  A workgroup is four waves over
-//    16 packed rows each (query x head of the GQA group) of one (problem, KV
-//    head), optionally one key split of it.
-//  * attn_split<DT, DP>: the same on the 16-bit matrix cores, FP32 values as
-//    16-bit planes.
+//  * attn_split<DT, DP>: any head_dim D <= DP on the 16-bit matrix cores, FP32
+//    values as 16-bit planes.  A workgroup is four waves over 16 packed rows each
+//    (query x head of the GQA group) of one (problem, KV head), optionally one key
+//    split of it.
+//  * attn_tile<DP>: the same on the FP32 matrix cores, for FP32 storage above 128.
 //  * attn_tile_merge: combines split-K partials (max, mass, unnormalised
 //    context) and writes the context; makes the diagnostics' probabilities from
 //    the stored scores and each row's merged (max, mass).
@@ -21,39 +21,32 @@ namespace tkh {
 
 namespace {
 
-// Keys per staged tile: K and V tiles of FP32 rows in about 33 KiB of LDS at
-// head sizes to 128 (four workgroups per CU), 66 KiB above (two).
-__host__ __device__ constexpr int tile_keys(int DP) { return DP <= 64 ? 64 : (DP <= 256 ? 32 : 16); }
+// attn_tile's keys per staged tile: K and V tiles of FP32 rows in about 66 KiB of LDS
+// (two workgroups per CU).
+__host__ __device__ constexpr int tile_keys(int DP) { return DP <= 256 ? 32 : 16; }
 
-// Waves that share a row group's features: a wave holds the Q and context of at
-// most 128, so head sizes above that fit two waves per SIMD without spills.
-__host__ __device__ constexpr int tile_feature_waves(int DP) { return DP <= 128 ? 1 : DP / 128; }
+// Its waves that share a row group's features: a wave holds the Q and context of 128,
+// which fits two waves per SIMD without spills.
+__host__ __device__ constexpr int tile_feature_waves(int DP) { return DP / 128; }
 
 // Four consecutive stored elements.
 template <int DT> struct Raw4 { using T = uint32_t __attribute__((ext_vector_type(2))); };
 template <> struct Raw4<F32> { using T = u32x4; };
 
 template <int DT> __device__ __forceinline__ f32x4 widen4(typename Raw4<DT>::T w) {
-    f32x4 x;
+    static_assert(DT == F32 || DT == F16, "bf16 is its own plane");
     if constexpr (DT == F32) {
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t u = w[e];
-            x[e] = __builtin_bit_cast(float, u);
-        }
+        return __builtin_bit_cast(f32x4, w);
     } else {
+        f32x4 x;
         for (int e = 0; e < 2; ++e) {
             const uint32_t u = w[e];
-            if constexpr (DT == BF16) {
-                x[2 * e] = __builtin_bit_cast(float, u << 16);
-                x[2 * e + 1] = __builtin_bit_cast(float, u & 0xffff0000u);
-            } else {
-                const f16x2 h = __builtin_bit_cast(f16x2, u);
-                x[2 * e] = (float)h[0];
-                x[2 * e + 1] = (float)h[1];
-            }
+            const f16x2 h = __builtin_bit_cast(f16x2, u);
+            x[2 * e] = (float)h[0];
+            x[2 * e + 1] = (float)h[1];
         }
+        return x;
     }
-    return x;
 }
 
 // Elements [off, off + 4) of a row of which the first n exist.  VEC (every row
@@ -304,14 +297,13 @@ struct TileOut {
 // share the groups' keys (a.kw of them, 16-key blocks in turn), each writing
 // a partial of its own, so short row blocks keep every SIMD busy.
 //
-// It replaced one wave per (query, head) on the vector unit, whose lanes each
-// read a key row of their own.  Per call: a 128-token FP32 chunk at offset
-// 1920 (14/2/64) with its append 1017 -> 25 us, a 512-token FP32 prompt 313 ->
-// 39 us, 128 queries over 1025 keys at 8/1/512 (bf16) 2240 -> 71 us, and 300
-// tokens of 16/8/128 with both diagnostics 243 -> 52 us.  (With each chunk's
-// load under a branch of its own the compiler waited for one before the next:
-// 40, 42, 281 and 57 us; whole 512-wide rows per wave spilled 390 registers.)
-template <int DT, int DP, bool VEC>
+// It replaced one wave per (query, head) on the vector unit, whose lanes each read a
+// key row of their own.  Calls back to back, FP32: 128 queries over 1025 keys at
+// 8/1/512 2419 -> 53 us, over 1920 keys at 8/4/256 1807 -> 43 us, 300 tokens of
+// 8/4/256 with both diagnostics 285 -> 29 us.  (Each chunk's load under a branch of
+// its own made the compiler wait for one before the next, and 512-wide rows held by
+// one wave spilled 390 registers.)
+template <int DP, bool VEC>
 __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
     constexpr int KT = tile_keys(DP), NB = KT / 16, FS = tile_feature_waves(DP);
@@ -320,8 +312,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     constexpr int NCH = KT * DP / 4 / 256;   // 4-element chunks per thread and tile
     __shared__ __attribute__((aligned(16))) float kt[KT * KS];
     __shared__ __attribute__((aligned(16))) float vt[KT * DP];
-    __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? 4 * NB * 64 : 1];  // partial scores
-    using Raw = typename Raw4<DT>::T;
+    __shared__ __attribute__((aligned(16))) f32x4 dots[4 * NB * 64];  // partial scores
+    using Raw = typename Raw4<F32>::T;
     const Params &p = a.p;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int j = lane & 15, g = lane >> 4;
@@ -346,7 +338,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
     for (int c = 0; c < FC; ++c) {
         const int d = f0 + 16 * c + 4 * g;
         const int64_t at = (int64_t)t_row * pr->q_row_stride + (int64_t)h_row * D;
-        q[c] = widen4<DT>(load4<DT, VEC>(pr->q, at + feature(d), D - d));
+        q[c] = widen4<F32>(load4<F32, VEC>(pr->q, at + feature(d), D - d));
     }
     if constexpr (VEC)
         for (int c = 0; c < FC; ++c)
@@ -366,8 +358,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
             for (int m = 0; m < NCH; ++m) {
                 const int i = tid + 256 * m, d = 4 * (i % CPR);
                 const int64_t off = at + min(t0 + i / CPR, n - 1) * rs + feature(d);
-                kreg[m] = load4<DT, VEC>(kb, off, D - d);
-                vreg[m] = load4<DT, VEC>(vb, off, D - d);
+                kreg[m] = load4<F32, VEC>(kb, off, D - d);
+                vreg[m] = load4<F32, VEC>(vb, off, D - d);
             }
         } else {
 #pragma unroll
@@ -375,8 +367,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
                 const int i = tid + 256 * m, d = 4 * (i % CPR);
                 const void *kb, *vb;
                 const int64_t off = seg_select(pr, lo + min(t0 + i / CPR, n - 1), kvh, &kb, &vb) + feature(d);
-                kreg[m] = load4<DT, VEC>(kb, off, D - d);
-                vreg[m] = load4<DT, VEC>(vb, off, D - d);
+                kreg[m] = load4<F32, VEC>(kb, off, D - d);
+                vreg[m] = load4<F32, VEC>(vb, off, D - d);
             }
         }
     };
@@ -386,8 +378,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
         for (int m = 0; m < NCH; ++m) {
             const int i = tid + 256 * m, r = i / CPR, d = 4 * (i % CPR);
             const bool head = !VEC || d <= last, in = t0 + r >= vlo && t0 + r < vhi;
-            *reinterpret_cast<f32x4 *>(kt + r * KS + d) = head ? widen4<DT>(kreg[m]) : zero;
-            *reinterpret_cast<f32x4 *>(vt + r * DP + d) = head && in ? widen4<DT>(vreg[m]) : zero;
+            *reinterpret_cast<f32x4 *>(kt + r * KS + d) = head ? widen4<F32>(kreg[m]) : zero;
+            *reinterpret_cast<f32x4 *>(vt + r * DP + d) = head && in ? widen4<F32>(vreg[m]) : zero;
         }
     };
 
@@ -403,8 +395,8 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
         stage(t0);
         __syncthreads();
         if (t0 + KT < n) fetch(t0 + KT);
-        // Scores of the wave's blocks: dots over its features, then, when waves
-        // share the features, the sum of their dots (the same order in each).
+        // Scores of the wave's blocks: dots over its features, then the sum of the
+        // dots of the waves that share them (the same order in each).
         f32x4 st[NB];
         bool seen[NB], scored[NB];  // some row of the wave sees a key of the block; its scores are wanted
 #pragma unroll
@@ -427,17 +419,15 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
                 }
             }
             for (int r = 0; r < 4; ++r) st[b][r] = s0[r] + s1[r];
-            if constexpr (FS > 1) dots[(wave * NB + b) * 64 + lane] = st[b];
+            dots[(wave * NB + b) * 64 + lane] = st[b];
         }
-        if constexpr (FS > 1) {
-            __syncthreads();
+        __syncthreads();
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const f32x4 *d = dots + (wave - fs) * NB * 64 + b * 64 + lane;
-                st[b] = d[0];
-                for (int w = 1; w < FS; ++w)
-                    for (int r = 0; r < 4; ++r) st[b][r] += d[w * NB * 64][r];
-            }
+        for (int b = 0; b < NB; ++b) {
+            const f32x4 *d = dots + (wave - fs) * NB * 64 + b * 64 + lane;
+            st[b] = d[0];
+            for (int w = 1; w < FS; ++w)
+                for (int r = 0; r < 4; ++r) st[b][r] += d[w * NB * 64][r];
         }
         float tmax = finish_scores<NB>(p, w, pr, t0, g, fs == 0, scored, st, amax);
         // The tile's maximum over the row's four lanes; O and l move with it.
@@ -483,8 +473,9 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 
 // ---------------------------------------------------------------------------
 // attn_split: the same walk on the 16-bit matrix cores (v_mfma_f32_16x16x32,
-// sixteen times the FP32 rate), with FP32 operands split into 16-bit planes whose
-// products lose nothing FP32 arithmetic keeps.
+// sixteen times the FP32 rate), with FP32 values as 16-bit planes, in which a product
+// is known to 2^-25 of itself and sums are FP32's.  Launches and memory round trips
+// bound it at the sizes below, the staging through registers on long ranges.
 //
 //  * Probabilities are three bf16 planes, each the rounding of what the last left:
 //    their sum is the FP32 value, over all of FP32's normal range.
@@ -500,6 +491,12 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 //    values is the six plane products down to 2^-18 of it; the three left out are
 //    below 2^-25 of it together, half of FP32's own rounding.  Planes hold an
 //    element below 2^-110 to 2^-133, bf16's smallest number.
+//
+// Against one wave per (query, head) on the vector unit, per call with the wait or
+// the append where the call has one: a 128-token FP32 chunk at offset 1920 (14/2/64)
+// 1017 -> 24.0 us, a 512-token FP32 prompt 313 -> 35.6 us, 300 tokens of 16/8/128 bf16
+// with both diagnostics 243 -> 37.1 us, 128 queries over 1025 keys at 8/1/512 bf16
+// 2240 -> 53.5 us; errors against 64 bits a fifth to half of its.
 //
 // Lane (j, g) holds query row j.  Q.K: A = K plane (key j of a 16-key block,
 // features 32 s + 8 g .. + 7), B = Q.  P.V over 32 keys: the MFMA's k index
@@ -576,9 +573,10 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     constexpr int KPL = KT * KROW, VPL = DP * VROW;           // bytes per plane
     constexpr bool VEC = VE > 1;
     // A thread's K chunks of eight features and V blocks of four keys by VF
-    // features; with whole 16-byte vectors of 16-bit elements a wide tile's
-    // blocks take eight: half the load instructions (300 tokens of 16/8/128 with
-    // diagnostics 39.7 -> 37.1 us a call, 128 queries of 8/1/512 59.7 -> 57.1).
+    // features.  Rows of whole 16-byte vectors of 16-bit elements load eight at a time
+    // (K and Q: 300 tokens of 16/8/128 with diagnostics 39.7 -> 37.1 us a call); a wide
+    // tile's V blocks take eight as well (with K and Q, 128 queries of 8/1/512 59.7 ->
+    // 57.1), where narrower tiles have too few blocks for every thread.
     constexpr int VF = VE == 8 && DP >= 256 ? 8 : 4;
     constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / (4 * VF) / 256;
     static_assert(NK >= 1 && NV >= 1, "staging covers the tile");
@@ -967,8 +965,8 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
 #define TKH_LAUNCH(...) hipExtLaunchKernelGGL((__VA_ARGS__), grid, block, 0, stream, start, stop, 0, *a)
 #define TKH_TILE(DP)                                                                    \
     if (dtype == F32 && dp == DP) {                                                     \
-        if (a->vec >= 4) TKH_LAUNCH(attn_tile<F32, DP, true>);                          \
-        else TKH_LAUNCH(attn_tile<F32, DP, false>);                                     \
+        if (a->vec >= 4) TKH_LAUNCH(attn_tile<DP, true>);                               \
+        else TKH_LAUNCH(attn_tile<DP, false>);                                          \
         return hipGetLastError();                                                       \
     }
 #define TKH_SPLIT(DT, DP)                                                               \

@@ -149,10 +149,10 @@ struct Params {
     float softcap_log2;     // softcap * log2(e): tanh units -> log2 units
     int64_t total_tiles;
     // split-K partials
-    float *part_o;          // per slot: [head size] (tile kernel), [D, rows] (chunk kernel)
+    float *part_o;          // per slot: [built head size] (FP32-exact kernels), [D, rows] (chunk kernel)
     float *part_ml;         // [rows, splits, 2] (max in log2 units, mass)
     uint32_t *status;
-    // optional diagnostics (tile kernel only)
+    // optional diagnostics (FP32-exact kernels only)
     float *scores;
     float *probs;
     int32_t diag_mode;      // 0 none, 1 full [Hq, queries, keys], 2 last row [keys]
@@ -293,7 +293,7 @@ struct ProduceLayersArgs {
     ProduceLayer e[DECODE_LAYERS_MAX];
 };
 
-// The FP32 tile kernels' argument (attention.hip).
+// The FP32-exact kernels' argument (attention.hip).
 struct TileArgs {
     Params p;             // first: the single-problem path reads it at the kernel-argument base
     int32_t rw;           // 16-row groups per workgroup (1, 2 or 4)
@@ -316,20 +316,10 @@ template <class T> __device__ __forceinline__ global_ptr<T> gstore_ptr(void *p) 
     return (global_ptr<T>)p;
 }
 
-__device__ __forceinline__ int find_problem(const Params &p, int64_t tile) {
-    const_ptr<Problem> probs = (const_ptr<Problem>)p.problems;
-    int lo = 0, hi = p.nproblems - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (probs[mid].tile_base <= tile) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
-// The same search by a whole wave: each lane tests one candidate, a ballot
-// picks the interval, so up to 64 problems take one round trip of loads and up
-// to 4096 two (the scalar binary search above is a chain of log2(n) dependent
-// loads).  Every lane of the wave must be active.
+// The problem that owns a tile (the last that starts at or before it), by a whole
+// wave: each lane tests one candidate, a ballot picks the interval, so up to 64
+// problems take one round trip of loads and up to 4096 two (a scalar binary search
+// is a chain of log2(n) dependent loads).  Every lane of the wave must be active.
 __device__ __forceinline__ int find_problem_wave(const Problem *problems, int n, int64_t tile) {
     const int lane = threadIdx.x & 63;
     int lo = 0, count = n;
@@ -345,10 +335,6 @@ __device__ __forceinline__ int find_problem_wave(const Problem *problems, int n,
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// The problem owning global tile `tile`, as a constant-space pointer: either
-// the copy inside the kernel arguments (Params must be the kernel's first
-// argument) or an entry of the uploaded descriptor array.  Its fields are
-// uniform and load through the scalar cache.  Call with the whole wave active.
 // Bring the first NL 64-byte lines of the kernel arguments, and the line at
 // byte EXTRA (the hidden arguments after them: the grid size), into the
 // scalar cache at once: one scalar load per line, all in flight together,
@@ -402,18 +388,16 @@ template <class T, int NL, int EXTRA> __device__ __forceinline__ const_ptr<T> wa
     return (const_ptr<T>)((const_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() + z);
 }
 
+// The problem owning global tile `tile`, as a constant-space pointer: either
+// the copy inside the kernel arguments (Params must be the kernel's first
+// argument) or an entry of the uploaded descriptor array.  Its fields are
+// uniform and load through the scalar cache.  Call with the whole wave active.
 __device__ __forceinline__ const_ptr<Problem> problem_ptr(const Params &p, int64_t tile) {
     if (p.nproblems == 1) {
         const_ptr<Params> args = (const_ptr<Params>)__builtin_amdgcn_kernarg_segment_ptr();
         return &args->single;
     }
     return (const_ptr<Problem>)p.problems + find_problem_wave(p.problems, p.nproblems, tile);
-}
-
-// Generic reference form used by the VALU and MFMA kernels.
-__device__ __forceinline__ const Problem &tile_problem(const Params &p, int64_t tile) {
-    if (p.nproblems == 1) return p.single;
-    return p.problems[find_problem(p, tile)];
 }
 
 // Load one K or V element (any dtype) as float.
@@ -444,17 +428,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float x) {
 
 __device__ __forceinline__ bool is_finite_f(float x) {
     return __builtin_isfinite(x);
-}
-
-// Position of logical key `key` inside the problem's segments.
-__device__ __forceinline__ int64_t seg_offset(const Problem &pr, int64_t key, int kvh,
-                                              int *which) {
-    int s = 0;
-    if (pr.nseg > 1 && key >= pr.seg[1].start) s = 1;
-    if (pr.nseg > 2 && key >= pr.seg[2].start) s = 2;
-    *which = s;
-    const Segment &g = pr.seg[s];
-    return (int64_t)kvh * g.head_stride + (key - g.start) * g.row_stride;
 }
 
 // K/V addresses of logical key `key` by per-lane selects over the three

@@ -129,7 +129,7 @@ struct tkh_context {
     bool ring_used[kSlots] = {};
     int ring_next = 0;
     int split_keys_override = 0;
-    int force_generic = 0;
+    int force_generic = 0;       // every attention call on the FP32-exact kernels
     int decode_waves = 8;        // waves per decode workgroup
     int decode_keys_per_lane = 4;  // keys each lane holds per streamed block
     int cus = 256;               // compute units of the device
@@ -157,7 +157,7 @@ struct tkh_context {
     int prefill16 = 1;           // four-wave launches at head_dim 128/256 on the 16-row kernel (0: never)
     int prefill16_groups = 64;   // split target of the 16-row kernel's launches (in 128-row workgroups)
     int prefill16_waves = 4;     // 16-row waves per workgroup: 4 (64-row blocks) or 8 (128-row blocks)
-    int tile_groups = 512;       // FP32 tile kernel: below this many row-block workgroups, split the keys
+    int tile_groups = 512;       // FP32-exact kernels: below this many row-block workgroups, split the keys (two per CU)
     // Set only while a session adds a chunk's layer: where its attention call goes.
     tkh_host::ChunkBatchOfLayers *collect = nullptr;
     // profiling: per launch, start/stop of the attention kernel and of the combine kernel
