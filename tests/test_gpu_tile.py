@@ -1,9 +1,9 @@
-"""The FP32 tile kernel (attention.hip) at the sizes where it can go wrong: row
+"""The FP32-exact kernels (attention.hip) at the sizes where they can go wrong: row
 blocks and staged key tiles with remainders, head sizes that end inside a build,
 rows that rule out vector loads, waves that share a row group's keys, and the
 diagnostics.  Bar: the reference's gate 1e-5 + 1e-4|e| (tests/cpu_attention.rs:6-14)
-on the stored values, for every storage type, since the kernel's arithmetic is
-FP32 throughout."""
+on the stored values, for every storage type: products in planes keep FP32's
+precision, and sums are FP32's."""
 
 import numpy as np
 import pytest

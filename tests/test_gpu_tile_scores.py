@@ -137,3 +137,17 @@ def test_scores_past_the_largest_are_refused(torch_mod, orc, dt, D, diag):
         with pytest.raises(ops.TkhError) as e:
             _run(torch_mod, orc, q, stored(k, dt), np.ones_like(k), dt, 1e30, diag=diag, check=False)
         assert e.value.name == "NonFinite"
+
+
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("dt,D,diag", [("f32", 64, False), ("f32", 256, True), ("bf16", 96, False), ("f16", 128, True)])
+def test_nan_operands_are_refused(torch_mod, orc, dt, D, diag, softcap):
+    """Also with a softcap, whose tanh saturates for any size of score."""
+    from toklet_amd import ops
+
+    for at in range(3):
+        operands = [np.ones((QUERIES, HQ, D), np.float32), *(np.ones((HKV, 40, D), np.float32) for _ in range(2))]
+        operands[at][1, 3, 5] = np.nan
+        with pytest.raises(ops.TkhError) as e:
+            _run(torch_mod, orc, *operands, dt, 1.0, softcap, diag, check=False)
+        assert e.value.name == "NonFinite"

@@ -524,7 +524,8 @@ __device__ __forceinline__ float softcap_f(float x, float cap) {
         float y2 = y * y;
         t = y * (1.0f + y2 * (-1.0f / 3.0f + y2 * (2.0f / 15.0f + y2 * (-17.0f / 315.0f))));
     } else {
-        float e = __builtin_amdgcn_exp2f(fminf(2.0f * LOG2E * a, 126.0f));
+        const float x2 = 2.0f * LOG2E * a;
+        const float e = __builtin_amdgcn_exp2f(x2 > 126.0f ? 126.0f : x2);  // not fminf: NaN stays NaN
         t = copysignf(1.0f - 2.0f / (e + 1.0f), y);
     }
     return cap * t;
