@@ -485,7 +485,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 //    of 1 and none of one of 2^-36: 69 keys e^-25 as heavy as one whose V is zero
 //    summed to 23% of their context.  They took 23.2 us for 128 queries over 2048
 //    keys at 12/4/96, 24.2 for 300 tokens of 16/8/128 with diagnostics and 40.5 for
-//    128 queries over 1025 keys at 8/1/512; these 26.1, 25.7 and 44.0.)
+//    128 queries over 1025 keys at 8/1/512; these 26.1, 25.8 and 37.3.)
 //  * F32 storage: Q, K and V are three bf16 planes each, and a product of two
 //    values is the six plane products down to 2^-18 of it; the three left out are
 //    below 2^-25 of it together, half of FP32's own rounding.  Planes hold an
@@ -507,6 +507,11 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 // 512-wide heads fit a CU) have their 16-byte chunks XOR-swizzled by row.
 __host__ __device__ constexpr int split_keys(int DP) { return DP <= 64 ? 64 : 32; }
 __host__ __device__ constexpr int split_feature_waves(int DP) { return DP <= 256 ? 1 : 2; }
+// Waves of a workgroup.  Four, and two workgroups per CU; but 512-wide f16 tiles (V in
+// two planes: 113 KiB with the dots) leave room for one, which takes eight (with four,
+// 128 queries over 1025 keys at 8/1/512 took 44.0 us and 256 over 2300 at 8/2/512 107,
+// with eight 37.3 and 63; a wave then holds the next tile without spills, too).
+__host__ __device__ constexpr int split_waves(int DT, int DP) { return DT == F16 && DP == 512 ? 8 : 4; }
 
 namespace {
 
@@ -563,9 +568,10 @@ __device__ __forceinline__ void prob_planes(const f32x4 &x, const f32x4 &y, u32x
 
 // VE: elements that start and end every row in whole vectors (1: element loads).
 template <int DT, int DP, int VE>
-__global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
+__global__ __launch_bounds__(64 * split_waves(DT, DP), 2) void attn_split(TileArgs a) {
     warm_kernarg<(sizeof(TileArgs) + 63) / 64, 0>();
     constexpr int KT = split_keys(DP), NB = KT / 16, NG = KT / 32, FS = split_feature_waves(DP);
+    constexpr int NW = split_waves(DT, DP), NT = 64 * NW;     // waves and threads
     constexpr int DW = DP / FS, QS = DW / 32, FB = DW / 16;   // a wave's features, Q.K steps, P.V blocks
     constexpr int SP = Planes<DT>::qk, VP = Planes<DT>::v;
     constexpr int KROW = DP * 2 + 16, VROW = KT * 2;          // staged row bytes: K per key, V per feature
@@ -577,11 +583,11 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     // tile's V blocks take eight as well (with K and Q, 128 queries of 8/1/512 59.7 ->
     // 57.1), where narrower tiles have too few blocks for every thread.
     constexpr int VF = VE == 8 && DP >= 256 ? 8 : 4;
-    constexpr int NK = KT * DP / 8 / 256, NV = KT * DP / (4 * VF) / 256;
+    constexpr int NK = KT * DP / 8 / NT, NV = KT * DP / (4 * VF) / NT;
     static_assert(NK >= 1 && NV >= 1, "staging covers the tile");
     __shared__ __attribute__((aligned(16))) uint8_t kt[SP * KPL];
     __shared__ __attribute__((aligned(16))) uint8_t vt[VP * VPL];
-    __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? 4 * NB * 64 : 1];  // partial scores
+    __shared__ __attribute__((aligned(16))) f32x4 dots[FS > 1 ? NW * NB * 64 : 1];  // partial scores
     using Raw = typename Raw4<DT>::T;
     const Params &p = a.p;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -625,14 +631,14 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     auto fetch_rows = [&](auto at) {
 #pragma unroll
         for (int m = 0; m < NK; ++m) {
-            const int i = tid + 256 * m, d = 8 * (i % CPR);
+            const int i = tid + NT * m, d = 8 * (i % CPR);
             const void *kb, *vb;
             const auto off = at(i / CPR, &kb, &vb);
             load_eight(kb, off, d, kreg[m]);
         }
 #pragma unroll
         for (int m = 0; m < NV; ++m) {
-            const int i = tid + 256 * m, d = VF * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
+            const int i = tid + NT * m, d = VF * (i / 8 % FPR), k0 = i / (8 * FPR) * 32 + 4 * (i % 8);
             for (int r = 0; r < 4; ++r) {
                 const void *kb, *vb;
                 const auto off = at(k0 + r, &kb, &vb);
@@ -674,14 +680,14 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
     auto stage = [&](int t0) {
 #pragma unroll
         for (int m = 0; m < NK; ++m) {
-            const int i = tid + 256 * m, d = 8 * (i % CPR);
+            const int i = tid + NT * m, d = 8 * (i % CPR);
             u32x4 pl[SP];
             planes8<DT>(whole(d, 4) ? kreg[m][0] : none, whole(d + 4, 4) ? kreg[m][1] : none, pl);
             for (int s = 0; s < SP; ++s) *reinterpret_cast<u32x4 *>(kt + s * KPL + i / CPR * KROW + 2 * d) = pl[s];
         }
 #pragma unroll
         for (int m = 0; m < NV; ++m) {
-            const int i = tid + 256 * m, qd = i % 8, d0 = VF * (i / 8 % FPR), t = i / (8 * FPR);
+            const int i = tid + NT * m, qd = i % 8, d0 = VF * (i / 8 % FPR), t = i / (8 * FPR);
             const int k0 = t0 + 32 * t + 4 * qd;
             for (int half = 0; half < VF / 4; ++half) {
                 const int d = d0 + 4 * half;
@@ -697,7 +703,8 @@ __global__ __launch_bounds__(256, 2) void attn_split(TileArgs a) {
                         float v[4] = {y[0][e], y[1][e], y[2][e], y[3][e]};
                         for (int s = 0; s < VP; ++s) {
                             using Quad = typename Raw4<F16>::T;
-                            const Quad o = s == 0 ? Quad{plane2<true>(v[0], v[1]), plane2<true>(v[2], v[3])}
+                            constexpr bool LIMIT = DT == F32;
+                            const Quad o = s == 0 ? Quad{plane2<LIMIT>(v[0], v[1]), plane2<LIMIT>(v[2], v[3])}
                                                   : Quad{plane2<false>(v[0], v[1]), plane2<false>(v[2], v[3])};
                             *reinterpret_cast<Quad *>(to(e) + s * VPL) = o;
                         }
@@ -939,6 +946,11 @@ extern "C" int tkh_tile_head(int head_dim) {
 // products cost 6/16 of FP32 MFMAs; three planes of wider FP32 tiles do not leave
 // room for two workgroups in LDS, and those stay on attn_tile.
 static bool tile_splits(int dtype, int head_dim) { return dtype != tkh::F32 || tkh_tile_head(head_dim) <= 128; }
+// Waves of a workgroup, and workgroups a CU holds.
+static int tile_waves(int dtype, int head_dim) {
+    return tile_splits(dtype, head_dim) ? tkh::split_waves(dtype, tkh_tile_head(head_dim)) : 4;
+}
+extern "C" int tkh_tile_resident(int dtype, int head_dim) { return tile_waves(dtype, head_dim) > 4 ? 1 : 2; }
 // Keys of a staged tile, row groups a workgroup has waves for, and how many of
 // its waves may share a row group's keys.
 extern "C" int tkh_tile_keys(int dtype, int head_dim) {
@@ -947,11 +959,8 @@ extern "C" int tkh_tile_keys(int dtype, int head_dim) {
 }
 extern "C" int tkh_tile_row_waves(int dtype, int head_dim) {
     const int dp = tkh_tile_head(head_dim);
-    return 4 / (tile_splits(dtype, head_dim) ? tkh::split_feature_waves(dp) : tkh::tile_feature_waves(dp));
+    return tile_waves(dtype, head_dim) / (tile_splits(dtype, head_dim) ? tkh::split_feature_waves(dp) : tkh::tile_feature_waves(dp));
 }
-// Workgroups a CU holds: the 105 KiB of 512-wide f16 tiles leave room for one (128
-// queries over 1025 keys at 8/1/512, kernels alone: 53.9 us split for two, 44.0 for one).
-extern "C" int tkh_tile_resident(int dtype, int head_dim) { return dtype == tkh::F16 && tkh_tile_head(head_dim) == 512 ? 1 : 2; }
 extern "C" int tkh_tile_share(int dtype, int head_dim) {
     return tile_splits(dtype, head_dim) ? 1 : tkh_tile_keys(dtype, head_dim) / 16;
 }
@@ -963,7 +972,7 @@ extern "C" hipError_t tkh_launch_tile(const tkh::TileArgs *a, int dtype, hipStre
                                       hipEvent_t start, hipEvent_t stop) {
     using namespace tkh;
     const int dp = tkh_tile_head(a->p.head_dim);
-    dim3 grid((unsigned)a->p.total_tiles), block(256);
+    dim3 grid((unsigned)a->p.total_tiles), block((unsigned)(64 * tile_waves(dtype, a->p.head_dim)));
 #define TKH_LAUNCH(...) hipExtLaunchKernelGGL((__VA_ARGS__), grid, block, 0, stream, start, stop, 0, *a)
 #define TKH_TILE(DP)                                                                    \
     if (dtype == F32 && dp == DP) {                                                     \
