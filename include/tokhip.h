@@ -101,7 +101,7 @@ void *tkh_context_stream(tkh_context *ctx);
  * reference's Metal encoder timestamps, src/metal/profile.rs:1-3).  Enabling
  * resets the totals; reading waits for the stream.  Times are milliseconds
  * summed over launches: `attention` is the attention kernel alone, `combine`
- * the split-K combine/publish kernel. */
+ * the split-K combine kernel (with the diagnostics' probabilities). */
 typedef struct tkh_profile {
     uint64_t launches;
     double attention_ms;

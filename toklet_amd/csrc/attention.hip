@@ -5,9 +5,9 @@
 // instead.
 //
 //  * attn_split<DT, DP>: any head_dim D <= DP on the 16-bit matrix cores, FP32
-//    values as 16-bit planes.  A workgroup is four waves over 16 packed rows each
-//    (query x head of the GQA group) of one (problem, KV head), optionally one key
-//    split of it.
+//    values as 16-bit planes.  A workgroup is four waves (eight: split_waves) over 16
+//    packed rows each (query x head of the GQA group) of one (problem, KV head),
+//    optionally one key split of it.
 //  * attn_tile<DP>: the same on the FP32 matrix cores, for FP32 storage above 128.
 //  * attn_tile_merge: combines split-K partials (max, mass, unnormalised
 //    context) and writes the context; makes the diagnostics' probabilities from
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 // bound it at the sizes below, the staging through registers on long ranges.
 //
 //  * Probabilities are three bf16 planes, each the rounding of what the last left:
-//    their sum is the FP32 value, over all of FP32's normal range.
+//    their sum is the FP32 value.
 //  * bf16 storage: Q, K and V are planes as they are.
 //  * f16 storage: Q and K are, on the f16 form of the MFMA; V's 11 bits are two bf16
 //    planes, exactly, and the product left out is below 2^-26 of the whole.  (Two
@@ -488,14 +488,19 @@ __global__ __launch_bounds__(256, 2) void attn_tile(TileArgs a) {
 //    128 queries over 1025 keys at 8/1/512; these 26.1, 25.8 and 37.3.)
 //  * F32 storage: Q, K and V are three bf16 planes each, and a product of two
 //    values is the six plane products down to 2^-18 of it; the three left out are
-//    below 2^-25 of it together, half of FP32's own rounding.  Planes hold an
-//    element below 2^-110 to 2^-133, bf16's smallest number.
+//    below 2^-25 of it together, half of FP32's own rounding.
+//
+// Planes end at bf16's smallest number, 2^-133, so an element (or weight) below
+// 2^-109 keeps fewer bits than FP32 has: contexts of V about 1e-33 are off by 2e-7 as
+// all others, of 1e-36 by 3e-5, where FP32 products gave 4e-7.  Planes scaled apart
+// would hold them at the price of a sum each (the sums apart below took FP32 1.5%
+// longer), for values that no activation has.
 //
 // Against one wave per (query, head) on the vector unit, per call with the wait or
 // the append where the call has one: a 128-token FP32 chunk at offset 1920 (14/2/64)
-// 1017 -> 24.0 us, a 512-token FP32 prompt 313 -> 35.6 us, 300 tokens of 16/8/128 bf16
+// 1017 -> 23.0 us, a 512-token FP32 prompt 313 -> 35.6 us, 300 tokens of 16/8/128 bf16
 // with both diagnostics 243 -> 37.1 us, 128 queries over 1025 keys at 8/1/512 bf16
-// 2240 -> 53.5 us; errors against 64 bits a fifth to half of its.
+// 2240 -> 55 us; errors against 64 bits a quarter to 0.6 of its.
 //
 // Lane (j, g) holds query row j.  Q.K: A = K plane (key j of a 16-key block,
 // features 32 s + 8 g .. + 7), B = Q.  P.V over 32 keys: the MFMA's k index
